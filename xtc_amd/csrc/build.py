@@ -255,7 +255,7 @@ def _compile(src: Path, obj: Path, verbose: bool) -> tuple[Path, float]:
 def build(jobs: int | None = None, verbose: bool = False) -> Path:
     """Compiles every kernel instance and links in-tree libxtc_hip.so."""
     t0 = time.time()
-    srcs = [CSRC / "runtime.hip", *generate()]
+    srcs = [CSRC / "runtime.hip", *sorted(CSRC.glob("planes_*.hip")), *generate()]
     objs = [BUILD / (s.stem + ".o") for s in srcs]
     jobs = jobs or max(1, min(16, os.cpu_count() or 1))
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:

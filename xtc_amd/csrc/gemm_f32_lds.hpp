@@ -1,5 +1,5 @@
 // SPDX-License-Identifier: BSD-3-Clause
-// fp32 GEMM for aligned shapes on gfx950, LDS-DMA pipeline, one workgroup
+// fp32 GEMM on fp32 MFMAs for aligned shapes on gfx950, LDS-DMA pipeline, one workgroup
 // of 8 waves per CU:
 //   C[M,N] = epilogue( A[M,K] @ B[K,N] ), fp32 row-major, optional split-K
 // with M % BM == 0, N % BN == 0, each split's K range a multiple of BK (16 or 32),

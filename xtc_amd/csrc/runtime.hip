@@ -27,6 +27,7 @@
 #include "gemm_f64.hpp"
 #include "conv_direct.hpp"
 #include "mfma_peak.hpp"
+#include "planes_table.hpp"
 #include "registry.hpp"
 #include "xtc_hip.h"
 
@@ -1045,9 +1046,41 @@ bool skinny_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, in
   return true;
 }
 
-// The LDS-DMA fp32 kernel (gemm_f32_lds.hpp) implements the 128x256x32 (2x4
-// waves), 256x128x32 (4x2 waves) and 128x128x32 (2x4 waves) fp32 tiles,
-// split-K included, when the
+// gemm_planes (gemm_planes.hpp) runs fp32 matmuls on bf16 MFMAs behind the
+// 128x256x32 (2x4 waves), 256x128x32 (4x2) and 128x128x32 (2x4) tiles, any M,
+// N and K of whole 16-byte vectors, split-K included.  Against the LDS-DMA
+// kernel on fp32 MFMAs that these tiles had before: 4096^3 980 -> 631 us,
+// 2048x4096x1024 130-144 -> 88-95 us, 2048x1024x4096 at split 2 150 -> 103 us,
+// at a fifth of its error against float64.  Those tiles at a slab depth of 16
+// keep the fp32 MFMAs (gemm_f32_lds.hpp): an instruction takes 32 of k.
+const PlanesEntry* planes_entry(int dtype, int conv, int bt, int vec, const xtc_hip_tile& t, int ring) {
+  int n = 0;
+  const PlanesEntry* e = planes_f32(&n);
+  for (int i = 0; i < n; ++i)
+    if (e[i].dtype == dtype && e[i].conv == conv && e[i].bt == bt && e[i].vec == vec && e[i].bm == t.bm &&
+        e[i].bn == t.bn && e[i].wgm == t.wgm && e[i].wgn == t.wgn && (ring == 0 || e[i].ring == ring))
+      return &e[i];
+  return nullptr;
+}
+
+bool generic_only() {
+  static const bool v = [] {
+    const char* e = getenv("XTC_HIP_GENERIC_GEMM");
+    return e && e[0] == '1';
+  }();
+  return v;
+}
+
+// Whether gemm_planes runs a matmul whose operands are whole 16-byte vectors.
+bool planes_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int lda, int ldb) {
+  if (generic_only() || d.dtype != XTC_HIP_F32 || t.bk != 32) return false;
+  if (!planes_entry(0, 0, 0, 1, t, 0)) return false;
+  // byte offsets inside a tile's rows fit in 32 bits
+  return (int64_t)t.bm * lda <= INT32_MAX / 4 && (int64_t)(t.bk + 1) * ldb <= INT32_MAX / 4;
+}
+
+// The LDS-DMA fp32 kernel (gemm_f32_lds.hpp) implements the 128x256x16 (2x4
+// waves) and 256x128x16 (4x2 waves) fp32 tiles, split-K included, when the
 // shape needs no bounds checks: one workgroup of 8 waves per CU.
 bool f32_lds_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_k, int lda,
                           int ldb, int ldc, const void* A, const void* B, const void* C,
@@ -1059,10 +1092,7 @@ bool f32_lds_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, i
   if (disabled || d.dtype != XTC_HIP_F32) return false;
   const bool t1 = t.bm == 128 && t.bn == 256 && t.wgm == 2 && t.wgn == 4;
   const bool t2 = t.bm == 256 && t.bn == 128 && t.wgm == 4 && t.wgn == 2;
-  const bool t3 = t.bm == 128 && t.bn == 128 && t.wgm == 2 && t.wgn == 4;
-  // BK 32 (3 stages) for all three tiles; BK 16 (deeper stages) for the two
-  // 256-wide ones
-  if (!(t1 || t2 || t3) || !(t.bk == 32 || (t.bk == 16 && !t3))) return false;
+  if (!(t1 || t2) || t.bk != 16) return false;
   const int splits = split_k < 1 ? 1 : split_k;
   if (d.M % t.bm || d.N % t.bn || d.K % (t.bk * splits)) return false;
   if (lda % 4 || ldb % 4 || ldc % 4) return false;
@@ -1078,10 +1108,7 @@ void launch_f32_lds(const GemmArgs& a, dim3 grid, hipStream_t s) {
 }
 
 // Compiled pipeline depths (LDS stages) of the LDS-DMA fp32 kernel, per tile;
-// the first entry of a tile is its default.  BK 16 stages are 24 KB (up to
-// 6 fit), BK 32 stages 48 KB for the 256-wide tiles (up to 3) and 32 KB for
-// 128x128 (up to 4: five would leave no room for the split-K flag).  Against 3 stages of BK 32, 4-5 stages of BK 16
-// measured 2-4 % faster on one box and 1-1.5 % slower on another.
+// the first entry of a tile is its default.  A stage is 24 KB (up to 6 fit).
 struct F32LdsVariant {
   int bm, bn, bk, wgm, wgn, stages;
   GemmLaunch launch;
@@ -1095,13 +1122,6 @@ const F32LdsVariant kF32Lds[] = {
     {128, 256, 16, 2, 4, 3, &launch_f32_lds<128, 256, 16, 2, 4, 3>},
     {128, 256, 16, 2, 4, 4, &launch_f32_lds<128, 256, 16, 2, 4, 4>},
     {128, 256, 16, 2, 4, 6, &launch_f32_lds<128, 256, 16, 2, 4, 6>},
-    {256, 128, 32, 4, 2, 3, &launch_f32_lds<256, 128, 32, 4, 2, 3>},
-    {256, 128, 32, 4, 2, 2, &launch_f32_lds<256, 128, 32, 4, 2, 2>},
-    {128, 256, 32, 2, 4, 3, &launch_f32_lds<128, 256, 32, 2, 4, 3>},
-    {128, 256, 32, 2, 4, 2, &launch_f32_lds<128, 256, 32, 2, 4, 2>},
-    {128, 128, 32, 2, 4, 3, &launch_f32_lds<128, 128, 32, 2, 4, 3>},
-    {128, 128, 32, 2, 4, 2, &launch_f32_lds<128, 128, 32, 2, 4, 2>},
-    {128, 128, 32, 2, 4, 4, &launch_f32_lds<128, 128, 32, 2, 4, 4>},
 };
 
 // The variant of tile t with `stages` (0: the tile's default), or null.
@@ -1507,7 +1527,7 @@ const void* transposed_copy(int slot, const void* src, int R, int Cc, int ld_src
 
 // The kernel family a matmul runs on, chosen from the shape, tile, split,
 // strides and operand alignment in the order of matmul_impl.
-enum class MatmulPath { LdsDmaBt, Naive, LdsDma, Skinny, SplitWave, F32Lds, F64, Generic };
+enum class MatmulPath { LdsDmaBt, Naive, LdsDma, Skinny, SplitWave, Planes, F32Lds, F64, Generic };
 
 const char* path_name(MatmulPath p) {
   switch (p) {
@@ -1520,6 +1540,8 @@ const char* path_name(MatmulPath p) {
       return "skinny bf16";
     case MatmulPath::SplitWave:
       return "split-wave fp32";
+    case MatmulPath::Planes:
+      return "bf16-plane";
     case MatmulPath::F32Lds:
       return "LDS-DMA fp32";
     case MatmulPath::F64:
@@ -1555,6 +1577,13 @@ int path_depths(MatmulPath p, const xtc_hip_tile& t, int ring, int* out, int max
       break;
     case MatmulPath::SplitWave:
       for (int v : kSplitWaveDepths) tmp[n++] = v;
+      break;
+    case MatmulPath::Planes:
+      // one pipeline behind every depth a schedule may name: two LDS buffers
+      // and the next slab in registers
+      tmp[n++] = 3;
+      tmp[n++] = 2;
+      if (t.bm == 128 && t.bn == 128) tmp[n++] = 4;
       break;
     case MatmulPath::F32Lds:
       for (const F32LdsVariant& v : kF32Lds)
@@ -1640,6 +1669,8 @@ int natural_path(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_
     *path = MatmulPath::Skinny;
   else if (splitwave_gemm_applies(d, t, split_k, lda, A))
     *path = MatmulPath::SplitWave;
+  else if (planes_gemm_applies(d, t, lda, ldb))
+    *path = MatmulPath::Planes;
   else if (f32_lds_gemm_applies(d, t, split_k, lda, ldb, ldc, A, B, C, (const float*)bias))
     *path = MatmulPath::F32Lds;
   else
@@ -1728,14 +1759,14 @@ int matmul_impl(const xtc_hip_matmul_desc& d, const void* A, const void* B, void
   if (path == MatmulPath::SplitWave)
     return launch_splitwave_gemm(d, split_k, d.stages, lda, ldb, ldc, A, B, C, bias, s);
   const GemmEntry* e = find_entry(d.dtype, 0, t);
-  GemmEntry lds_entry;
-  if (path == MatmulPath::F32Lds) {
+  GemmEntry own;
+  if (path == MatmulPath::F32Lds || path == MatmulPath::Planes) {
     // same tiles, split-K set-up and grid as the generic instance; only the
     // kernel differs
-    lds_entry = *e;
-    lds_entry.launch = f32_lds_variant(t, d.stages)->launch;
-    lds_entry.launch_ring = nullptr;
-    e = &lds_entry;
+    own = *e;
+    own.launch = path == MatmulPath::F32Lds ? f32_lds_variant(t, d.stages)->launch : planes_entry(0, 0, 0, 1, t, 0)->launch;
+    own.launch_ring = nullptr;
+    e = &own;
   }
   GemmArgs a;
   memset(&a, 0, sizeof(a));
