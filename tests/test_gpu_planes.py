@@ -15,7 +15,8 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from test_gpu_kernels import needs_specialised, rng_uniform, run_matmul
+from oracle import reference as ref
+from test_gpu_kernels import _run_depth, needs_specialised, rng_uniform, run_matmul
 from xtc_amd.runtimes.hip.buffer import ensure_device
 
 pytestmark = [pytest.mark.gpu, needs_specialised]
@@ -47,6 +48,35 @@ def test_edges(tile, M, N, K, split):
     print(f"[planes] {tile} {M}x{N}x{K} split {split}", flush=True)
     a, b = rng_uniform(M + K, (M, K)), rng_uniform(N + K, (K, N))
     check(run_matmul(a, b, tile=tile, split_k=split), a, b)
+
+
+# no whole vectors anywhere: fp32 and bf16 rows at element alignment, units cut
+# by K and N, tiles cut by M and N, split-K partial rows of whole vectors
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("M,N,K,split", [(1, 1, 1, 1), (3, 5, 7, 1), (64, 65, 63, 1), (67, 129, 131, 1),
+                                         (130, 63, 257, 2), (65, 71, 515, 0), (33, 1021, 777, 0)])
+def test_any_alignment(dtype, M, N, K, split):
+    print(f"[planes any] {dtype} {M}x{N}x{K} split {split}", flush=True)
+    a, b = rng_uniform(M + K, (M, K)), rng_uniform(N + K, (K, N))
+    if dtype == "bfloat16":
+        a, b = ref.round_bf16(a), ref.round_bf16(b)
+    bias = rng_uniform(7, (N,))
+    out = run_matmul(a, b, dtype, split_k=split, relu=True, thr=-1.0, bias=bias)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    want = np.maximum(a64 @ b64 + bias, -1.0)
+    # bf16 products are exact: at most one rounding per product and per split
+    terms = K / 32 + 17 if dtype == "float32" else K + 17
+    assert np.all(np.abs(out - want) <= terms * 2.0**-24 * (np.abs(a64) @ np.abs(b64) + 1))
+    ai, bi = ref.np_init((M, K), "float32"), ref.np_init((K, N), "float32")
+    np.testing.assert_array_equal(run_matmul(ai, bi, dtype, split_k=split), ai.astype(np.float64) @ bi)
+
+
+def test_splitwave_behind_the_default_depth_of_64x64x32():
+    # the same splits in the same order: bit-identical to the template
+    a, b = rng_uniform(3, (96, 512)), rng_uniform(4, (512, 160))
+    runs = [_run_depth(a, b, "float32", (64, 64, 32, 2, 2), 4, depth, False) for depth in (0, 2, 4)]
+    np.testing.assert_array_equal(runs[0], runs[1])
+    np.testing.assert_array_equal(runs[0], runs[2])
 
 
 def test_half_zero_and_wide_operands():
@@ -83,3 +113,12 @@ def test_infinities_and_nan():
         np.testing.assert_array_equal(np.isneginf(out), np.isneginf(want))
         fin = np.isfinite(want)
         np.testing.assert_allclose(out[fin], want[fin], rtol=160 * 2.0**-24)
+
+
+def test_small_tile_edges():
+    # 64x64x32 runs here from 512 workgroups of 8 slabs unsplit
+    for M, N, K in ((1400, 1540, 260), (2050, 1028, 1000)):
+        a, b = rng_uniform(M, (M, K)), rng_uniform(N, (K, N))
+        check(run_matmul(a, b, tile=(64, 64, 32, 2, 2), split_k=1), a, b)
+    a, b = rng_uniform(8, (1004, 1200)), rng_uniform(9, (1200, 1104))
+    check(run_matmul(a, b, tile=(64, 64, 32, 2, 2), split_k=8), a, b)

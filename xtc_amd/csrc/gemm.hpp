@@ -53,7 +53,8 @@ struct GemmArgs {
   const void* B;      // [K][ldb]
   float* C;           // [M][ldc]
   const float* bias;  // [N] or null
-  float* partial;     // split-K workspace [splits][M][N] or null
+  float* partial;     // split-K workspace [splits][M][N] ([splits][M][ldp] for gemm_planes) or null
+  int ldp;            // gemm_planes: row stride of the workspace, N up to whole vectors of 4
   unsigned* counters; // split-K arrival counters [tiles_m * tiles_n], zero between launches
   int M, N, K;
   int lda, ldb, ldc;
@@ -456,7 +457,7 @@ gemm_kernel(GemmArgs args) {
     }
   }
   if (to_partial && splitk_arrive(args.counters + tile_m * args.tiles_n + tile_n, (int)gridDim.z)) {
-    splitk_finish_tile<BM, BN, NT>(args.partial, args.C, args.bias, args.M, args.N, args.ldc, (int)gridDim.z,
+    splitk_finish_tile<BM, BN, NT>(args.partial, args.N, args.C, args.bias, args.M, args.N, args.ldc, (int)gridDim.z,
                                    args.relu, args.relu_threshold, m0, n0);
     splitk_release(args.counters + tile_m * args.tiles_n + tile_n);
   }

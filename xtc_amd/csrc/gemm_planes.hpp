@@ -688,9 +688,10 @@ gemm_planes(GemmArgs args) {
 
   // ---- epilogue: lane holds C[m][n .. n+3]
   const bool to_partial = args.partial != nullptr;
-  float* const out = to_partial ? args.partial + (size_t)split * args.M * args.N : args.C;
-  const int ldo = to_partial ? args.N : args.ldc;
-  const bool vec_out = ((args.N | ldo) & 3) == 0 && ((uintptr_t)out & 15) == 0;
+  float* const out = to_partial ? args.partial + (size_t)split * args.M * args.ldp : args.C;
+  const int ldo = to_partial ? args.ldp : args.ldc;
+  // the workspace has room for whole vectors
+  const bool vec_out = to_partial || (((args.N | ldo) & 3) == 0 && ((uintptr_t)out & 15) == 0);
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
     const int n = ncol + 16 * j;
@@ -719,15 +720,12 @@ gemm_planes(GemmArgs args) {
       } else {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (n + r < args.N) {
-            if (to_partial) splitk_store(p + r, v[r]);
-            else p[r] = v[r];
-          }
+          if (n + r < args.N) p[r] = v[r];
       }
     }
   }
   if (to_partial && splitk_arrive(args.counters + tile_m * args.tiles_n + tile_n, (int)gridDim.z)) {
-    splitk_finish_tile<BM, BN, NT>(args.partial, args.C, args.bias, args.M, args.N, args.ldc, (int)gridDim.z, args.relu,
+    splitk_finish_tile<BM, BN, NT>(args.partial, args.ldp, args.C, args.bias, args.M, args.N, args.ldc, (int)gridDim.z, args.relu,
                                    args.relu_threshold, m0, n0);
     splitk_release(args.counters + tile_m * args.tiles_n + tile_n);
   }

@@ -956,7 +956,8 @@ int launch_gemm_common(GemmArgs& a, const GemmEntry* e, int split_k, int stages,
   a.partial = nullptr;
   a.counters = nullptr;
   if (splits > 1) {
-    size_t bytes = (size_t)splits * a.M * a.N * sizeof(float);
+    if (!a.ldp) a.ldp = a.N;
+    size_t bytes = (size_t)splits * a.M * a.ldp * sizeof(float);
     a.partial = x.partials(bytes);
     if (!a.partial) return 1;
     a.counters = x.counters((size_t)a.tiles_m * a.tiles_n);
@@ -1046,19 +1047,12 @@ bool skinny_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, in
   return true;
 }
 
-// gemm_planes (gemm_planes.hpp) runs fp32 matmuls on bf16 MFMAs behind the
-// 128x256x32 (2x4 waves), 256x128x32 (4x2) and 128x128x32 (2x4) tiles, any M,
-// N and K of whole 16-byte vectors, split-K included.  Against the LDS-DMA
-// kernel on fp32 MFMAs that these tiles had before: 4096^3 980 -> 631 us,
-// 2048x4096x1024 130-144 -> 88-95 us, 2048x1024x4096 at split 2 150 -> 103 us,
-// at a fifth of its error against float64.  Those tiles at a slab depth of 16
-// keep the fp32 MFMAs (gemm_f32_lds.hpp): an instruction takes 32 of k.
-const PlanesEntry* planes_entry(int dtype, int conv, int bt, int vec, const xtc_hip_tile& t, int ring) {
+const PlanesEntry* planes_entry(int dtype, int conv, int bt, int vec, const xtc_hip_tile& t) {
   int n = 0;
-  const PlanesEntry* e = planes_f32(&n);
+  const PlanesEntry* e = dtype == XTC_HIP_F32 ? planes_f32(&n) : planes_bf16(&n);
   for (int i = 0; i < n; ++i)
-    if (e[i].dtype == dtype && e[i].conv == conv && e[i].bt == bt && e[i].vec == vec && e[i].bm == t.bm &&
-        e[i].bn == t.bn && e[i].wgm == t.wgm && e[i].wgn == t.wgn && (ring == 0 || e[i].ring == ring))
+    if (e[i].conv == conv && e[i].bt == bt && e[i].vec == vec && e[i].bm == t.bm && e[i].bn == t.bn &&
+        e[i].wgm == t.wgm && e[i].wgn == t.wgn)
       return &e[i];
   return nullptr;
 }
@@ -1071,13 +1065,42 @@ bool generic_only() {
   return v;
 }
 
-// Whether gemm_planes runs a matmul whose operands are whole 16-byte vectors.
-bool planes_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int lda, int ldb) {
-  if (generic_only() || d.dtype != XTC_HIP_F32 || t.bk != 32) return false;
-  if (!planes_entry(0, 0, 0, 1, t, 0)) return false;
-  // byte offsets inside a tile's rows fit in 32 bits
-  return (int64_t)t.bm * lda <= INT32_MAX / 4 && (int64_t)(t.bk + 1) * ldb <= INT32_MAX / 4;
+// Byte offsets inside the rows of a gemm_planes tile fit in 32 bits.
+bool planes_offsets_fit(int esz, int lda, int ldb) {
+  return (int64_t)256 * lda <= INT32_MAX / esz && (int64_t)256 * ldb <= INT32_MAX / esz;
 }
+
+// Whether gemm_planes (gemm_planes.hpp: fp32 products on bf16 MFMAs) runs an
+// fp32 matmul of whole 16-byte vectors, any M, N and K.
+//  * The 8-wave tiles 128x256x32 (2x4), 256x128x32 (4x2) and 128x128x32 (2x4):
+//    always.  Against the LDS-DMA kernel on fp32 MFMAs that they had before:
+//    4096^3 980 -> 631 us, 2048x4096x1024 130-144 -> 88-99 us, 2048x1024x4096
+//    at split 2 150 -> 104 us, at a fifth of its error against float64.  These
+//    tiles at a slab depth of 16 keep the fp32 MFMAs (gemm_f32_lds.hpp): one
+//    bf16 instruction takes 32 of k.
+//  * 64x64x32: splitting both operands of so small a tile costs as many vector
+//    ALU cycles as its fp32 MFMAs take, so it wins only where several
+//    workgroups share a CU and walk K for a while (us, generic -> this):
+//    1536^2x512 unsplit 35.7 -> 28.3, 1023x5584x432 58.4 -> 48.5, 2000x2304x600
+//    66.3 -> 51.9, 405x2332x1660 split 8 53.3 -> 49.2, 256x4608x8192 split 8
+//    184 -> 153; but 512x1024x1024 split 8 (1024 workgroups of 4 slabs)
+//    18.9 -> 22.0, 300x500x2000 split 8 (320 of 7) 19.2 -> 20.8.
+bool planes_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_k, int lda, int ldb) {
+  if (generic_only() || d.dtype != XTC_HIP_F32 || t.bk != 32) return false;
+  if (!planes_entry(XTC_HIP_F32, 0, 0, 1, t) || !planes_offsets_fit(4, lda, ldb)) return false;
+  if (t.bm > 64) return true;
+  const int splits = effective_splits(d.K, split_k, t.bk);
+  const int64_t groups = (int64_t)((d.M + 63) / 64) * ((d.N + 63) / 64) * splits;
+  const int slabs = split_depth(d.K, split_k, t.bk) / 32;
+  return splits == 1 ? groups >= 512 && slabs >= 8 : groups >= 1152 && slabs >= 4;
+}
+
+// Matmuls that are not whole 16-byte vectors (strides, K, N or operand
+// addresses) run on gemm_planes behind this tile, whatever tile the descriptor
+// names: before, one thread per output walked K (fp32 509x1021x777: 214 us,
+// now 18 us at the default split 4; other blocks there: 128x64 18-24 us,
+// 128x128 26 us).
+constexpr xtc_hip_tile kPlanesAnyTile[2] = {{64, 64, 32, 2, 2}, {64, 64, 64, 2, 2}};  // fp32, bf16
 
 // The LDS-DMA fp32 kernel (gemm_f32_lds.hpp) implements the 128x256x16 (2x4
 // waves) and 256x128x16 (4x2 waves) fp32 tiles, split-K included, when the
@@ -1144,11 +1167,19 @@ bool splitwave_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t,
     return v && v[0] == '1';
   }();
   if (disabled || d.dtype != XTC_HIP_F32) return false;
-  if (t.bm != 32 || t.bn != 32 || t.bk != 16 || t.wgm != 1 || t.wgn != 1) return false;
   if (split_k < 2 || split_k > 8) return false;
   if (d.M % 32 || d.N % 32 || d.K % (16 * split_k)) return false;
   if (lda % 4 || !aligned16(A)) return false;
-  return true;
+  if (t.bm == 32 && t.bn == 32 && t.bk == 16 && t.wgm == 1 && t.wgn == 1) return true;
+  // The default depth of the 64x64x32 tile (2x2 waves of 32x32), when its
+  // 32x32 blocks fit in one wave of 256 CUs: the wave blocks become workgroups
+  // whose waves are the splits, which meet in LDS instead of memory, in the
+  // same order (the results are bit-identical when a split is whole slabs).
+  // 512^3 at split 4 11.0 -> 5.5 us, 256^3 at split 2 9.5 -> 4.9, 32x4096x1024
+  // at split 8 13.2 -> 10.7; with 512 blocks it loses (512x1024x1024 at split 8
+  // 18.9 -> 20.7 us).
+  return t.bm == 64 && t.bn == 64 && t.bk == 32 && t.wgm == 2 && t.wgn == 2 && d.stages == 0 &&
+         d.K % (32 * split_k) == 0 && (int64_t)(d.M / 32) * (d.N / 32) <= 256;
 }
 
 // Pipeline depths (register ring chunks) of the split-wave kernel, default
@@ -1527,7 +1558,7 @@ const void* transposed_copy(int slot, const void* src, int R, int Cc, int ld_src
 
 // The kernel family a matmul runs on, chosen from the shape, tile, split,
 // strides and operand alignment in the order of matmul_impl.
-enum class MatmulPath { LdsDmaBt, Naive, LdsDma, Skinny, SplitWave, Planes, F32Lds, F64, Generic };
+enum class MatmulPath { LdsDmaBt, Naive, PlanesAny, LdsDma, Skinny, SplitWave, Planes, F32Lds, F64, Generic };
 
 const char* path_name(MatmulPath p) {
   switch (p) {
@@ -1541,6 +1572,7 @@ const char* path_name(MatmulPath p) {
     case MatmulPath::SplitWave:
       return "split-wave fp32";
     case MatmulPath::Planes:
+    case MatmulPath::PlanesAny:
       return "bf16-plane";
     case MatmulPath::F32Lds:
       return "LDS-DMA fp32";
@@ -1576,11 +1608,21 @@ int path_depths(MatmulPath p, const xtc_hip_tile& t, int ring, int* out, int max
       tmp[n++] = 2;
       break;
     case MatmulPath::SplitWave:
+      if (t.bm == 64) {  // the 64x64x32 tile's own depths: its default runs here, a named one on the template
+        tmp[n++] = 4;
+        tmp[n++] = 2;
+        break;
+      }
       for (int v : kSplitWaveDepths) tmp[n++] = v;
       break;
     case MatmulPath::Planes:
       // one pipeline behind every depth a schedule may name: two LDS buffers
       // and the next slab in registers
+      if (t.bm == 64) {
+        tmp[n++] = ring == 2 ? 4 : 2;
+        tmp[n++] = ring == 2 ? 2 : 4;
+        break;
+      }
       tmp[n++] = 3;
       tmp[n++] = 2;
       if (t.bm == 128 && t.bn == 128) tmp[n++] = 4;
@@ -1591,6 +1633,7 @@ int path_depths(MatmulPath p, const xtc_hip_tile& t, int ring, int* out, int max
           tmp[n++] = v.stages;
       break;
     case MatmulPath::Naive:
+    case MatmulPath::PlanesAny:
       tmp[n++] = 1;
       break;
     case MatmulPath::F64:
@@ -1651,7 +1694,9 @@ int natural_path(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_
   const bool vec_ok = lda % vec == 0 && ldb % vec == 0 && d.K % vec == 0 && d.N % vec == 0 && aligned16(A) &&
                       aligned16(B);
   if (!vec_ok) {
-    *path = MatmulPath::Naive;
+    const bool any = !generic_only() && d.dtype != XTC_HIP_F64 &&
+                     planes_offsets_fit(d.dtype == XTC_HIP_F32 ? 4 : 2, lda, ldb);
+    *path = any ? MatmulPath::PlanesAny : MatmulPath::Naive;
     return 0;
   }
   if (d.dtype == XTC_HIP_F64) {
@@ -1669,7 +1714,7 @@ int natural_path(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_
     *path = MatmulPath::Skinny;
   else if (splitwave_gemm_applies(d, t, split_k, lda, A))
     *path = MatmulPath::SplitWave;
-  else if (planes_gemm_applies(d, t, lda, ldb))
+  else if (planes_gemm_applies(d, t, split_k, lda, ldb))
     *path = MatmulPath::Planes;
   else if (f32_lds_gemm_applies(d, t, split_k, lda, ldb, ldc, A, B, C, (const float*)bias))
     *path = MatmulPath::F32Lds;
@@ -1702,6 +1747,31 @@ int launch_f64_gemm(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int spl
   return launch_f64_common(a, f, split_k, d.group_m, d.xcd_remap, x);
 }
 
+// Row stride of the split-K workspace of gemm_planes: whole vectors of 4.
+int planes_ldp(int N) { return (N + 3) / 4 * 4; }
+
+// Splits of a launch that must not fail for want of scratch (shapes whose
+// calls took none before they ran on gemm_planes): `split_k`, or 1 where the
+// split-K scratch would pass the fixed scratch or 1 GiB, or would have to be
+// allocated while the stream is being captured.
+int splits_with_room(int split_k, int M, int N, int K, const xtc_hip_tile& t, const Scratch& x) {
+  const int splits = effective_splits(K, split_k, t.bk);
+  if (splits == 1) return 1;
+  const size_t tiles = (size_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+  const size_t bytes = (size_t)splits * M * planes_ldp(N) * sizeof(float);
+  if (x.fixed)  // two 256-byte alignments
+    return bytes + tiles * sizeof(unsigned) + 512 <= x.cap - x.used ? split_k : 1;
+  if (bytes > ((size_t)1 << 30)) return 1;
+  {
+    std::lock_guard<std::mutex> lk(g_mutex);
+    const StreamScratch* y = stream_scratch(x.s);
+    if (y && y->workspace_bytes >= bytes && y->counters_len >= tiles) return split_k;
+  }
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(x.s, &status) != hipSuccess) return 1;
+  return status == hipStreamCaptureStatusNone ? split_k : 1;
+}
+
 int matmul_impl(const xtc_hip_matmul_desc& d, const void* A, const void* B, void* Cv, const void* biasv,
                 Scratch& x) {
   float* C = (float*)Cv;
@@ -1732,8 +1802,9 @@ int matmul_impl(const xtc_hip_matmul_desc& d, const void* A, const void* B, void
   }
   MatmulPath path;
   if (natural_path(d, t, split_k, lda, ldb, ldc, A, B, C, bias, &path)) return 1;
-  const int ring =
-      path == MatmulPath::Generic ? generic_ring(find_entry(d.dtype, 0, t), effective_splits(d.K, split_k, t.bk)) : 0;
+  const int ring = path == MatmulPath::Generic || path == MatmulPath::Planes
+                       ? generic_ring(find_entry(d.dtype, 0, t), effective_splits(d.K, split_k, t.bk))
+                       : 0;
   if (check_depth(path, t, ring, d.stages)) return 1;
   if (path == MatmulPath::Naive) {
     dim3 grid(grid_for((uint64_t)d.M * d.N, 128));
@@ -1760,11 +1831,17 @@ int matmul_impl(const xtc_hip_matmul_desc& d, const void* A, const void* B, void
     return launch_splitwave_gemm(d, split_k, d.stages, lda, ldb, ldc, A, B, C, bias, s);
   const GemmEntry* e = find_entry(d.dtype, 0, t);
   GemmEntry own;
-  if (path == MatmulPath::F32Lds || path == MatmulPath::Planes) {
+  if (path == MatmulPath::PlanesAny) {
+    const xtc_hip_tile& u = kPlanesAnyTile[d.dtype];
+    own = GemmEntry{d.dtype, 0, u.bm, u.bn, u.bk, u.wgm, u.wgn, 0, 0, planes_entry(d.dtype, 0, 0, 0, u)->launch, nullptr};
+    e = &own;
+    split_k = splits_with_room(split_k, d.M, d.N, d.K, u, x);
+  } else if (path == MatmulPath::F32Lds || path == MatmulPath::Planes) {
     // same tiles, split-K set-up and grid as the generic instance; only the
     // kernel differs
     own = *e;
-    own.launch = path == MatmulPath::F32Lds ? f32_lds_variant(t, d.stages)->launch : planes_entry(0, 0, 0, 1, t, 0)->launch;
+    own.launch = path == MatmulPath::F32Lds ? f32_lds_variant(t, d.stages)->launch
+                                            : planes_entry(d.dtype, 0, 0, 1, t)->launch;
     own.launch_ring = nullptr;
     e = &own;
   }
@@ -1782,6 +1859,7 @@ int matmul_impl(const xtc_hip_matmul_desc& d, const void* A, const void* B, void
   a.ldc = ldc;
   a.relu = d.relu;
   a.relu_threshold = d.relu_threshold;
+  if (path == MatmulPath::Planes || path == MatmulPath::PlanesAny) a.ldp = planes_ldp(d.N);
   return launch_gemm_common(a, e, split_k, path == MatmulPath::Generic ? d.stages : 0, d.group_m, d.xcd_remap, x);
 }
 
@@ -2071,8 +2149,9 @@ int xtc_hip_matmul_pipeline_depths(const xtc_hip_matmul_desc* desc, int* depths,
     if (d.trans_b) ldb = d.N;
     if (natural_path(d, t, split_k, lda, ldb, ldc, p, p, p, nullptr, &path)) return -1;
   }
-  const int ring =
-      path == MatmulPath::Generic ? generic_ring(find_entry(d.dtype, 0, t), effective_splits(d.K, split_k, t.bk)) : 0;
+  const int ring = path == MatmulPath::Generic || path == MatmulPath::Planes
+                       ? generic_ring(find_entry(d.dtype, 0, t), effective_splits(d.K, split_k, t.bk))
+                       : 0;
   return path_depths(path, t, ring, depths, max_depths);
 }
 

@@ -171,37 +171,47 @@ __device__ __forceinline__ void splitk_release(unsigned* counter) {
 }
 
 // The last workgroup's sum over one BM x BN output tile at (m0, n0):
-// C[m][n] = epilogue( sum_s partial[s][m][n] ), partial is [splits][M][N].
-// Four columns per thread when N, ldc and the pointers allow it; the sums
-// are the same element by element either way.
+// C[m][n] = epilogue( sum_s partial[s][m][n] ), partial is [splits][M][ldp].
+// Four columns per thread when ldp and the workspace allow it; the sums are
+// the same element by element either way.
 template <int BM, int BN, int NT>
-__device__ __forceinline__ void splitk_finish_tile(const float* partial, float* C, const float* bias, int M,
+__device__ __forceinline__ void splitk_finish_tile(const float* partial, int ldp, float* C, const float* bias, int M,
                                                    int N, int ldc, int splits, int relu, float thr, int m0,
                                                    int n0) {
   using splitk::f32x4;
-  const size_t plane = (size_t)M * N;
+  const size_t plane = (size_t)M * ldp;
   const int tid = threadIdx.x;
-  const bool vec = BN % 4 == 0 && ((N | ldc) & 3) == 0 && (((uintptr_t)C | (uintptr_t)partial) & 15) == 0 &&
-                   (bias == nullptr || ((uintptr_t)bias & 15) == 0);
-  if (vec) {
+  if (BN % 4 == 0 && (ldp & 3) == 0 && ((uintptr_t)partial & 15) == 0) {
+    const bool vec_out = ((N | ldc) & 3) == 0 && (((uintptr_t)C | (uintptr_t)bias) & 15) == 0;
     for (int idx = tid; idx < BM * BN / 4; idx += NT) {
       const int m = m0 + idx / (BN / 4);
       const int n = n0 + 4 * (idx % (BN / 4));
       if (m >= M || n >= N) continue;
-      f32x4 v = splitk_sum4(partial + (size_t)m * N + n, plane, splits);
-      if (bias) v += *(const f32x4*)(bias + n);
-      if (relu) {
+      f32x4 v = splitk_sum4(partial + (size_t)m * ldp + n, plane, splits);
+      if (vec_out) {
+        if (bias) v += *(const f32x4*)(bias + n);
+        if (relu) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = v[r] < thr ? thr : v[r];
+          for (int r = 0; r < 4; ++r) v[r] = v[r] < thr ? thr : v[r];
+        }
+        *(f32x4*)(C + (size_t)m * ldc + n) = v;
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (n + r >= N) break;
+          float x = v[r];
+          if (bias) x += bias[n + r];
+          if (relu && x < thr) x = thr;
+          C[(size_t)m * ldc + n + r] = x;
+        }
       }
-      *(f32x4*)(C + (size_t)m * ldc + n) = v;
     }
   } else {
     for (int idx = tid; idx < BM * BN; idx += NT) {
       const int m = m0 + idx / BN;
       const int n = n0 + idx % BN;
       if (m >= M || n >= N) continue;
-      float v = splitk_sum1(partial + (size_t)m * N + n, plane, splits);
+      float v = splitk_sum1(partial + (size_t)m * ldp + n, plane, splits);
       if (bias) v += bias[n];
       if (relu && v < thr) v = thr;
       C[(size_t)m * ldc + n] = v;
