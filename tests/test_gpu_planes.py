@@ -16,7 +16,7 @@ import numpy as np
 import pytest
 
 from oracle import reference as ref
-from test_gpu_kernels import _run_depth, needs_specialised, rng_uniform, run_matmul
+from test_gpu_kernels import _run_depth, needs_specialised, rng_uniform, run_matmul, run_matmul_layout
 from xtc_amd.runtimes.hip.buffer import ensure_device
 
 pytestmark = [pytest.mark.gpu, needs_specialised]
@@ -77,6 +77,19 @@ def test_splitwave_behind_the_default_depth_of_64x64x32():
     runs = [_run_depth(a, b, "float32", (64, 64, 32, 2, 2), 4, depth, False) for depth in (0, 2, 4)]
     np.testing.assert_array_equal(runs[0], runs[1])
     np.testing.assert_array_equal(runs[0], runs[2])
+
+
+# B stored transposed, read in place: rows of B^T cut by N, slabs cut by K
+@pytest.mark.parametrize("dtype,tile", [("float32", TILES[0]), ("float32", TILES[1]), ("float32", TILES[2]),
+                                        ("float32", (64, 64, 32, 2, 2)), ("bfloat16", (64, 64, 64, 2, 2)),
+                                        ("bfloat16", (128, 128, 64, 2, 2))])
+@pytest.mark.parametrize("M,N,K,split", [(1, 8, 8, 1), (130, 264, 136, 1), (257, 136, 1048, 3)])
+def test_transposed_b(dtype, tile, M, N, K, split):
+    print(f"[planes bt] {dtype} {tile} {M}x{N}x{K} split {split}", flush=True)
+    ai, bi = ref.np_init((M, K), "float32"), ref.np_init((K, N), "float32")[::-1].copy()
+    for bt in (True, False):
+        out = run_matmul_layout(ai, bi, dtype, False, bt, tile=tile, split_k=split, pad_a=8, pad_b=16)
+        np.testing.assert_array_equal(out, ai.astype(np.float64) @ bi)
 
 
 def test_half_zero_and_wide_operands():

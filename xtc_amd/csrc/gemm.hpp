@@ -457,7 +457,7 @@ gemm_kernel(GemmArgs args) {
     }
   }
   if (to_partial && splitk_arrive(args.counters + tile_m * args.tiles_n + tile_n, (int)gridDim.z)) {
-    splitk_finish_tile<BM, BN, NT>(args.partial, args.N, args.C, args.bias, args.M, args.N, args.ldc, (int)gridDim.z,
+    splitk_finish_tile<BM, BN, NT>(args.partial, (size_t)args.M * args.N, args.N, args.C, args.bias, args.M, args.N, args.ldc, (int)gridDim.z,
                                    args.relu, args.relu_threshold, m0, n0);
     splitk_release(args.counters + tile_m * args.tiles_n + tile_n);
   }

@@ -220,7 +220,7 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512))) gemm_bf16
     // reads and DMAs are complete before the barrier that opens the arrival
     unsigned* counter = args.counters + tile_m * args.tiles_n + tile_n;
     if (splitk_arrive_in(counter, (int)gridDim.z, reinterpret_cast<unsigned*>(st0))) {
-      splitk_finish_tile<BM, BN, 512>(args.partial, args.N, args.C, args.bias, args.M, args.N, args.ldc, (int)gridDim.z,
+      splitk_finish_tile<BM, BN, 512>(args.partial, (size_t)args.M * args.N, args.N, args.C, args.bias, args.M, args.N, args.ldc, (int)gridDim.z,
                                       args.relu, args.relu_threshold, m0, n0);
       splitk_release(counter);
     }

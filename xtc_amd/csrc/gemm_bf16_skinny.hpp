@@ -186,23 +186,9 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(256, 256))) gemm_bf16
   }
   if (direct || !splitk_arrive(args.counters + nb, splits)) return;
 
-  // ---- last workgroup of the column block: C[m][n0 + 4c .. +3] =
-  // epilogue( sum_s W[s][m][...] ), 16 x 32 float4 over 256 threads
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int idx = tid + 256 * q;
-    const int m = idx >> 5;
-    const int n = n0 + 4 * (idx & 31);
-    if (m < args.M) {
-      f32x4 v = splitk_sum4(args.W + (size_t)m * args.ldw + n, (size_t)16 * args.ldw, splits);
-      if (args.bias) v += *(const f32x4*)(args.bias + n);
-      if (args.relu) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = v[r] < args.relu_threshold ? args.relu_threshold : v[r];
-      }
-      *(f32x4*)(args.C + (size_t)m * args.ldc + n) = v;
-    }
-  }
+  // ---- last workgroup of the column block
+  splitk_finish_tile<16, BN, 256>(args.W, (size_t)16 * args.ldw, args.ldw, args.C, args.bias, args.M, args.N, args.ldc,
+                                  splits, args.relu, args.relu_threshold, 0, n0);
   splitk_release(args.counters + nb);
 }
 

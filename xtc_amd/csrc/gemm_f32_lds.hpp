@@ -249,7 +249,7 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512))) gemm_f32_
     for (int j = 0; j < TN; ++j) splitk_store4(row + ncol + 16 * j, acc[i][j]);
   }
   if (splitk_arrive(args.counters + tile_m * args.tiles_n + tile_n, (int)gridDim.z)) {
-    splitk_finish_tile<BM, BN, 512>(args.partial, args.N, args.C, args.bias, args.M, args.N, args.ldc, (int)gridDim.z,
+    splitk_finish_tile<BM, BN, 512>(args.partial, (size_t)args.M * args.N, args.N, args.C, args.bias, args.M, args.N, args.ldc, (int)gridDim.z,
                                     args.relu, args.relu_threshold, m0, n0);
     splitk_release(args.counters + tile_m * args.tiles_n + tile_n);
   }

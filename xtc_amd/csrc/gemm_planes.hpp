@@ -725,7 +725,7 @@ gemm_planes(GemmArgs args) {
     }
   }
   if (to_partial && splitk_arrive(args.counters + tile_m * args.tiles_n + tile_n, (int)gridDim.z)) {
-    splitk_finish_tile<BM, BN, NT>(args.partial, args.ldp, args.C, args.bias, args.M, args.N, args.ldc, (int)gridDim.z, args.relu,
+    splitk_finish_tile<BM, BN, NT>(args.partial, (size_t)args.M * args.ldp, args.ldp, args.C, args.bias, args.M, args.N, args.ldc, (int)gridDim.z, args.relu,
                                    args.relu_threshold, m0, n0);
     splitk_release(args.counters + tile_m * args.tiles_n + tile_n);
   }

@@ -1085,14 +1085,36 @@ bool planes_offsets_fit(int esz, int lda, int ldb) {
 //    66.3 -> 51.9, 405x2332x1660 split 8 53.3 -> 49.2, 256x4608x8192 split 8
 //    184 -> 153; but 512x1024x1024 split 8 (1024 workgroups of 4 slabs)
 //    18.9 -> 22.0, 300x500x2000 split 8 (320 of 7) 19.2 -> 20.8.
+//  * bf16 (one plane) 128x128x64 and 64x64x64 (2x2 waves): always.  Transposing
+//    LDS reads instead of byte permutes on the way in, loads a step ahead
+//    without bounds branches (us, generic -> this): 2000x2304x2600 68 -> 54,
+//    256x8192x4608 split 4 49 -> 43, 1000x1104x1200 24.2 -> 14.3, 512x1024x1024
+//    split 4 12.4 -> 10.6.
 bool planes_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_k, int lda, int ldb) {
-  if (generic_only() || d.dtype != XTC_HIP_F32 || t.bk != 32) return false;
-  if (!planes_entry(XTC_HIP_F32, 0, 0, 1, t) || !planes_offsets_fit(4, lda, ldb)) return false;
-  if (t.bm > 64) return true;
+  if (generic_only() || d.dtype == XTC_HIP_F64) return false;
+  const bool f32 = d.dtype == XTC_HIP_F32;
+  if (t.bk != (f32 ? 32 : 64) || !planes_entry(d.dtype, 0, 0, 1, t)) return false;
+  if (!planes_offsets_fit(f32 ? 4 : 2, lda, ldb)) return false;
+  if (!f32 || t.bm > 64) return true;
   const int splits = effective_splits(d.K, split_k, t.bk);
   const int64_t groups = (int64_t)((d.M + 63) / 64) * ((d.N + 63) / 64) * splits;
   const int slabs = split_depth(d.K, split_k, t.bk) / 32;
   return splits == 1 ? groups >= 512 && slabs >= 8 : groups >= 1152 && slabs >= 4;
+}
+
+bool splitwave_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_k, int lda, const void* A);
+
+// Whether gemm_planes reads B^T [N][ldb] in place behind tile t (the same
+// tiles, any grid but the small ones of the split-wave kernel): the other
+// kernels need a transposed copy of B first, which for 4608x8192 bf16 took
+// 31 us of a 96 us product.
+bool planes_bt_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_k, int lda, int ldb,
+                       const void* A, const void* B) {
+  if (generic_only() || d.dtype == XTC_HIP_F64) return false;
+  const int vec = d.dtype == XTC_HIP_F32 ? 4 : 8;
+  if (t.bk != (vec == 4 ? 32 : 64) || !planes_entry(d.dtype, 0, 1, 1, t)) return false;
+  if (lda % vec || ldb % vec || d.K % vec || d.N % vec || !aligned16(A) || !aligned16(B)) return false;
+  return planes_offsets_fit(vec == 4 ? 4 : 2, lda, ldb) && !splitwave_gemm_applies(d, t, split_k, lda, A);
 }
 
 // Matmuls that are not whole 16-byte vectors (strides, K, N or operand
@@ -1618,6 +1640,10 @@ int path_depths(MatmulPath p, const xtc_hip_tile& t, int ring, int* out, int max
     case MatmulPath::Planes:
       // one pipeline behind every depth a schedule may name: two LDS buffers
       // and the next slab in registers
+      if (t.bk == 64 && t.bm == 128) {
+        tmp[n++] = 2;
+        break;
+      }
       if (t.bm == 64) {
         tmp[n++] = ring == 2 ? 4 : 2;
         tmp[n++] = ring == 2 ? 2 : 4;
@@ -1782,26 +1808,27 @@ int matmul_impl(const xtc_hip_matmul_desc& d, const void* A, const void* B, void
   if (resolve_matmul(d, &lda, &ldb, &ldc, &t, &split_k)) return 1;
   const bool ta = d.trans_a != 0, tb = d.trans_b != 0;
   const hipStream_t s = x.s;
-  // B stored transposed feeds the LDS-DMA kernel directly (B^T tiles are
-  // read like A tiles); every other transposed operand gets a natural copy
-  // in a staging buffer first (one HBM-bound transpose).
+  // B stored transposed feeds the LDS-DMA kernel and gemm_planes directly
+  // (B^T tiles are read like A tiles); every other transposed operand gets a
+  // natural copy in a staging buffer first (one HBM-bound transpose).
   if (tb && !ta && lds_dma_gemm_applies(d, t, split_k, lda, ldb, ldc, A, B, C, bias, true)) {
     if (check_depth(MatmulPath::LdsDmaBt, t, 0, d.stages)) return 1;
     return launch_lds_dma_gemm(d, t, split_k, d.stages, lda, ldb, ldc, A, B, C, bias, x, true);
   }
+  const bool bt = tb && !ta && planes_bt_applies(d, t, split_k, lda, ldb, A, B);
   const int esz = d.dtype == XTC_HIP_F64 ? 8 : d.dtype == XTC_HIP_F32 ? 4 : 2;
   if (ta) {
     A = transposed_copy(0, A, d.K, d.M, lda, esz, x);
     if (!A) return 1;
     lda = d.K;
   }
-  if (tb) {
+  if (tb && !bt) {
     B = transposed_copy(1, B, d.N, d.K, ldb, esz, x);
     if (!B) return 1;
     ldb = d.N;
   }
-  MatmulPath path;
-  if (natural_path(d, t, split_k, lda, ldb, ldc, A, B, C, bias, &path)) return 1;
+  MatmulPath path = MatmulPath::Planes;
+  if (!bt && natural_path(d, t, split_k, lda, ldb, ldc, A, B, C, bias, &path)) return 1;
   const int ring = path == MatmulPath::Generic || path == MatmulPath::Planes
                        ? generic_ring(find_entry(d.dtype, 0, t), effective_splits(d.K, split_k, t.bk))
                        : 0;
@@ -1841,7 +1868,7 @@ int matmul_impl(const xtc_hip_matmul_desc& d, const void* A, const void* B, void
     // kernel differs
     own = *e;
     own.launch = path == MatmulPath::F32Lds ? f32_lds_variant(t, d.stages)->launch
-                                            : planes_entry(d.dtype, 0, 0, 1, t)->launch;
+                                            : planes_entry(d.dtype, 0, bt, 1, t)->launch;
     own.launch_ring = nullptr;
     e = &own;
   }
@@ -2144,6 +2171,8 @@ int xtc_hip_matmul_pipeline_depths(const xtc_hip_matmul_desc* desc, int* depths,
   MatmulPath path;
   if (d.trans_b && !d.trans_a && lds_dma_gemm_applies(d, t, split_k, lda, ldb, ldc, p, p, p, nullptr, true)) {
     path = MatmulPath::LdsDmaBt;
+  } else if (d.trans_b && !d.trans_a && planes_bt_applies(d, t, split_k, lda, ldb, p, p)) {
+    path = MatmulPath::Planes;
   } else {
     if (d.trans_a) lda = d.K;
     if (d.trans_b) ldb = d.N;

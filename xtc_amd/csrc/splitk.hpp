@@ -13,8 +13,8 @@
 //      workgroup synchronises and one lane increments the tile's arrival
 //      counter (agent-scope atomic add);
 //   3. the workgroup that sees splits-1 is the last one: it reads the
-//      partials back with sc1 loads (16 bytes, or 4-byte agent-scope atomic
-//      loads), sums partial[0..splits-1] in split order (the result does not
+//      partials back with sc1 loads (16 bytes, 16 in flight per lane, or
+//      4-byte agent-scope atomic loads), sums partial[0..splits-1] in split order (the result does not
 //      depend on which workgroup arrived last), applies bias / relu, stores C
 //      and sets the counter back to 0 for the next launch.
 // Every access to the published data carries the agent-scope policy, so no
@@ -31,6 +31,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 namespace xtc_hip {
 
@@ -61,73 +63,14 @@ __device__ __forceinline__ void splitk_store4(float* p, splitk::f32x4 v) {
                : "memory");
 }
 
-__device__ __forceinline__ splitk::f32x4 splitk_load4(const float* p) {
-  uint64_t* q = reinterpret_cast<uint64_t*>(const_cast<float*>(p));
-  const uint64_t lo = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const uint64_t hi = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return splitk::f32x4{__uint_as_float((unsigned)lo), __uint_as_float((unsigned)(lo >> 32)),
-                       __uint_as_float((unsigned)hi), __uint_as_float((unsigned)(hi >> 32))};
-}
-
-// Loads of 16 bytes with the agent-scope cache policy (sc1), from asm; each
-// asm block waits for its own loads (s_waitcnt vmcnt(0)) before its outputs
-// are defined.
-#define XTC_SPLITK_LD(i, a) "global_load_dwordx4 %" #i ", %" #a ", off sc1\n\t"
-__device__ __forceinline__ void splitk_ld8(splitk::f32x4* t, const float* p, size_t stride) {
-  asm volatile(XTC_SPLITK_LD(0, 8) XTC_SPLITK_LD(1, 9) XTC_SPLITK_LD(2, 10) XTC_SPLITK_LD(3, 11)
-               XTC_SPLITK_LD(4, 12) XTC_SPLITK_LD(5, 13) XTC_SPLITK_LD(6, 14) XTC_SPLITK_LD(7, 15) "s_waitcnt vmcnt(0)"
-               : "=&v"(t[0]), "=&v"(t[1]), "=&v"(t[2]), "=&v"(t[3]), "=&v"(t[4]), "=&v"(t[5]), "=&v"(t[6]),
-                 "=&v"(t[7])
-               : "v"(p), "v"(p + stride), "v"(p + 2 * stride), "v"(p + 3 * stride), "v"(p + 4 * stride),
-                 "v"(p + 5 * stride), "v"(p + 6 * stride), "v"(p + 7 * stride)
-               : "memory");
-}
-__device__ __forceinline__ void splitk_ld4(splitk::f32x4* t, const float* p, size_t stride) {
-  asm volatile(XTC_SPLITK_LD(0, 4) XTC_SPLITK_LD(1, 5) XTC_SPLITK_LD(2, 6) XTC_SPLITK_LD(3, 7) "s_waitcnt vmcnt(0)"
-               : "=&v"(t[0]), "=&v"(t[1]), "=&v"(t[2]), "=&v"(t[3])
-               : "v"(p), "v"(p + stride), "v"(p + 2 * stride), "v"(p + 3 * stride)
-               : "memory");
-}
-__device__ __forceinline__ void splitk_ld2(splitk::f32x4* t, const float* p, size_t stride) {
-  asm volatile(XTC_SPLITK_LD(0, 2) XTC_SPLITK_LD(1, 3) "s_waitcnt vmcnt(0)"
-               : "=&v"(t[0]), "=&v"(t[1])
-               : "v"(p), "v"(p + stride)
-               : "memory");
-}
-__device__ __forceinline__ void splitk_ld1(splitk::f32x4* t, const float* p) {
-  asm volatile(XTC_SPLITK_LD(0, 1) "s_waitcnt vmcnt(0)" : "=&v"(t[0]) : "v"(p) : "memory");
-}
-#undef XTC_SPLITK_LD
-
-// sum_{s < splits} p[s * stride] in split order, starting from +0.0, up to 8
-// loads in flight.  Only the splits that exist are loaded: these loads go
-// past the L2.
-__device__ __forceinline__ splitk::f32x4 splitk_sum4(const float* p, size_t stride, int splits) {
-  splitk::f32x4 v = {0.f, 0.f, 0.f, 0.f};
-  splitk::f32x4 t[8];
-  int s = 0;
-  for (; s + 8 <= splits; s += 8) {
-    splitk_ld8(t, p + (size_t)s * stride, stride);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v += t[j];
-  }
-  if (s + 4 <= splits) {
-    splitk_ld4(t, p + (size_t)s * stride, stride);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v += t[j];
-    s += 4;
-  }
-  if (s + 2 <= splits) {
-    splitk_ld2(t, p + (size_t)s * stride, stride);
-    v += t[0];
-    v += t[1];
-    s += 2;
-  }
-  if (s < splits) {
-    splitk_ld1(t, p + (size_t)s * stride);
-    v += t[0];
-  }
-  return v;
+// The 16 bytes at byte `off` past the uniform address p, with the agent-scope
+// cache policy (sc1).  A buffer load, so that the compiler counts it and many
+// stay in flight.
+__device__ __forceinline__ splitk::f32x4 splitk_load4(const float* p, unsigned off) {
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  constexpr int kWords = 0x00027000, kSc1 = 16;  // raw 32-bit data format; gfx940 cache policy bit sc1
+  const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, 0x7fffffff, kWords);
+  return __builtin_bit_cast(splitk::f32x4, (u32x4)__builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, kSc1));
 }
 
 __device__ __forceinline__ float splitk_sum1(const float* p, size_t stride, int splits) {
@@ -171,38 +114,81 @@ __device__ __forceinline__ void splitk_release(unsigned* counter) {
 }
 
 // The last workgroup's sum over one BM x BN output tile at (m0, n0):
-// C[m][n] = epilogue( sum_s partial[s][m][n] ), partial is [splits][M][ldp].
+// C[m][n] = epilogue( sum_s partial[s * plane + m * ldp + n] ).
 // Four columns per thread when ldp and the workspace allow it; the sums are
 // the same element by element either way.
 template <int BM, int BN, int NT>
-__device__ __forceinline__ void splitk_finish_tile(const float* partial, int ldp, float* C, const float* bias, int M,
-                                                   int N, int ldc, int splits, int relu, float thr, int m0,
-                                                   int n0) {
+__device__ __forceinline__ void splitk_finish_tile(const float* partial, size_t plane, int ldp, float* C,
+                                                   const float* bias, int M, int N, int ldc, int splits, int relu,
+                                                   float thr, int m0, int n0) {
   using splitk::f32x4;
-  const size_t plane = (size_t)M * ldp;
   const int tid = threadIdx.x;
-  if (BN % 4 == 0 && (ldp & 3) == 0 && ((uintptr_t)partial & 15) == 0) {
+  if (BN % 4 == 0 && (ldp & 3) == 0 && ((uintptr_t)partial & 15) == 0 && (int64_t)BM * ldp < (1 << 29)) {
     const bool vec_out = ((N | ldc) & 3) == 0 && (((uintptr_t)C | (uintptr_t)bias) & 15) == 0;
-    for (int idx = tid; idx < BM * BN / 4; idx += NT) {
-      const int m = m0 + idx / (BN / 4);
-      const int n = n0 + 4 * (idx % (BN / 4));
-      if (m >= M || n >= N) continue;
-      f32x4 v = splitk_sum4(partial + (size_t)m * ldp + n, plane, splits);
-      if (vec_out) {
-        if (bias) v += *(const f32x4*)(bias + n);
-        if (relu) {
+    // U quads of columns per thread at once, several splits of each: the loads go
+    // past the L2, so it is their round trips that count.  One quad of 4
+    // splits at a time took 14 us of a 46 us 256x8192x4608 bf16 product.
+    constexpr int QUADS = BM * BN / 4, PER = (QUADS + NT - 1) / NT;
+    constexpr int U = PER < 4 ? PER : 4;
+    const float* const tile = partial + (size_t)m0 * ldp + n0;
+    for (int i0 = 0; i0 < PER; i0 += U) {
+      f32x4 v[U];
+      unsigned off[U];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = v[r] < thr ? thr : v[r];
-        }
-        *(f32x4*)(C + (size_t)m * ldc + n) = v;
-      } else {
+      for (int u = 0; u < U; ++u) {
+        // quads outside the tile or the matrix read the tile's first
+        const int idx = tid + (i0 + u) * NT;
+        const int dm = idx / (BN / 4), dn = 4 * (idx % (BN / 4));
+        const bool in = idx < QUADS && m0 + dm < M && n0 + dn < N;
+        off[u] = in ? ((unsigned)dm * (unsigned)ldp + dn) * 4u : 0u;
+        v[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+      // only the splits that exist, in order, at most 16 loads in flight
+      auto add = [&](int s0, auto count) {
+        constexpr int C = decltype(count)::value;
+        f32x4 t[C][U];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          if (n + r >= N) break;
-          float x = v[r];
-          if (bias) x += bias[n + r];
-          if (relu && x < thr) x = thr;
-          C[(size_t)m * ldc + n + r] = x;
+        for (int j = 0; j < C; ++j)
+#pragma unroll
+          for (int u = 0; u < U; ++u) t[j][u] = splitk_load4(tile + (size_t)(s0 + j) * plane, off[u]);
+#pragma unroll
+        for (int j = 0; j < C; ++j)
+#pragma unroll
+          for (int u = 0; u < U; ++u) v[u] += t[j][u];
+      };
+      int s0 = 0;
+      if constexpr (U <= 2) {
+        for (; s0 + 8 <= splits; s0 += 8) add(s0, std::integral_constant<int, 8>{});
+      }
+      for (; s0 + 4 <= splits; s0 += 4) add(s0, std::integral_constant<int, 4>{});
+      if (s0 + 2 <= splits) {
+        add(s0, std::integral_constant<int, 2>{});
+        s0 += 2;
+      }
+      if (s0 < splits) add(s0, std::integral_constant<int, 1>{});
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int idx = tid + (i0 + u) * NT;
+        const int m = m0 + idx / (BN / 4);
+        const int n = n0 + 4 * (idx % (BN / 4));
+        if (idx >= QUADS || m >= M || n >= N) continue;
+        if (vec_out) {
+          f32x4 x = v[u];
+          if (bias) x += *(const f32x4*)(bias + n);
+          if (relu) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[r] = x[r] < thr ? thr : x[r];
+          }
+          *(f32x4*)(C + (size_t)m * ldc + n) = x;
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            if (n + r >= N) break;
+            float x = v[u][r];
+            if (bias) x += bias[n + r];
+            if (relu && x < thr) x = thr;
+            C[(size_t)m * ldc + n + r] = x;
+          }
         }
       }
     }
