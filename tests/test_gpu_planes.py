@@ -16,7 +16,7 @@ import numpy as np
 import pytest
 
 from oracle import reference as ref
-from test_gpu_kernels import _run_depth, needs_specialised, rng_uniform, run_matmul, run_matmul_layout
+from test_gpu_kernels import _run_depth, needs_specialised, rng_uniform, run_conv, run_matmul, run_matmul_layout
 from xtc_amd.runtimes.hip.buffer import ensure_device
 
 pytestmark = [pytest.mark.gpu, needs_specialised]
@@ -53,7 +53,7 @@ def test_edges(tile, M, N, K, split):
 # no whole vectors anywhere: fp32 and bf16 rows at element alignment, units cut
 # by K and N, tiles cut by M and N, split-K partial rows of whole vectors
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("M,N,K,split", [(1, 1, 1, 1), (3, 5, 7, 1), (64, 65, 63, 1), (67, 129, 131, 1),
+@pytest.mark.parametrize("M,N,K,split", [(1, 1, 33, 1), (3, 5, 37, 1), (64, 65, 63, 1), (67, 129, 131, 1),
                                          (130, 63, 257, 2), (65, 71, 515, 0), (33, 1021, 777, 0)])
 def test_any_alignment(dtype, M, N, K, split):
     print(f"[planes any] {dtype} {M}x{N}x{K} split {split}", flush=True)
@@ -135,3 +135,49 @@ def test_small_tile_edges():
         check(run_matmul(a, b, tile=(64, 64, 32, 2, 2), split_k=1), a, b)
     a, b = rng_uniform(8, (1004, 1200)), rng_uniform(9, (1200, 1104))
     check(run_matmul(a, b, tile=(64, 64, 32, 2, 2), split_k=8), a, b)
+
+
+def check_conv(dtype, n, h, w, c, f, r, s, stride, pads, pad_value, tile, split):
+    print(f"[planes conv] {dtype} {(n, h, w, c, f, r, s)} stride {stride} pads {pads} {tile} split {split}", flush=True)
+    rng = np.random.default_rng(h * w + c)
+    x = rng.integers(-3, 4, (n, h, w, c)).astype(np.float32)
+    wt = rng.integers(-2, 3, (r, s, c, f)).astype(np.float32)
+    bias = rng.integers(-2, 3, f).astype(np.float32)
+    out = run_conv(x, wt, dtype, stride, pads, pad_value, tile, split_k=split, bias=bias)
+    xp = ref.pad(x, [(0, 0), pads[:2], pads[2:], (0, 0)], pad_value)
+    np.testing.assert_array_equal(out, (ref.conv2d(xp, wt, stride) + bias).astype(np.float32))
+
+
+# channels and filters of no whole vector: windows that leave the image on
+# every side, runs of S C elements shorter and longer than a unit and a slab
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("n,h,w,c,f,r,s,stride,pads,pad_value,split", [
+    (1, 5, 4, 35, 1, 1, 1, (1, 1), (0, 0, 0, 0), 0.0, 0),
+    (2, 9, 7, 3, 64, 3, 3, (1, 1), (1, 1, 1, 1), 0.0, 1),
+    (1, 17, 15, 3, 24, 7, 7, (2, 2), (3, 2, 1, 3), 2.0, 2),
+    (1, 12, 11, 5, 7, 2, 3, (2, 1), (1, 0, 2, 1), -1.0, 0),
+    (1, 10, 10, 37, 66, 3, 3, (1, 2), (0, 2, 1, 0), 0.0, 3),
+    (3, 70, 72, 3, 72, 3, 3, (1, 1), (1, 1, 1, 1), 1.0, 1),
+])
+def test_conv_any_alignment(dtype, n, h, w, c, f, r, s, stride, pads, pad_value, split):
+    check_conv(dtype, n, h, w, c, f, r, s, stride, pads, pad_value, None, split)
+
+
+@pytest.mark.parametrize("dtype,tile", [("bfloat16", (64, 64, 64, 2, 2)), ("bfloat16", (128, 64, 64, 2, 2)),
+                                        ("bfloat16", (128, 128, 64, 2, 2)), ("float32", (64, 64, 32, 2, 2)),
+                                        ("float32", (64, 64, 16, 2, 2))])
+@pytest.mark.parametrize("n,h,w,c,f,r,s,stride,pads,pad_value,split", [
+    (1, 9, 10, 8, 8, 1, 1, (1, 1), (0, 0, 0, 0), 0.0, 1),
+    (2, 13, 11, 24, 72, 3, 3, (2, 1), (1, 2, 0, 1), 2.0, 2),
+    (1, 182, 182, 32, 40, 3, 3, (1, 1), (1, 1, 1, 1), -1.0, 1),
+])
+def test_conv_vectors(dtype, tile, n, h, w, c, f, r, s, stride, pads, pad_value, split):
+    check_conv(dtype, n, h, w, c, f, r, s, stride, pads, pad_value, tile, split)
+
+
+def test_conv_infinite_pad():
+    x, wt = np.ones((1, 6, 6, 3), np.float32), np.ones((3, 3, 3, 8), np.float32)
+    out = run_conv(x, wt, "float32", (1, 1), (1, 1, 1, 1), float("inf"))
+    want = np.full((1, 6, 6, 8), np.inf, np.float32)
+    want[:, 1:5, 1:5] = 27
+    np.testing.assert_array_equal(out, want)

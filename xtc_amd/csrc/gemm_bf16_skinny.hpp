@@ -186,9 +186,16 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(256, 256))) gemm_bf16
   }
   if (direct || !splitk_arrive(args.counters + nb, splits)) return;
 
-  // ---- last workgroup of the column block
-  splitk_finish_tile<16, BN, 256>(args.W, (size_t)16 * args.ldw, args.ldw, args.C, args.bias, args.M, args.N, args.ldc,
-                                  splits, args.relu, args.relu_threshold, 0, n0);
+  // ---- last workgroup of the column block: one or two columns per thread
+  auto finish = [&](auto rows) {
+    splitk_finish_tile<decltype(rows)::value, BN, 256>(args.W, (size_t)16 * args.ldw, args.ldw, args.C, args.bias,
+                                                       args.M, args.N, args.ldc, splits, args.relu,
+                                                       args.relu_threshold, 0, n0);
+  };
+  if (args.M <= 8)
+    finish(std::integral_constant<int, 8>{});
+  else
+    finish(std::integral_constant<int, 16>{});
   splitk_release(args.counters + nb);
 }
 

@@ -29,5 +29,6 @@ PlanesEntry planes_instance() {
 // Filled by planes_*.hip.
 const PlanesEntry* planes_f32(int* count);
 const PlanesEntry* planes_bf16(int* count);
+const PlanesEntry* planes_conv(int* count);
 
 }  // namespace xtc_hip

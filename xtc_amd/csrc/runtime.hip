@@ -1049,9 +1049,9 @@ bool skinny_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, in
 
 const PlanesEntry* planes_entry(int dtype, int conv, int bt, int vec, const xtc_hip_tile& t) {
   int n = 0;
-  const PlanesEntry* e = dtype == XTC_HIP_F32 ? planes_f32(&n) : planes_bf16(&n);
+  const PlanesEntry* e = conv ? planes_conv(&n) : dtype == XTC_HIP_F32 ? planes_f32(&n) : planes_bf16(&n);
   for (int i = 0; i < n; ++i)
-    if (e[i].conv == conv && e[i].bt == bt && e[i].vec == vec && e[i].bm == t.bm && e[i].bn == t.bn &&
+    if (e[i].dtype == dtype && e[i].conv == conv && e[i].bt == bt && e[i].vec == vec && e[i].bm == t.bm && e[i].bn == t.bn &&
         e[i].wgm == t.wgm && e[i].wgn == t.wgn)
       return &e[i];
   return nullptr;
@@ -1102,6 +1102,36 @@ bool planes_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, in
   return splits == 1 ? groups >= 512 && slabs >= 8 : groups >= 1152 && slabs >= 4;
 }
 
+// The gemm_planes instance that runs a conv2d of whole 16-byte channel vectors
+// as an implicit GEMM, or null (the generic template).
+//  * bf16 64x64x64, 128x64x64 and 128x128x64 (2x2 waves): always (us, generic
+//    -> this; 3x3 unless noted): 68x68x128 over 256 filters 27.9 -> 16.6,
+//    8x56x56x64 over 64 16.6 -> 10.6, 14x14x512 over 512 split 8 17.5 -> 13.4,
+//    34x34x256 over 512 on 128x64 split 4 25.7 -> 19.1, 17x17x1024 over 28272
+//    1x1 on 128x128 77.7 -> 58.4, 2x28x28x256 over 512 1x1 9.0 -> 5.8.
+//  * fp32 64x64 (2x2 waves): from 512 workgroups that walk 8 slabs of 32, as
+//    for matmuls: 272x272x32 over 64 44.0 -> 35.6, 34x34x256 over 512 split 4
+//    55.7 -> 41.3; but 14x14x256 over 256 split 16 15.9 -> 16.6, 4x56x56x64
+//    over 256 1x1 (2 slabs) 12.8 -> 13.9.
+const PlanesEntry* planes_conv_entry(const xtc_hip_conv2d_desc& d, const xtc_hip_tile& t, int split_k, int M, int K) {
+  if (generic_only() || !planes_offsets_fit(4, 1, d.F)) return nullptr;
+  if (d.dtype == XTC_HIP_BF16) return t.bk == 64 ? planes_entry(d.dtype, 1, 0, 1, t) : nullptr;
+  const int splits = effective_splits(K, split_k, t.bk);
+  const int64_t groups = (int64_t)((M + 63) / 64) * ((d.F + 63) / 64) * splits;
+  return groups >= 512 && split_depth(K, split_k, t.bk) >= 256 ? planes_entry(d.dtype, 1, 0, 1, t) : nullptr;
+}
+
+// Block of a conv2d whose channels or filters are not whole vectors on
+// gemm_planes: 64x64, or in fp32 128x64 over 8 waves from 192 workgroups of
+// it.  4x224x224x3, 7x7 stride 2 over 64 filters: 27.5 us on 64x64, 22.4 on
+// 128x64 (35.5 with the channels copied to whole vectors first); 56x56x10 3x3
+// over 64 (25 blocks): 9.6 and 10.5 us (13.8).
+xtc_hip_tile planes_conv_any_tile(int dtype, int M, int N, int splits) {
+  if (dtype == XTC_HIP_BF16) return {64, 64, 64, 2, 2};
+  if ((int64_t)((M + 127) / 128) * ((N + 63) / 64) * splits >= 192) return {128, 64, 32, 4, 2};
+  return {64, 64, 32, 2, 2};
+}
+
 bool splitwave_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_k, int lda, const void* A);
 
 // Whether gemm_planes reads B^T [N][ldb] in place behind tile t (the same
@@ -1115,6 +1145,15 @@ bool planes_bt_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int 
   if (t.bk != (vec == 4 ? 32 : 64) || !planes_entry(d.dtype, 0, 1, 1, t)) return false;
   if (lda % vec || ldb % vec || d.K % vec || d.N % vec || !aligned16(A) || !aligned16(B)) return false;
   return planes_offsets_fit(vec == 4 ? 4 : 2, lda, ldb) && !splitwave_gemm_applies(d, t, split_k, lda, A);
+}
+
+// Sums so short that one thread per output (gemm_naive_kernel) beats a tile
+// of gemm_planes, whose pipeline takes 4 to 6 us to fill: fp32 205x329 at K 17
+// 3.7 against 6.1 us, at K 33 5.5 against 7.0, at K 49 7.5 against 7.0; bf16 at
+// K 17 3.7 against 4.6, at K 25 4.6 each; fp32 1501x1499 at K 9 10.7 against
+// 10.9 us.
+bool short_sums(int dtype, int64_t M, int64_t N, int K) {
+  return K <= (dtype == XTC_HIP_F32 ? 32 : 16) && M * N * K <= (16 << 20);
 }
 
 // Matmuls that are not whole 16-byte vectors (strides, K, N or operand
@@ -1720,7 +1759,7 @@ int natural_path(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_
   const bool vec_ok = lda % vec == 0 && ldb % vec == 0 && d.K % vec == 0 && d.N % vec == 0 && aligned16(A) &&
                       aligned16(B);
   if (!vec_ok) {
-    const bool any = !generic_only() && d.dtype != XTC_HIP_F64 &&
+    const bool any = !generic_only() && d.dtype != XTC_HIP_F64 && !short_sums(d.dtype, d.M, d.N, d.K) &&
                      planes_offsets_fit(d.dtype == XTC_HIP_F32 ? 4 : 2, lda, ldb);
     *path = any ? MatmulPath::PlanesAny : MatmulPath::Naive;
     return 0;
@@ -1888,6 +1927,37 @@ int matmul_impl(const xtc_hip_matmul_desc& d, const void* A, const void* B, void
   a.relu_threshold = d.relu_threshold;
   if (path == MatmulPath::Planes || path == MatmulPath::PlanesAny) a.ldp = planes_ldp(d.N);
   return launch_gemm_common(a, e, split_k, path == MatmulPath::Generic ? d.stages : 0, d.group_m, d.xcd_remap, x);
+}
+
+// Implicit-GEMM arguments of conv2d descriptor d.
+GemmArgs conv_args(const xtc_hip_conv2d_desc& d, int OH, int OW, const void* input, const void* weight, float* out,
+                   const float* bias) {
+  GemmArgs a;
+  memset(&a, 0, sizeof(a));
+  a.A = input;
+  a.B = weight;
+  a.C = out;
+  a.bias = bias;
+  a.M = d.N * OH * OW;
+  a.N = d.F;
+  a.K = d.R * d.S * d.C;
+  a.lda = a.K;
+  a.ldb = d.F;
+  a.ldc = d.F;
+  a.relu = d.relu;
+  a.relu_threshold = d.relu_threshold;
+  a.cH = d.H;
+  a.cW = d.W;
+  a.cC = d.C;
+  a.cOH = OH;
+  a.cOW = OW;
+  a.cS = d.S;
+  a.cSH = d.stride_h;
+  a.cSW = d.stride_w;
+  a.cPH = d.pad_top;
+  a.cPW = d.pad_left;
+  a.pad_value = d.pad_value;
+  return a;
 }
 
 }  // namespace
@@ -2280,7 +2350,39 @@ int xtc_hip_conv2d(const xtc_hip_conv2d_desc* desc, const void* input, const voi
   const int K = d.R * d.S * d.C;
   const bool vec_ok = d.C % vec == 0 && d.F % vec == 0 && aligned16(input) && aligned16(weight);
   const bool padded = d.pad_top || d.pad_bottom || d.pad_left || d.pad_right;
-  if (!vec_ok && d.F % vec == 0 && (!padded || isfinite(f64 ? d.pad_value_f64 : (double)d.pad_value))) {
+  const bool can_stage = d.F % vec == 0 && (!padded || isfinite(f64 ? d.pad_value_f64 : (double)d.pad_value));
+  if (!vec_ok && !f64 && !generic_only() && planes_offsets_fit(4, 1, d.F)) {
+    // Channels or filters that are not whole 16-byte vectors, or operands not
+    // 16-byte aligned: gemm_planes gathers the window element by element.
+    // fp32 always; bf16, whose products are cheaper beside the gather, below
+    // 16 channels (56x56x50 3x3 over 64: 20.3 us gathered, 18.9 copied to
+    // whole vectors first) and where the copy cannot be made.
+    xtc_hip_conv2d_desc dc = d;  // the tile, split and refusals of the copied conv
+    if (can_stage) dc.C = (d.C + vec - 1) / vec * vec;
+    xtc_hip_tile t = d.tile;
+    int split_k = d.split_k;
+    if (t.bm == 0) {
+      int sk = 1;
+      default_conv_tile(dc, OH, OW, &t, &sk);
+      if (split_k <= 0) split_k = sk;
+    }
+    const GemmEntry* e = can_stage ? find_entry(d.dtype, 1, t) : nullptr;
+    const void* p = (const void*)(uintptr_t)256;
+    const bool gather = (!can_stage && !short_sums(d.dtype, M, d.F, K)) || (e && e->launch && (d.dtype == XTC_HIP_F32 || d.C < 16) &&
+                                       !direct_conv_applies(dc, t, split_k, OH, OW, p, p, p, nullptr));
+    if (gather) {
+      Scratch x{s};
+      xtc_hip_tile u = planes_conv_any_tile(d.dtype, M, d.F, 1);
+      split_k = splits_with_room(split_k < 1 ? 1 : split_k, M, d.F, K, u, x);
+      u = planes_conv_any_tile(d.dtype, M, d.F, effective_splits(K, split_k, u.bk));
+      const GemmEntry own{d.dtype, 1, u.bm, u.bn, u.bk, u.wgm, u.wgn, 0, 0, planes_entry(d.dtype, 1, 0, 0, u)->launch,
+                          nullptr};
+      GemmArgs a = conv_args(d, OH, OW, input, weight, out, bias);
+      a.ldp = planes_ldp(d.F);
+      return launch_gemm_common(a, &own, split_k, 0, d.group_m, d.xcd_remap, x);
+    }
+  }
+  if (!vec_ok && can_stage) {
     // Channels that are not whole 16-byte vectors (C = 3 image inputs): the
     // input and the weights are copied with zero channels up to Cp, a
     // multiple of the vector, and the MFMA conv runs on the copies.  A zero
@@ -2383,32 +2485,16 @@ int xtc_hip_conv2d(const xtc_hip_conv2d_desc* desc, const void* input, const voi
                 "split-K, C and F multiples of 64, 16-byte aligned operands and an input halo that fits its "
                 "LDS buffer",
                 t.bm, t.bn, t.bk, t.wgm, t.wgn);
-  GemmArgs a;
-  memset(&a, 0, sizeof(a));
-  a.A = input;
-  a.B = weight;
-  a.C = out;
-  a.bias = bias;
-  a.M = M;
-  a.N = d.F;
-  a.K = K;
-  a.lda = K;
-  a.ldb = d.F;
-  a.ldc = d.F;
-  a.relu = d.relu;
-  a.relu_threshold = d.relu_threshold;
-  a.cH = d.H;
-  a.cW = d.W;
-  a.cC = d.C;
-  a.cOH = OH;
-  a.cOW = OW;
-  a.cS = d.S;
-  a.cSH = d.stride_h;
-  a.cSW = d.stride_w;
-  a.cPH = d.pad_top;
-  a.cPW = d.pad_left;
-  a.pad_value = d.pad_value;
+  GemmArgs a = conv_args(d, OH, OW, input, weight, out, bias);
   Scratch x{s};
+  GemmEntry own;
+  if (const PlanesEntry* pe = planes_conv_entry(d, t, split_k, M, K)) {
+    own = *e;
+    own.launch = pe->launch;
+    own.launch_ring = nullptr;
+    a.ldp = planes_ldp(d.F);
+    e = &own;
+  }
   return launch_gemm_common(a, e, split_k, 0, d.group_m, d.xcd_remap, x);
 }
 

@@ -134,6 +134,7 @@ __device__ __forceinline__ void splitk_finish_tile(const float* partial, size_t 
     for (int i0 = 0; i0 < PER; i0 += U) {
       f32x4 v[U];
       unsigned off[U];
+      bool any = false;
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         // quads outside the tile or the matrix read the tile's first
@@ -142,7 +143,9 @@ __device__ __forceinline__ void splitk_finish_tile(const float* partial, size_t 
         const bool in = idx < QUADS && m0 + dm < M && n0 + dn < N;
         off[u] = in ? ((unsigned)dm * (unsigned)ldp + dn) * 4u : 0u;
         v[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+        any = any || in;
       }
+      if (!__any(any)) continue;
       // only the splits that exist, in order, at most 16 loads in flight
       auto add = [&](int s0, auto count) {
         constexpr int C = decltype(count)::value;
