@@ -90,11 +90,6 @@ __device__ __forceinline__ void store_partial(double* p, double v) {
                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ double load_partial(const double* p) {
-  return __longlong_as_double((long long)__hip_atomic_load(
-      reinterpret_cast<unsigned long long*>(const_cast<double*>(p)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-}
-
 }  // namespace f64k
 
 template <int BM, int BN, int WGM, int WGN, bool CONV>
@@ -290,16 +285,65 @@ gemm_f64_kernel(GemmArgs64 args) {
     }
   }
   if (to_partial && splitk_arrive(args.counters + tile_m * args.tiles_n + tile_n, (int)gridDim.z)) {
+    // pairs of columns (N is even), U of them and up to 4 splits in flight per
+    // lane: the loads go past the L2, one element at a time cost 17 of the
+    // 63 us of a 1024^3 product
     const size_t plane = (size_t)args.M * args.N;
     const int splits = (int)gridDim.z;
-    for (int idx = tid; idx < BM * BN; idx += NT) {
-      const int m = m0 + idx / BN, n = n0 + idx % BN;
-      if (m >= args.M || n >= args.N) continue;
-      double v = 0.0;
-      for (int s = 0; s < splits; ++s) v += f64k::load_partial(args.partial + s * plane + (size_t)m * args.N + n);
-      if (args.bias) v += args.bias[n];
-      if (args.relu && v < args.relu_threshold) v = args.relu_threshold;
-      args.C[(size_t)m * args.ldc + n] = v;
+    constexpr int PAIRS = BM * BN / 2, PER = (PAIRS + NT - 1) / NT, U = PER < 4 ? PER : 4;
+    const double* const tile = args.partial + (size_t)m0 * args.N + n0;
+    const bool vec_out = ((args.ldc | args.N) & 1) == 0 && ((uintptr_t)args.C & 15) == 0;
+    for (int i0 = 0; i0 < PER; i0 += U) {
+      f64x2 v[U];
+      unsigned off[U];
+      bool in[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int idx = tid + (i0 + u) * NT;
+        const int dm = idx / (BN / 2), dn = 2 * (idx % (BN / 2));
+        in[u] = idx < PAIRS && m0 + dm < args.M && n0 + dn < args.N;
+        off[u] = in[u] ? ((unsigned)dm * (unsigned)args.N + dn) * 8u : 0u;
+        v[u] = f64x2{0.0, 0.0};
+      }
+      auto add = [&](int s0, auto count) {
+        constexpr int C = decltype(count)::value;
+        f64x2 t[C][U];
+#pragma unroll
+        for (int j = 0; j < C; ++j)
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+            t[j][u] = __builtin_bit_cast(
+                f64x2, splitk_load4(reinterpret_cast<const float*>(tile + (size_t)(s0 + j) * plane), off[u]));
+#pragma unroll
+        for (int j = 0; j < C; ++j)
+#pragma unroll
+          for (int u = 0; u < U; ++u) v[u] += t[j][u];
+      };
+      int s0 = 0;
+      for (; s0 + 4 <= splits; s0 += 4) add(s0, std::integral_constant<int, 4>{});
+      if (s0 + 2 <= splits) {
+        add(s0, std::integral_constant<int, 2>{});
+        s0 += 2;
+      }
+      if (s0 < splits) add(s0, std::integral_constant<int, 1>{});
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (!in[u]) continue;
+        const int idx = tid + (i0 + u) * NT;
+        const int m = m0 + idx / (BN / 2), n = n0 + 2 * (idx % (BN / 2));
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          if (args.bias) v[u][e] += args.bias[n + e];
+          if (args.relu && v[u][e] < args.relu_threshold) v[u][e] = args.relu_threshold;
+        }
+        double* p = args.C + (size_t)m * args.ldc + n;
+        if (vec_out) {
+          *(f64x2*)p = v[u];
+        } else {
+          p[0] = v[u][0];
+          p[1] = v[u][1];
+        }
+      }
     }
     splitk_release(args.counters + tile_m * args.tiles_n + tile_n);
   }
