@@ -375,6 +375,99 @@ __global__ void unpad_rows_kernel(const uint4* __restrict__ x, uint4* __restrict
   }
 }
 
+// Constant pad (PAD) or crop of tensors of fewer than 2^31 elements, four
+// consecutive elements of an output row per thread: one 32-bit division per
+// outer dim (the per-element kernels divide in 64 bits for every element and
+// dim) and vector accesses at element alignment.  1000x1196 -> 1004x1200 fp32:
+// 6.5 -> 3.1 us, 1004x1104 -> 1000x1100 5.6 -> 2.9 us, launch included.
+struct RowCopyDims {
+  int outer;  // dims before the innermost
+  unsigned out_shape[7];
+  int in_shape[7], before[7];
+  unsigned out_len, in_len;  // innermost
+  int shift;                 // its `before`
+  unsigned groups;           // ceil(out_len / 4)
+  unsigned total;            // rows * groups
+};
+template <typename T, bool PAD>
+__global__ void __launch_bounds__(256) row_copy_kernel(const T* __restrict__ x, T* __restrict__ y, RowCopyDims d,
+                                                       T value) {
+  const unsigned i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= d.total) return;
+  const unsigned row = i / d.groups;
+  const int col = (int)(4u * (i - row * d.groups));
+  unsigned rem = row;
+  int src_row = 0, stride = 1;
+  bool inside = true;
+  for (int k = d.outer - 1; k >= 0; --k) {
+    const unsigned q = k > 0 ? rem / d.out_shape[k] : 0u;
+    const int o = (int)(rem - q * d.out_shape[k]);
+    rem = q;
+    const int s = PAD ? o - d.before[k] : o + d.before[k];
+    inside = inside && s >= 0 && s < d.in_shape[k];
+    src_row += s * stride;
+    stride *= d.in_shape[k];
+  }
+  const int c = PAD ? col - d.shift : col + d.shift;  // innermost source index
+  const T* src = x + (int64_t)src_row * d.in_len + c;
+  T v[4];
+  if (PAD && !inside) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = value;
+  } else if (c >= 0 && c + 4 <= (int)d.in_len) {
+    __builtin_memcpy(v, src, sizeof(v));
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[e] = value;
+      if (c + e >= 0 && c + e < (int)d.in_len) v[e] = src[e];
+    }
+  }
+  T* dst = y + (size_t)row * d.out_len + col;
+  if (col + 4 <= (int)d.out_len) {
+    __builtin_memcpy(dst, v, sizeof(v));
+  } else {
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+      if (col + e < (int)d.out_len) dst[e] = v[e];
+  }
+}
+
+// Launches row_copy_kernel for d on `s`; false where an extent needs 64 bits.
+template <typename T, bool PAD>
+bool launch_row_copy(const T* x, T* y, const PadDims& d, T value, hipStream_t s) {
+  uint64_t in = 1, rows = 1;
+  RowCopyDims r;
+  memset(&r, 0, sizeof(r));
+  r.outer = d.ndim - 1;
+  for (int k = 0; k < d.ndim; ++k) {
+    if (d.in_shape[k] > INT32_MAX || d.out_shape[k] > INT32_MAX || d.before[k] > INT32_MAX) return false;
+    in *= (uint64_t)d.in_shape[k];
+    if (in > INT32_MAX) return false;
+    if (k == d.ndim - 1) break;
+    rows *= (uint64_t)d.out_shape[k];
+    if (rows > INT32_MAX) return false;
+    r.out_shape[k] = (unsigned)d.out_shape[k];
+    r.in_shape[k] = (int)d.in_shape[k];
+    r.before[k] = (int)d.before[k];
+  }
+  const int last = d.ndim - 1;
+  r.out_len = (unsigned)d.out_shape[last];
+  r.in_len = (unsigned)d.in_shape[last];
+  r.shift = (int)d.before[last];
+  r.groups = (r.out_len + 3) / 4;
+  if (rows * r.out_len > INT32_MAX || rows * r.groups > INT32_MAX - 256) return false;
+  r.total = (unsigned)(rows * r.groups);
+  hipLaunchKernelGGL((row_copy_kernel<T, PAD>), dim3((r.total + 255) / 256), dim3(256), 0, s, x, y, r, value);
+  return true;
+}
+
+template <typename T>
+void launch_unpad(const T* x, T* y, const PadDims& d, uint64_t total, hipStream_t s) {
+  if (!launch_row_copy<T, false>(x, y, d, T(0), s))
+    hipLaunchKernelGGL(unpad_kernel<T>, dim3(grid_for(total, 256)), dim3(256), 0, s, x, y, d, total);
+}
+
 __device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
   unsigned u = __float_as_uint(f);
   if ((u & 0x7f800000u) == 0x7f800000u && (u & 0x007fffffu)) return (uint16_t)((u >> 16) | 0x40u);
@@ -977,6 +1070,8 @@ int launch_f64_common(GemmArgs64& a, const F64Tile* f, int split_k, int group_m,
   a.tiles_n = (a.N + f->tile.bn - 1) / f->tile.bn;
   a.group_m = group_m > 0 ? group_m : 8;
   a.xcd_remap = xcd_remap;
+  // the finishing workgroup addresses a tile's partials with 31-bit offsets
+  if ((int64_t)f->tile.bm * a.N > INT32_MAX / 8) split_k = 1;
   const int kps = split_depth(a.K, split_k, f->tile.bk);
   const int splits = (a.K + kps - 1) / kps;
   a.k_per_split = kps;
@@ -2533,8 +2628,9 @@ int xtc_hip_pad(const float* x, float* y, int ndim, const int64_t* shape, const 
     HIP_TRY(hipGetLastError());
     return 0;
   }
-  hipLaunchKernelGGL(pad_kernel, dim3(grid_for(total, 256)), dim3(256), 0, pick_stream(stream),
-                     x, y, d, total, value);
+  if (!launch_row_copy<float, true>(x, y, d, value, pick_stream(stream)))
+    hipLaunchKernelGGL(pad_kernel, dim3(grid_for(total, 256)), dim3(256), 0, pick_stream(stream),
+                       x, y, d, total, value);
   HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -2565,8 +2661,9 @@ int xtc_hip_pad_f64(const double* x, double* y, int ndim, const int64_t* shape, 
     total *= (uint64_t)d.out_shape[k];
   }
   if (total == 0) return 0;
-  hipLaunchKernelGGL(pad_f64_kernel, dim3(grid_for(total, 256)), dim3(256), 0, pick_stream(stream), x, y, d, total,
-                     value);
+  if (!launch_row_copy<double, true>(x, y, d, value, pick_stream(stream)))
+    hipLaunchKernelGGL(pad_f64_kernel, dim3(grid_for(total, 256)), dim3(256), 0, pick_stream(stream), x, y, d, total,
+                       value);
   HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -2599,14 +2696,11 @@ int xtc_hip_unpad(const void* x, void* y, int elem_bytes, int ndim, const int64_
     hipLaunchKernelGGL(unpad_rows_kernel, dim3(grid_for(total16, 256)), dim3(256), 0, pick_stream(stream),
                        (const uint4*)x, (uint4*)y, d, total16, row_bytes / 16);
   } else if (elem_bytes == 2) {
-    hipLaunchKernelGGL(unpad_kernel<uint16_t>, dim3(grid_for(total, 256)), dim3(256), 0, pick_stream(stream),
-                       (const uint16_t*)x, (uint16_t*)y, d, total);
+    launch_unpad((const uint16_t*)x, (uint16_t*)y, d, total, pick_stream(stream));
   } else if (elem_bytes == 4) {
-    hipLaunchKernelGGL(unpad_kernel<uint32_t>, dim3(grid_for(total, 256)), dim3(256), 0, pick_stream(stream),
-                       (const uint32_t*)x, (uint32_t*)y, d, total);
+    launch_unpad((const uint32_t*)x, (uint32_t*)y, d, total, pick_stream(stream));
   } else {
-    hipLaunchKernelGGL(unpad_kernel<uint64_t>, dim3(grid_for(total, 256)), dim3(256), 0, pick_stream(stream),
-                       (const uint64_t*)x, (uint64_t*)y, d, total);
+    launch_unpad((const uint64_t*)x, (uint64_t*)y, d, total, pick_stream(stream));
   }
   HIP_TRY(hipGetLastError());
   return 0;
