@@ -92,6 +92,19 @@ def test_transposed_b(dtype, tile, M, N, K, split):
         np.testing.assert_array_equal(out, ai.astype(np.float64) @ bi)
 
 
+# bf16 workgroups of 4 or 8 waves (512 and 520 of them), and more splits asked
+# for than the 128-row tiles run (66 tiles, 18.1 and 4 slabs)
+@pytest.mark.parametrize("tile,M,N,K,split", [((64, 64, 64, 2, 2), 1024, 2048, 136, 1), ((64, 64, 64, 2, 2), 505, 4136, 136, 1),
+                                              ((64, 64, 64, 2, 2), 505, 2088, 264, 2), ((128, 128, 64, 2, 2), 129, 4104, 1160, 8),
+                                              ((128, 128, 64, 2, 2), 256, 4224, 256, 4)])
+def test_bf16_workgroups_and_splits(tile, M, N, K, split):
+    print(f"[planes bf16] {tile} {M}x{N}x{K} split {split}", flush=True)
+    ai, bi = ref.np_init((M, K), "float32"), ref.np_init((K, N), "float32")[::-1].copy()
+    for bt in (True, False):
+        out = run_matmul_layout(ai, bi, "bfloat16", False, bt, tile=tile, split_k=split)
+        np.testing.assert_array_equal(out, ai.astype(np.float64) @ bi)
+
+
 def test_half_zero_and_wide_operands():
     # relu'd activations, and magnitudes spread over 2^-40 .. 2^40 in one sum
     rng = np.random.default_rng(5)

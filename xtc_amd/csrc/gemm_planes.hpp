@@ -44,7 +44,9 @@
 //     image row oh * sh + r - ph at element (ow * sw - pw) * C + kk: in
 //     bounds when both lie inside the image, no division by C.
 //   * B is the first MFMA operand, so a lane holds C[m][n .. n+3].
-//   * Split-K: partial planes and arrival counters of splitk.hpp.
+//   * Split-K: partial planes and arrival counters of splitk.hpp.  KG > 1: the
+//     workgroup holds KG groups of WGM x WGN waves, each with its own LDS
+//     buffers and its own run of the split's slabs; their sums meet in LDS.
 //
 // What bounds it.  At 4096^3 the board's power: 6 x 1.37e11 FLOP in 631 us is
 // 1.31 PFLOP/s of bf16 MFMAs, where a library bf16 product reaches 1.41
@@ -185,9 +187,9 @@ __device__ __forceinline__ void split2(const Unit<float>& u, int e, u32x4 (&w)[3
 
 }  // namespace planes
 
-template <typename T, int BM, int BN, int BK, int WGM, int WGN, bool CONV, bool BT, bool VEC, int RING>
+template <typename T, int BM, int BN, int BK, int WGM, int WGN, bool CONV, bool BT, bool VEC, int RING, int KG = 1>
 struct PlanesTile {
-  static constexpr int NT = WGM * WGN * 64;
+  static constexpr int NT = WGM * WGN * 64;  // threads of a k-group
   static constexpr bool F32 = sizeof(T) == 4;
   static constexpr int P = F32 ? 3 : 1;              // planes
   static constexpr int VE = F32 ? 4 : 8, VPU = 8 / VE;  // elements per vector, vectors per unit
@@ -204,23 +206,28 @@ struct PlanesTile {
   static_assert(A_EVEN || A_UNITS < NT, "A units");
   static_assert(B_EVEN || B_UNITS < NT, "B units");
   static_assert(NT % (BK / 8) == 0 && (BT || NT % (BN / 8) == 0), "a thread keeps its column");
-  static_assert(2 * STAGE <= 160 * 1024, "LDS");
+  static_assert(KG * 2 * STAGE <= 160 * 1024, "LDS");
+  static_assert(KG == 1 || !F32, "the fp32 kernel redoes a whole split's sums");
+  static_assert((KG - 1) * BM * BN * 4 <= KG * 2 * STAGE, "the groups' sums fit in the slabs' LDS");
 };
 
-template <typename T, int BM, int BN, int BK, int WGM, int WGN, bool CONV, bool BT, bool VEC, int RING>
-__global__ void __attribute__((amdgpu_flat_work_group_size(WGM * WGN * 64, WGM * WGN * 64)))
+template <typename T, int BM, int BN, int BK, int WGM, int WGN, bool CONV, bool BT, bool VEC, int RING, int KG = 1>
+__global__ void __attribute__((amdgpu_flat_work_group_size(KG * WGM * WGN * 64, KG * WGM * WGN * 64)))
 __attribute__((amdgpu_waves_per_eu(2)))
 gemm_planes(GemmArgs args) {
   using namespace planes;
-  using X = PlanesTile<T, BM, BN, BK, WGM, WGN, CONV, BT, VEC, RING>;
+  using X = PlanesTile<T, BM, BN, BK, WGM, WGN, CONV, BT, VEC, RING, KG>;
   constexpr int NT = X::NT, TM = X::TM, TN = X::TN;
   constexpr bool F32 = X::F32;
 
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[2 * X::STAGE];
+  __shared__ __attribute__((aligned(1024))) unsigned char shared[KG * 2 * X::STAGE];
 
-  const unsigned tid = threadIdx.x;
+  const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kg = KG > 1 ? wave_id / (WGM * WGN) : 0;  // k-group
+  unsigned char* const smem = shared + kg * 2 * X::STAGE;
+  const unsigned tid = threadIdx.x - kg * NT;  // in the k-group
   const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = wave_id - kg * (WGM * WGN);
   const int wm = wave / WGN, wn = wave % WGN;
   const int l16 = lane & 15, g = lane >> 4;
 
@@ -228,8 +235,11 @@ gemm_planes(GemmArgs args) {
   tile_coords(args, tile_m, tile_n);
   const int m0 = tile_m * BM, n0 = tile_n * BN;
   const int split = blockIdx.z;
-  const int k_begin = split * args.k_per_split;
-  const int k_end = min(args.K, k_begin + args.k_per_split);
+  // the split's slabs, a run of `steps` of them for each k-group
+  const int split_begin = split * args.k_per_split, split_end = min(args.K, split_begin + args.k_per_split);
+  const int steps = ((split_end - split_begin + BK - 1) / BK + KG - 1) / KG;
+  const int k_begin = min(split_begin + kg * steps * BK, split_end);
+  const int k_end = KG > 1 ? min(split_end, k_begin + steps * BK) : split_end;
   const int nk = (k_end - k_begin + BK - 1) / BK;
 
   const T* const A = reinterpret_cast<const T*>(args.A);
@@ -270,7 +280,7 @@ gemm_planes(GemmArgs args) {
   // K stagger: tile (tm, tn) starts its K walk at slab (tm + 2 tn) mod 16, so
   // that tiles sharing a panel do not ask for the same lines at once (a K of
   // whole slabs only, so that a partial slab stays the last)
-  const int kofs = (k_end - k_begin) % BK == 0 ? ((tile_m + 2 * tile_n) & 15) % nk : 0;
+  const int kofs = (KG == 1 || nk > 0) && (k_end - k_begin) % BK == 0 ? ((tile_m + 2 * tile_n) & 15) % nk : 0;
   auto slab_k = [&](int t) {  // k of step t's slab, relative to k_begin
     const int r = t + kofs;
     return (r >= nk ? r - nk : r) * BK;
@@ -473,9 +483,11 @@ gemm_planes(GemmArgs args) {
 #pragma unroll
   for (int r = 0; r < RING; ++r)
     if (r < nk) load_slab(r, r);
-  mask_slab(0, 0);
-  store_slab(smem, 0);
-  if (RING < nk) load_slab(RING, 0);
+  if (KG == 1 || nk > 0) {
+    mask_slab(0, 0);
+    store_slab(smem, 0);
+    if (RING < nk) load_slab(RING, 0);
+  }
   __syncthreads();
 
   if constexpr (F32) {
@@ -613,6 +625,9 @@ gemm_planes(GemmArgs args) {
     }
   }
 
+  // a k-group with fewer slabs passes every step's barrier with the others
+  for (int t = nk; KG > 1 && t < steps; ++t) __syncthreads();
+
   const int mrow = m0 + wm * (16 * TM) + l16;
   const int ncol = n0 + wn * (16 * TN) + 4 * g;
 
@@ -686,6 +701,26 @@ gemm_planes(GemmArgs args) {
     }
   }
 
+  // ---- the k-groups' sums meet in LDS, added in k order by the first group
+  if constexpr (KG > 1) {
+    f32x4* const sums = reinterpret_cast<f32x4*>(shared);
+    if (kg > 0) {  // the last step's barrier is behind every slab's last read
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) sums[(((kg - 1) * TM + i) * TN + j) * NT + tid] = acc[i][j];
+    }
+    __syncthreads();
+    if (kg == 0) {
+#pragma unroll
+      for (int q = 0; q < KG - 1; ++q)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] += sums[((q * TM + i) * TN + j) * NT + tid];
+    }
+  }
+
   // ---- epilogue: lane holds C[m][n .. n+3]
   const bool to_partial = args.partial != nullptr;
   float* const out = to_partial ? args.partial + (size_t)split * args.M * args.ldp : args.C;
@@ -695,7 +730,7 @@ gemm_planes(GemmArgs args) {
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
     const int n = ncol + 16 * j;
-    if (n >= args.N) continue;
+    if (n >= args.N || kg > 0) continue;
     f32x4 bv = {0.f, 0.f, 0.f, 0.f};
     if (!to_partial && args.bias) {
 #pragma unroll
@@ -725,7 +760,7 @@ gemm_planes(GemmArgs args) {
     }
   }
   if (to_partial && splitk_arrive(args.counters + tile_m * args.tiles_n + tile_n, (int)gridDim.z)) {
-    splitk_finish_tile<BM, BN, NT>(args.partial, (size_t)args.M * args.ldp, args.ldp, args.C, args.bias, args.M, args.N, args.ldc, (int)gridDim.z, args.relu,
+    splitk_finish_tile<BM, BN, KG * NT>(args.partial, (size_t)args.M * args.ldp, args.ldp, args.C, args.bias, args.M, args.N, args.ldc, (int)gridDim.z, args.relu,
                                    args.relu_threshold, m0, n0);
     splitk_release(args.counters + tile_m * args.tiles_n + tile_n);
   }

@@ -11,8 +11,11 @@ const PlanesEntry* planes_conv(int* count) {
       planes_instance<float, 128, 64, 32, 4, 2, true, false, false, 1>(),
       planes_instance<__bf16, 64, 64, 64, 2, 2, true, false, true, 2>(),
       planes_instance<__bf16, 64, 64, 64, 2, 2, true, false, false, 1>(),
-      planes_instance<__bf16, 128, 64, 64, 2, 2, true, false, true, 1>(),
-      planes_instance<__bf16, 128, 128, 64, 2, 2, true, false, true, 1>(),
+      planes_instance<__bf16, 64, 64, 64, 2, 4, true, false, true, 2>(2, 2),
+      planes_instance<__bf16, 128, 64, 64, 4, 2, true, false, true, 2>(2, 2),
+      planes_instance<__bf16, 128, 64, 64, 4, 2, true, false, true, 1, 2>(2, 2),
+      planes_instance<__bf16, 128, 128, 64, 2, 4, true, false, true, 2>(2, 2),
+      planes_instance<__bf16, 128, 128, 64, 2, 4, true, false, true, 1, 2>(2, 2),
   };
   *count = (int)(sizeof(table) / sizeof(table[0]));
   return table;

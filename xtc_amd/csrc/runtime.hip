@@ -1023,6 +1023,11 @@ int effective_splits(int K, int split_k, int bk) {
   return (K + kps - 1) / kps;
 }
 
+// Workgroups of a launch of tile t.
+int64_t launch_groups(int M, int N, int K, int split_k, const xtc_hip_tile& t) {
+  return (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * effective_splits(K, split_k, t.bk);
+}
+
 // Ring instances of the generic template (three register sets of loads in
 // flight, pipeline depth 4) for entry e at `splits` splits: 0 none, 1 one
 // exists and depth 2 is the default, 2 one exists and is the default.  Split
@@ -1142,14 +1147,55 @@ bool skinny_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, in
   return true;
 }
 
-const PlanesEntry* planes_entry(int dtype, int conv, int bt, int vec, const xtc_hip_tile& t) {
+// The gemm_planes instance of tile t (its slab depth aside), of the listed
+// waves and k-groups; any if 0.
+const PlanesEntry* planes_entry(int dtype, int conv, int bt, int vec, const xtc_hip_tile& t, int waves = 0, int kg = 0) {
   int n = 0;
   const PlanesEntry* e = conv ? planes_conv(&n) : dtype == XTC_HIP_F32 ? planes_f32(&n) : planes_bf16(&n);
   for (int i = 0; i < n; ++i)
     if (e[i].dtype == dtype && e[i].conv == conv && e[i].bt == bt && e[i].vec == vec && e[i].bm == t.bm && e[i].bn == t.bn &&
-        e[i].wgm == t.wgm && e[i].wgn == t.wgn)
+        e[i].wgm == t.wgm && e[i].wgn == t.wgn && (!waves || e[i].waves == waves) && (!kg || e[i].kg == kg))
       return &e[i];
   return nullptr;
+}
+
+// The instance that runs tile t over whole 16-byte vectors, and how many
+// splits of K it runs.  fp32 has one instance a tile.  bf16:
+//  * 128-row tiles whose workgroups fit the 256 CUs once: two k-groups of 8
+//    waves each share a workgroup and walk half of its K.  A CU holds as many
+//    waves as from two workgroups, and half the splits leave as many partial
+//    chains with half the partial sums in memory; no chain is longer than
+//    asked for.  (us; two k-groups at half the splits, or as many as fit,
+//    against 8 waves at all of them) 256x8192x4608 split 4 39.9 -> 34.5,
+//    256x4608x8192 split 4 51.9 -> 38.2 on 3, 128x4096x8192 split 16 33.2 ->
+//    26.9, 1280x2048x4096 split 2 47.9 -> 43.5, 1280x2048x8192 unsplit 93.8 ->
+//    79.8.  Below 8 slabs a workgroup the second group's sums cost what it
+//    saves (1024x1024x1024 split 4: 14.9 against 14.7).
+//  * 128-row tiles otherwise: 8 waves.  Four of 64x64 each leave a CU's
+//    matrix cores idle behind their LDS reads (2000x2304x2600 54.8 -> 51.1,
+//    17x17x1024 1x1 over 28272 57.9 -> 46.4).
+//  * 64x64 tiles: 8 waves hide more of the load latency where a CU has one or
+//    two workgroups, 4 read less from LDS where it has several (4 waves -> 8):
+//    7x7x512 3x3 over 512 split 8 (64 workgroups) 12.2 -> 10.7, 2x28x28x256 1x1
+//    over 512 (200) 5.9 -> 5.3, 1000x1104x1200 (288) 14.5 -> 13.8,
+//    512x1024x1024 split 4 (512) 10.0 -> 9.1; but 68x68x128 3x3
+//    over 256 (292) 16.6 -> 17.0, 8x56x56x64 over 64 (392) 10.7 -> 10.9,
+//    17x17x512 over 1024 split 8 (640) 16.5 -> 16.8, 128x4096x8192 split 8
+//    (1024) 27.2 -> 28.3.
+struct PlanesPick {
+  const PlanesEntry* e;
+  int split_k;
+};
+PlanesPick planes_pick(int dtype, int conv, int bt, const xtc_hip_tile& t, int M, int N, int K, int split_k) {
+  if (dtype == XTC_HIP_F32) return {planes_entry(dtype, conv, bt, 1, t), split_k};
+  const int splits = effective_splits(K, split_k, t.bk);
+  const int64_t tiles = launch_groups(M, N, K, 1, t);
+  if (t.bm == 128) {
+    const int fit = (int)std::min<int64_t>(splits, 256 / tiles);
+    const bool two = fit > 0 && 2 * fit >= splits && split_depth(K, fit, t.bk) / t.bk >= 8;
+    return {planes_entry(dtype, conv, bt, 1, t, 8, two ? 2 : 1), two ? fit : split_k};
+  }
+  return {planes_entry(dtype, conv, bt, 1, t, tiles * splits <= (conv ? 256 : 512) ? 8 : 4, 1), split_k};
 }
 
 bool generic_only() {
@@ -1182,9 +1228,9 @@ bool planes_offsets_fit(int esz, int lda, int ldb) {
 //    18.9 -> 22.0, 300x500x2000 split 8 (320 of 7) 19.2 -> 20.8.
 //  * bf16 (one plane) 128x128x64 and 64x64x64 (2x2 waves): always.  Transposing
 //    LDS reads instead of byte permutes on the way in, loads a step ahead
-//    without bounds branches (us, generic -> this): 2000x2304x2600 68 -> 54,
-//    256x8192x4608 split 4 49 -> 43, 1000x1104x1200 24.2 -> 14.3, 512x1024x1024
-//    split 4 12.4 -> 10.6.
+//    without bounds branches (us, generic -> this): 2000x2304x2600 68 -> 51,
+//    256x8192x4608 split 4 49 -> 35, 1000x1104x1200 24.2 -> 13.8, 512x1024x1024
+//    split 4 12.4 -> 9.1.
 bool planes_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_k, int lda, int ldb) {
   if (generic_only() || d.dtype == XTC_HIP_F64) return false;
   const bool f32 = d.dtype == XTC_HIP_F32;
@@ -1192,7 +1238,7 @@ bool planes_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, in
   if (!planes_offsets_fit(f32 ? 4 : 2, lda, ldb)) return false;
   if (!f32 || t.bm > 64) return true;
   const int splits = effective_splits(d.K, split_k, t.bk);
-  const int64_t groups = (int64_t)((d.M + 63) / 64) * ((d.N + 63) / 64) * splits;
+  const int64_t groups = launch_groups(d.M, d.N, d.K, split_k, t);
   const int slabs = split_depth(d.K, split_k, t.bk) / 32;
   return splits == 1 ? groups >= 512 && slabs >= 8 : groups >= 1152 && slabs >= 4;
 }
@@ -1202,18 +1248,18 @@ bool planes_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, in
 //  * bf16 64x64x64, 128x64x64 and 128x128x64 (2x2 waves): always (us, generic
 //    -> this; 3x3 unless noted): 68x68x128 over 256 filters 27.9 -> 16.6,
 //    8x56x56x64 over 64 16.6 -> 10.6, 14x14x512 over 512 split 8 17.5 -> 13.4,
-//    34x34x256 over 512 on 128x64 split 4 25.7 -> 19.1, 17x17x1024 over 28272
-//    1x1 on 128x128 77.7 -> 58.4, 2x28x28x256 over 512 1x1 9.0 -> 5.8.
+//    34x34x256 over 512 on 128x64 split 4 25.7 -> 15.6, 17x17x1024 over 28272
+//    1x1 on 128x128 77.7 -> 46.4, 2x28x28x256 over 512 1x1 9.0 -> 5.3.
 //  * fp32 64x64 (2x2 waves): from 512 workgroups that walk 8 slabs of 32, as
 //    for matmuls: 272x272x32 over 64 44.0 -> 35.6, 34x34x256 over 512 split 4
 //    55.7 -> 41.3; but 14x14x256 over 256 split 16 15.9 -> 16.6, 4x56x56x64
 //    over 256 1x1 (2 slabs) 12.8 -> 13.9.
-const PlanesEntry* planes_conv_entry(const xtc_hip_conv2d_desc& d, const xtc_hip_tile& t, int split_k, int M, int K) {
-  if (generic_only() || !planes_offsets_fit(4, 1, d.F)) return nullptr;
-  if (d.dtype == XTC_HIP_BF16) return t.bk == 64 ? planes_entry(d.dtype, 1, 0, 1, t) : nullptr;
-  const int splits = effective_splits(K, split_k, t.bk);
-  const int64_t groups = (int64_t)((M + 63) / 64) * ((d.F + 63) / 64) * splits;
-  return groups >= 512 && split_depth(K, split_k, t.bk) >= 256 ? planes_entry(d.dtype, 1, 0, 1, t) : nullptr;
+PlanesPick planes_conv_pick(const xtc_hip_conv2d_desc& d, const xtc_hip_tile& t, int split_k, int M, int K) {
+  const bool applies = d.dtype == XTC_HIP_BF16
+                           ? t.bk == 64
+                           : launch_groups(M, d.F, K, split_k, t) >= 512 && split_depth(K, split_k, t.bk) >= 256;
+  if (!applies || generic_only() || !planes_offsets_fit(4, 1, d.F) || !planes_entry(d.dtype, 1, 0, 1, t)) return {nullptr, split_k};
+  return planes_pick(d.dtype, 1, 0, t, M, d.F, K, split_k);
 }
 
 // Block of a conv2d whose channels or filters are not whole vectors on
@@ -1999,10 +2045,15 @@ int matmul_impl(const xtc_hip_matmul_desc& d, const void* A, const void* B, void
     split_k = splits_with_room(split_k, d.M, d.N, d.K, u, x);
   } else if (path == MatmulPath::F32Lds || path == MatmulPath::Planes) {
     // same tiles, split-K set-up and grid as the generic instance; only the
-    // kernel differs
+    // kernel and, in bf16, the number of splits differ
     own = *e;
-    own.launch = path == MatmulPath::F32Lds ? f32_lds_variant(t, d.stages)->launch
-                                            : planes_entry(d.dtype, 0, bt, 1, t)->launch;
+    if (path == MatmulPath::F32Lds) {
+      own.launch = f32_lds_variant(t, d.stages)->launch;
+    } else {
+      const PlanesPick p = planes_pick(d.dtype, 0, bt, t, d.M, d.N, d.K, split_k);
+      own.launch = p.e->launch;
+      split_k = p.split_k;
+    }
     own.launch_ring = nullptr;
     e = &own;
   }
@@ -2583,10 +2634,11 @@ int xtc_hip_conv2d(const xtc_hip_conv2d_desc* desc, const void* input, const voi
   GemmArgs a = conv_args(d, OH, OW, input, weight, out, bias);
   Scratch x{s};
   GemmEntry own;
-  if (const PlanesEntry* pe = planes_conv_entry(d, t, split_k, M, K)) {
+  if (const PlanesPick p = planes_conv_pick(d, t, split_k, M, K); p.e) {
     own = *e;
-    own.launch = pe->launch;
+    own.launch = p.e->launch;
     own.launch_ring = nullptr;
+    split_k = p.split_k;
     a.ldp = planes_ldp(d.F);
     e = &own;
   }
