@@ -1379,9 +1379,15 @@ bool splitwave_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t,
   // same order (the results are bit-identical when a split is whole slabs).
   // 512^3 at split 4 11.0 -> 5.5 us, 256^3 at split 2 9.5 -> 4.9, 32x4096x1024
   // at split 8 13.2 -> 10.7; with 512 blocks it loses (512x1024x1024 at split 8
-  // 18.9 -> 20.7 us).
+  // 18.9 -> 20.7 us).  Up to 4 splits it wins at every depth (512x512x2048 at 4
+  // 21.6 -> 12.6); at 8, few blocks leave the walk to one CU's load latency
+  // (template -> this: 128x128x1280 10.6 -> 12.1, 384x128x4864 24.3 -> 39.6,
+  // 32x2048x1280 11.5 -> 12.2, 32x4096x4864 33.2 -> 39.3; but 32x4096x2048
+  // 19.9 -> 18.2, 32x8192x1536 23.0 -> 15.2).
+  const int64_t blocks = (int64_t)(d.M / 32) * (d.N / 32);
   return t.bm == 64 && t.bn == 64 && t.bk == 32 && t.wgm == 2 && t.wgn == 2 && d.stages == 0 &&
-         d.K % (32 * split_k) == 0 && (int64_t)(d.M / 32) * (d.N / 32) <= 256;
+         d.K % (32 * split_k) == 0 && blocks <= 256 &&
+         (split_k <= 4 || (blocks >= 128 && d.K <= 256 * split_k));
 }
 
 // Pipeline depths (register ring chunks) of the split-wave kernel, default
