@@ -50,6 +50,21 @@ def test_edges(tile, M, N, K, split):
     check(run_matmul(a, b, tile=tile, split_k=split), a, b)
 
 
+# tiles of four waves whose product runs on an 8-wave tile instead: the generic
+# 128x128 one at its edges, the 64x64 one where the estimate says so (K split
+# less often than asked, cut by M and N); the bound covers every split count
+@pytest.mark.parametrize("tile,M,N,K,split", [((128, 128, 32, 2, 2), 1, 4, 4, 1), ((128, 128, 32, 2, 2), 129, 260, 100, 1),
+                                              ((128, 128, 32, 2, 2), 300, 132, 1156, 3),
+                                              ((64, 64, 32, 2, 2), 1000, 1104, 1200, 8),
+                                              ((64, 64, 32, 2, 2), 257, 2308, 2052, 8),
+                                              ((64, 64, 32, 2, 2), 1281, 3076, 516, 1)])
+def test_four_wave_tiles_on_eight_waves(tile, M, N, K, split):
+    print(f"[planes wide] {tile} {M}x{N}x{K} split {split}", flush=True)
+    a, b = rng_uniform(M + K, (M, K)), rng_uniform(N + K, (K, N))
+    check(run_matmul(a, b, tile=tile, split_k=split), a, b)
+    check(run_matmul_layout(a, b, "float32", False, True, tile=tile, split_k=split), a, b)
+
+
 # no whole vectors anywhere: fp32 and bf16 rows at element alignment, units cut
 # by K and N, tiles cut by M and N, split-K partial rows of whole vectors
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])

@@ -1273,6 +1273,58 @@ xtc_hip_tile planes_conv_any_tile(int dtype, int M, int N, int splits) {
   return {64, 64, 32, 2, 2};
 }
 
+// The gemm_planes tile and split that run an fp32 matmul of whole vectors named
+// with the 64x64x32 or 128x128x32 tile of 2x2 waves at the default depth, when
+// one of the 8-wave tiles is estimated to take less time (us; a workgroup of
+// those has a CU to itself):
+//   8 waves  rounds of 256 workgroups * (9 + slabs * 1.4 (128x128) or 2.3
+//            (256 wide), a third more with column tiles cut by N)
+//            + what the last workgroup of a tile sums, 0.93 a 64 KB partial
+//   64x64    rounds of 256 * slabs * 0.55 (0.85 on the generic template) + 6
+//            (16 where gemm_planes splits K)
+// which follow the measured times of 20 shapes x 40 launches to 15 %.  The
+// generic 128x128 tile is never better.  K is split at most as often as asked
+// for, so the scratch holds the partials (us, before -> now): 3000^3 727 ->
+// 446, 2048x2048x1024 89.7 -> 54.2, 256x4608x8192 153 -> 117, 768x768x4096
+// 58.4 -> 44.8, 1280x4096x2048 159 -> 145, 1000x1104x1200 44.3 -> 34.5,
+// 2000x2304x2600 187 -> 182.
+struct WidePick {
+  const PlanesEntry* e;
+  int split_k;
+};
+WidePick planes_wide_pick(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_k, int lda, int ldb, bool bt,
+                          bool on_planes) {
+  const bool small = t.bm == 64 && t.bn == 64;
+  if (generic_only() || d.dtype != XTC_HIP_F32 || d.stages != 0 || t.bk != 32 || t.wgm != 2 || t.wgn != 2 ||
+      !(small || (t.bm == 128 && t.bn == 128)) || !planes_offsets_fit(4, lda, ldb))
+    return {nullptr, split_k};
+  const int asked = effective_splits(d.K, split_k, t.bk);
+  WidePick best{nullptr, split_k};
+  double least = 1e30;
+  if (small) {
+    const int64_t rounds = (launch_groups(d.M, d.N, d.K, split_k, t) + 255) / 256;
+    const int slabs = split_depth(d.K, split_k, 32) / 32;
+    // 12 % off: near ties stay (3072x1408x2432 166 -> 179, 1449x3416x140 24.2
+    // -> 25.1 at 8 %)
+    least = 0.88 * (rounds * slabs * (on_planes ? 0.55 : 0.85) + (on_planes && asked > 1 ? 16 : 6));
+  }
+  const xtc_hip_tile wide[] = {{256, 128, 32, 4, 2}, {128, 256, 32, 2, 4}, {128, 128, 32, 2, 4}};
+  for (const xtc_hip_tile& w : wide) {
+    const double slab = (w.bm == w.bn ? 1.4 : 2.3) * (d.N % w.bn && !bt ? 1.3 : 1.0);
+    for (int want = 1; want <= std::min(asked, 16); ++want) {
+      const int s = effective_splits(d.K, want, 32), slabs = split_depth(d.K, want, 32) / 32;
+      if (s != want || (s > 1 && slabs < 4)) continue;
+      const int64_t rounds = (launch_groups(d.M, d.N, d.K, s, w) + 255) / 256;
+      const double us = rounds * (9 + slabs * slab) + (s > 1 ? 0.93 * s * (w.bm * w.bn / 16384) : 0.0);
+      if (us < least) {
+        least = us;
+        best = {planes_entry(d.dtype, 0, bt, 1, w), s};
+      }
+    }
+  }
+  return best;
+}
+
 bool splitwave_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_k, int lda, const void* A);
 
 // Whether gemm_planes reads B^T [N][ldb] in place behind tile t (the same
@@ -2063,6 +2115,15 @@ int matmul_impl(const xtc_hip_matmul_desc& d, const void* A, const void* B, void
     own.launch_ring = nullptr;
     e = &own;
   }
+  bool planes = path == MatmulPath::Planes || path == MatmulPath::PlanesAny;
+  if (path == MatmulPath::Planes || path == MatmulPath::Generic) {
+    if (const WidePick w = planes_wide_pick(d, t, split_k, lda, ldb, bt, planes); w.e) {
+      own = GemmEntry{d.dtype, 0, w.e->bm, w.e->bn, 32, w.e->wgm, w.e->wgn, 0, 0, w.e->launch, nullptr};
+      e = &own;
+      split_k = w.split_k;
+      planes = true;
+    }
+  }
   GemmArgs a;
   memset(&a, 0, sizeof(a));
   a.A = A;
@@ -2077,7 +2138,7 @@ int matmul_impl(const xtc_hip_matmul_desc& d, const void* A, const void* B, void
   a.ldc = ldc;
   a.relu = d.relu;
   a.relu_threshold = d.relu_threshold;
-  if (path == MatmulPath::Planes || path == MatmulPath::PlanesAny) a.ldp = planes_ldp(d.N);
+  if (planes) a.ldp = planes_ldp(d.N);
   return launch_gemm_common(a, e, split_k, path == MatmulPath::Generic ? d.stages : 0, d.group_m, d.xcd_remap, x);
 }
 
