@@ -177,8 +177,9 @@ int xtc_hip_matmul_noalloc(const xtc_hip_matmul_desc *desc, const void *A,
  * (pad_top, pad_bottom, pad_left, pad_right) with pad_value: the XTCOperPad2D
  * producer (operators.py:350-591, MlirOps.py:719-735) fused into the loader.
  * Output and bias are fp32 for fp32 / bf16 operands and fp64 for fp64 ones.
- * Channel counts that are not whole 16-byte vectors are staged with zero
- * channels (or run on a scalar kernel when the filters are not either). */
+ * Channels or filters that are not whole 16-byte vectors: fp32, and bf16 below
+ * 16 channels or with such filters, gather the window in place; other bf16 and
+ * fp64 calls stage zero channels; short sums run a scalar kernel. */
 typedef struct {
   int dtype;
   int N, H, W, C;        /* unpadded input */
