@@ -29,6 +29,7 @@
 #include "mfma_peak.hpp"
 #include "planes_table.hpp"
 #include "registry.hpp"
+#include "row_copy.hpp"
 #include "xtc_hip.h"
 
 using namespace xtc_hip;
@@ -376,60 +377,38 @@ __global__ void unpad_rows_kernel(const uint4* __restrict__ x, uint4* __restrict
 }
 
 // Constant pad (PAD) or crop of tensors of fewer than 2^31 elements, four
-// consecutive elements of an output row per thread: one 32-bit division per
-// outer dim (the per-element kernels divide in 64 bits for every element and
-// dim) and vector accesses at element alignment.  1000x1196 -> 1004x1200 fp32:
-// 6.5 -> 3.1 us, 1004x1104 -> 1000x1100 5.6 -> 2.9 us, launch included.
-struct RowCopyDims {
-  int outer;  // dims before the innermost
-  unsigned out_shape[7];
-  int in_shape[7], before[7];
-  unsigned out_len, in_len;  // innermost
-  int shift;                 // its `before`
-  unsigned groups;           // ceil(out_len / 4)
-  unsigned total;            // rows * groups
-};
+// consecutive elements of an output row per thread (row_copy.hpp): one 32-bit
+// division per outer dim (the per-element kernels divide in 64 bits for every
+// element and dim) and vector accesses at element alignment.  1000x1196 ->
+// 1004x1200 fp32: 6.5 -> 3.1 us, 1004x1104 -> 1000x1100 5.6 -> 2.9 us, launch
+// included.
 template <typename T, bool PAD>
 __global__ void __launch_bounds__(256) row_copy_kernel(const T* __restrict__ x, T* __restrict__ y, RowCopyDims d,
                                                        T value) {
   const unsigned i = blockIdx.x * 256u + threadIdx.x;
   if (i >= d.total) return;
-  const unsigned row = i / d.groups;
-  const int col = (int)(4u * (i - row * d.groups));
-  unsigned rem = row;
-  int src_row = 0, stride = 1;
-  bool inside = true;
-  for (int k = d.outer - 1; k >= 0; --k) {
-    const unsigned q = k > 0 ? rem / d.out_shape[k] : 0u;
-    const int o = (int)(rem - q * d.out_shape[k]);
-    rem = q;
-    const int s = PAD ? o - d.before[k] : o + d.before[k];
-    inside = inside && s >= 0 && s < d.in_shape[k];
-    src_row += s * stride;
-    stride *= d.in_shape[k];
-  }
-  const int c = PAD ? col - d.shift : col + d.shift;  // innermost source index
-  const T* src = x + (int64_t)src_row * d.in_len + c;
+  const RowGroup g = row_group<PAD>(d, i);
+  const T* src = x + (int64_t)g.src_row * d.in_len + (int)g.c;
   T v[4];
-  if (PAD && !inside) {
+  if (PAD && !g.inside) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = value;
-  } else if (c >= 0 && c + 4 <= (int)d.in_len) {
+  } else if (row_has4(g.c, d.in_len)) {
     __builtin_memcpy(v, src, sizeof(v));
   } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       v[e] = value;
-      if (c + e >= 0 && c + e < (int)d.in_len) v[e] = src[e];
+      if (row_has(g.c, e, d.in_len)) v[e] = src[e];
     }
   }
-  T* dst = y + (size_t)row * d.out_len + col;
-  if (col + 4 <= (int)d.out_len) {
+  T* dst = y + (size_t)g.row * d.out_len + g.col;
+  if (row_has4(g.col, d.out_len)) {
     __builtin_memcpy(dst, v, sizeof(v));
   } else {
 #pragma unroll
     for (int e = 0; e < 3; ++e)
-      if (col + e < (int)d.out_len) dst[e] = v[e];
+      if (row_has(g.col, e, d.out_len)) dst[e] = v[e];
   }
 }
 
@@ -448,14 +427,14 @@ bool launch_row_copy(const T* x, T* y, const PadDims& d, T value, hipStream_t s)
     rows *= (uint64_t)d.out_shape[k];
     if (rows > INT32_MAX) return false;
     r.out_shape[k] = (unsigned)d.out_shape[k];
-    r.in_shape[k] = (int)d.in_shape[k];
-    r.before[k] = (int)d.before[k];
+    r.in_shape[k] = (unsigned)d.in_shape[k];
+    r.before[k] = (unsigned)d.before[k];
   }
   const int last = d.ndim - 1;
   r.out_len = (unsigned)d.out_shape[last];
   r.in_len = (unsigned)d.in_shape[last];
-  r.shift = (int)d.before[last];
-  r.groups = (r.out_len + 3) / 4;
+  r.shift = (unsigned)d.before[last];
+  r.groups = (r.out_len + 3) / 4;  // out_len < 2^31
   if (rows * r.out_len > INT32_MAX || rows * r.groups > INT32_MAX - 256) return false;
   r.total = (unsigned)(rows * r.groups);
   hipLaunchKernelGGL((row_copy_kernel<T, PAD>), dim3((r.total + 255) / 256), dim3(256), 0, s, x, y, r, value);
