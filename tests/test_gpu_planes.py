@@ -12,12 +12,15 @@ of a product each; 2^-148 for sums in the denormal range.
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
 from oracle import reference as ref
 from test_gpu_kernels import _run_depth, needs_specialised, rng_uniform, run_conv, run_matmul, run_matmul_layout
-from xtc_amd.runtimes.hip.buffer import ensure_device
+from xtc_amd.runtimes.hip import capi
+from xtc_amd.runtimes.hip.buffer import DeviceBuffer, ensure_device
 
 pytestmark = [pytest.mark.gpu, needs_specialised]
 
@@ -209,3 +212,52 @@ def test_conv_infinite_pad():
     want = np.full((1, 6, 6, 8), np.inf, np.float32)
     want[:, 1:5, 1:5] = 27
     np.testing.assert_array_equal(out, want)
+
+
+def test_captured_ragged_calls_keep_no_growable_scratch():
+    # an eager call splits K and leaves the stream's workspace behind, the
+    # captured one runs unsplit; a larger call then replaces the workspace
+    # between replays
+    L = capi.lib()
+    # the HIP runtime this process runs on
+    hip = ctypes.CDLL(next(ln.split()[-1] for ln in open("/proc/self/maps") if "libamdhip64" in ln))
+    stream = ctypes.c_void_p(L.xtc_hip_stream_create())
+    M, N, K = 130, 253, 515
+    a, b = rng_uniform(21, (M, K)), rng_uniform(22, (K, N))
+    A, B = DeviceBuffer.from_numpy(a), DeviceBuffer.from_numpy(b)
+    C, E = DeviceBuffer(M * N * 4), DeviceBuffer(M * N * 4)
+    big = DeviceBuffer(1021 * 1021 * 4)
+    big.zero()
+
+    def call(out, m, n, k, x, y, split):
+        d = capi.MatmulDesc(dtype=capi.XTC_HIP_F32, M=m, N=n, K=k, split_k=split, stream=stream, xcd_remap=1)
+        d.tile = capi.Tile(64, 64, 32, 2, 2)
+        capi.check(L.xtc_hip_matmul(ctypes.byref(d), x.c_ptr, y.c_ptr, out.c_ptr, None), "matmul")
+
+    def ok(code):
+        assert code == 0, code
+
+    def eager(split):
+        call(E, M, N, K, A, B, split)
+        capi.check(L.xtc_hip_stream_synchronize(stream), "sync")
+        return E.to_numpy((M, N), np.float32)
+
+    split4, unsplit = eager(4), eager(1)
+    check(split4, a, b)
+    graph, run = ctypes.c_void_p(), ctypes.c_void_p()
+    ok(hip.hipStreamBeginCapture(stream, 1))
+    call(C, M, N, K, A, B, 4)
+    ok(hip.hipStreamEndCapture(stream, ctypes.byref(graph)))
+    ok(hip.hipGraphInstantiate(ctypes.byref(run), graph, None, None, ctypes.c_size_t(0)))
+    for _ in range(4):
+        C.zero()
+        capi.check(L.xtc_hip_synchronize(), "sync")
+        ok(hip.hipGraphLaunch(run, stream))
+        capi.check(L.xtc_hip_stream_synchronize(stream), "sync")
+        np.testing.assert_array_equal(C.to_numpy((M, N), np.float32), unsplit)
+        out = DeviceBuffer(1021 * 1021 * 4)
+        call(out, 1021, 1021, 1021, big, big, 8)
+        np.testing.assert_array_equal(eager(4), split4)
+    ok(hip.hipGraphExecDestroy(run))
+    ok(hip.hipGraphDestroy(graph))
+    capi.check(L.xtc_hip_stream_destroy(stream), "destroy")

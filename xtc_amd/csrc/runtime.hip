@@ -1993,10 +1993,22 @@ int launch_f64_gemm(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int spl
 // Row stride of the split-K workspace of gemm_planes: whole vectors of 4.
 int planes_ldp(int N) { return (N + 3) / 4 * 4; }
 
+// Whether `s` is being captured in a graph (or cannot be asked).
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &status) != hipSuccess) {
+    (void)hipGetLastError();  // not the launch's error
+    return true;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
 // Splits of a launch that must not fail for want of scratch (shapes whose
 // calls took none before they ran on gemm_planes): `split_k`, or 1 where the
-// split-K scratch would pass the fixed scratch or 1 GiB, or would have to be
-// allocated while the stream is being captured.
+// split-K scratch would pass the fixed scratch or 1 GiB, and on a stream that
+// is being captured: the graph would keep the address of a growable buffer,
+// which a later call frees to enlarge it and a replay on another stream shares
+// with the launches of this one.
 int splits_with_room(int split_k, int M, int N, int K, const xtc_hip_tile& t, const Scratch& x) {
   const int splits = effective_splits(K, split_k, t.bk);
   if (splits == 1) return 1;
@@ -2004,15 +2016,7 @@ int splits_with_room(int split_k, int M, int N, int K, const xtc_hip_tile& t, co
   const size_t bytes = (size_t)splits * M * planes_ldp(N) * sizeof(float);
   if (x.fixed)  // two 256-byte alignments
     return bytes + tiles * sizeof(unsigned) + 512 <= x.cap - x.used ? split_k : 1;
-  if (bytes > ((size_t)1 << 30)) return 1;
-  {
-    std::lock_guard<std::mutex> lk(g_mutex);
-    const StreamScratch* y = stream_scratch(x.s);
-    if (y && y->workspace_bytes >= bytes && y->counters_len >= tiles) return split_k;
-  }
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(x.s, &status) != hipSuccess) return 1;
-  return status == hipStreamCaptureStatusNone ? split_k : 1;
+  return bytes > ((size_t)1 << 30) || capturing(x.s) ? 1 : split_k;
 }
 
 int matmul_impl(const xtc_hip_matmul_desc& d, const void* A, const void* B, void* Cv, const void* biasv,
