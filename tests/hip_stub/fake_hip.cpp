@@ -53,7 +53,9 @@ void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
 void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, void*, void*,
                            int*) {
   int status = 0;
-  char* plain = abi::__cxa_demangle(name, nullptr, nullptr, &status);
+  std::string mangled = name;  // the demangler does not know the type __bf16
+  for (size_t at; (at = mangled.find("DF16b")) != std::string::npos;) mangled.replace(at, 5, "u6__bf16");
+  char* plain = abi::__cxa_demangle(mangled.c_str(), nullptr, nullptr, &status);
   g_kernels[host] = status == 0 ? plain : name;
   free(plain);
 }

@@ -101,3 +101,24 @@ out.append(matmul("float32", 509, 1021, 777, fn="xtc_hip_matmul_noalloc"))
     assert conv_eager[-1][1] == 4 and conv_captured == [[conv_eager[-1][0], 1, conv_eager[-1][2]]]
     # the static scratch of the no-allocation entry point stays: split as ever
     assert noalloc[-1] == [kernel, 4, 256]
+
+
+def test_calls_without_whole_vectors_run_unsplit_where_scratch_cannot_be_had(run):
+    # no memory at all, and enough for the partial sums but not the counters;
+    # a conv whose filters are not whole vectors; then memory again
+    none, counters, conv, later, message = run("""
+fake.fake_memory(1 << 20)
+out.append(matmul("float32", 509, 1021, 777))
+fake.fake_memory(4 * 509 * 1024 * 4 + 1000)
+out.append(matmul("float32", 509, 1021, 777))
+fake.fake_memory(1000)
+out.append(conv("bfloat16", 1, 14, 14, 333, 67, 3, 3, pad=1, split=4))
+fake.fake_memory(1 << 30)
+out.append(matmul("float32", 509, 1021, 777))
+out.append(L.xtc_hip_last_error().decode())
+""")
+    kernel = "gemm_planes<float, 64, 64, 32, 2, 2, false, false, false, 1, 1>"
+    assert none == counters == [[kernel, 1, 256]]
+    assert conv == [["gemm_planes<__bf16, 64, 64, 64, 2, 2, true, false, false, 1, 1>", 1, 256]]
+    assert later[-1] == [kernel, 4, 256]
+    assert message == ""

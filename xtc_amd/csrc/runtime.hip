@@ -2005,10 +2005,10 @@ bool capturing(hipStream_t s) {
 
 // Splits of a launch that must not fail for want of scratch (shapes whose
 // calls took none before they ran on gemm_planes): `split_k`, or 1 where the
-// split-K scratch would pass the fixed scratch or 1 GiB, and on a stream that
-// is being captured: the graph would keep the address of a growable buffer,
-// which a later call frees to enlarge it and a replay on another stream shares
-// with the launches of this one.
+// split-K scratch would pass the fixed scratch or 1 GiB or cannot be allocated,
+// and on a stream that is being captured: the graph would keep the address of a
+// growable buffer, which a later call frees to enlarge it and a replay on
+// another stream shares with the launches of this one.
 int splits_with_room(int split_k, int M, int N, int K, const xtc_hip_tile& t, const Scratch& x) {
   const int splits = effective_splits(K, split_k, t.bk);
   if (splits == 1) return 1;
@@ -2016,7 +2016,10 @@ int splits_with_room(int split_k, int M, int N, int K, const xtc_hip_tile& t, co
   const size_t bytes = (size_t)splits * M * planes_ldp(N) * sizeof(float);
   if (x.fixed)  // two 256-byte alignments
     return bytes + tiles * sizeof(unsigned) + 512 <= x.cap - x.used ? split_k : 1;
-  return bytes > ((size_t)1 << 30) || capturing(x.s) ? 1 : split_k;
+  if (bytes > ((size_t)1 << 30) || capturing(x.s)) return 1;
+  if (workspace(bytes, x.s) && split_counters(tiles, x.s)) return split_k;
+  (void)hipGetLastError();  // of the failed allocation
+  return 1;
 }
 
 int matmul_impl(const xtc_hip_matmul_desc& d, const void* A, const void* B, void* Cv, const void* biasv,
