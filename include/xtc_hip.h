@@ -148,6 +148,14 @@ typedef struct {
                                 threshold cannot hold every fp64 value) */
 } xtc_hip_matmul_desc;
 
+/* Split-K partial sums, counters and copies of transposed operands live in
+ * buffers of the stream that grow on demand; a call fails with a message when
+ * one cannot be allocated.  fp32 and bf16 calls without whole 16-byte vectors
+ * (strides, K, N or operand addresses), which no scratch may stop, run unsplit
+ * instead: where their scratch would not fit in
+ * XTC_HIP_NOALLOC_SCRATCH_BYTES or cannot be allocated, and on a stream that is
+ * being captured, so that the graph keeps no address of a buffer that a later
+ * call replaces (the sums are then in another order). */
 int xtc_hip_matmul(const xtc_hip_matmul_desc *desc, const void *A, const void *B,
                    void *C, const void *bias);
 
@@ -158,13 +166,15 @@ int xtc_hip_matmul(const xtc_hip_matmul_desc *desc, const void *A, const void *B
  * allocation).  It has no counterpart in the reference: it is for callers
  * that cannot allocate device memory, such as code under HIP graph capture,
  * tight serving loops and harnesses that forbid allocation.  Same arguments,
- * kernels and results as xtc_hip_matmul.  Its scratch -- split-K partial sums
- * ([splits][M][N] fp32, or [splits][16][N] for the skinny kernel), one
- * arrival counter per output tile, and dense copies of transposed operands
- * that the kernels cannot read in place -- comes from one static array per
- * device of XTC_HIP_NOALLOC_SCRATCH_BYTES, set up by xtc_hip_init.  A call
- * that needs more fails with a message instead of launching its GEMM.  The
- * counters are cleared by a kernel on the call's stream before the GEMM.
+ * kernels and results as xtc_hip_matmul (of a stream that is not being
+ * captured).  Its scratch -- split-K partial sums ([splits][M][N] fp32, with N
+ * rounded up to 4 where it is not a multiple, or [splits][16][N] for the
+ * skinny kernel), one arrival counter per output tile, and dense copies of
+ * transposed operands that the kernels cannot read in place -- comes from one
+ * static array per device of XTC_HIP_NOALLOC_SCRATCH_BYTES, set up by
+ * xtc_hip_init.  A call that needs more fails with a message instead of
+ * launching its GEMM; an fp32 or bf16 call without whole 16-byte vectors runs
+ * unsplit instead, here and in xtc_hip_matmul.  The counters are cleared by a kernel on the call's stream before the GEMM.
  * Every call on a device shares that device's array, whatever its stream:
  * calls that overlap on one device race, so callers order them (one stream,
  * or a wait between streams). */

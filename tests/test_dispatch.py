@@ -122,3 +122,21 @@ out.append(L.xtc_hip_last_error().decode())
     assert conv == [["gemm_planes<__bf16, 64, 64, 64, 2, 2, true, false, false, 1, 1>", 1, 256]]
     assert later[-1] == [kernel, 4, 256]
     assert message == ""
+
+
+@pytest.mark.parametrize("shape,split,trans_a,splits", [
+    ((509, 1021, 777), 4, 0, 4),
+    ((4097, 4097, 300), 2, 0, 1),  # 134 MB of partial sums
+    ((2500, 1001, 4001), 3, 1, 1),  # 30 MB of them behind a 40 MB copy of A
+    ((2500, 1001, 2001), 3, 1, 3),
+])
+def test_both_entry_points_split_ragged_calls_alike(run, shape, split, trans_a, splits):
+    # the partial sums of either entry point stay within the static scratch,
+    # so that the sums are taken in the same order
+    M, N, K = shape
+    grown, static = run(f"""
+for fn in ("xtc_hip_matmul", "xtc_hip_matmul_noalloc"):
+    out.append(matmul("float32", {M}, {N}, {K}, split={split}, trans_a={trans_a}, tile=(64, 64, 32, 2, 2), fn=fn))
+""")
+    kernel = "gemm_planes<float, 64, 64, 32, 2, 2, false, false, false, 1, 1>"
+    assert grown[-1] == static[-1] == [kernel, splits, 256]

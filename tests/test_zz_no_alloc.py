@@ -101,6 +101,11 @@ CASES = [
     ("bfloat16", (256, 256, 32, 2, 4), 4, (512, 768, 2048), (256, 256, 1024), {"relu": True, "bias": True}),
     # ping-pong bf16 kernel reading B^T natively, split-K 2
     ("bfloat16", (256, 256, 32, 2, 4), 2, (512, 512, 1024), (256, 512, 512), {"trans_b": True}),
+    # no whole vectors: split with partial rows rounded up to 4, transposed copies ahead of
+    # them, and unsplit in both entry points where the partial sums pass the array (134 MB)
+    ("float32", (64, 64, 32, 2, 2), 4, (509, 1021, 777), (65, 131, 515), {"relu": True, "bias": True}),
+    ("bfloat16", (64, 64, 64, 2, 2), 3, (130, 253, 1030), (33, 67, 515), {"trans_a": True, "trans_b": True}),
+    ("float32", (64, 64, 32, 2, 2), 2, (4097, 4097, 150), (129, 131, 150), {}),
 ]
 
 

@@ -196,7 +196,7 @@ struct Scratch {
   hipStream_t s;
   char* fixed = nullptr;
   size_t cap = 0;
-  size_t used = 0;
+  size_t used = 0;  // in growing mode: by staged copies
 
   void* take(size_t bytes, const char* what) {
     const size_t off = (used + 255) & ~(size_t)255;
@@ -229,6 +229,7 @@ struct Scratch {
   }
   void* stage(int slot, size_t bytes) {
     if (fixed) return take(bytes, "transposed operand copies");
+    used = ((used + 255) & ~(size_t)255) + bytes;  // as take() counts (splits_with_room)
     void* p = staging(slot, bytes, s);
     if (!p) fail("cannot allocate %zu bytes of transpose staging", bytes);
     return p;
@@ -2005,18 +2006,21 @@ bool capturing(hipStream_t s) {
 
 // Splits of a launch that must not fail for want of scratch (shapes whose
 // calls took none before they ran on gemm_planes): `split_k`, or 1 where the
-// split-K scratch would pass the fixed scratch or 1 GiB or cannot be allocated,
-// and on a stream that is being captured: the graph would keep the address of a
-// growable buffer, which a later call frees to enlarge it and a replay on
-// another stream shares with the launches of this one.
+// split-K scratch would not fit in the no-allocation entry point's, whichever
+// entry point is called, so that both take their sums in the same order (the
+// library's own splits need 38 MB at most).  In growing mode also 1 where it
+// cannot be allocated, and on a stream that is being captured: the graph would
+// keep the address of a growable buffer, which a later call frees to enlarge it
+// and a replay on another stream shares with the launches of this one.
 int splits_with_room(int split_k, int M, int N, int K, const xtc_hip_tile& t, const Scratch& x) {
   const int splits = effective_splits(K, split_k, t.bk);
   if (splits == 1) return 1;
   const size_t tiles = (size_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
   const size_t bytes = (size_t)splits * M * planes_ldp(N) * sizeof(float);
-  if (x.fixed)  // two 256-byte alignments
-    return bytes + tiles * sizeof(unsigned) + 512 <= x.cap - x.used ? split_k : 1;
-  if (bytes > ((size_t)1 << 30) || capturing(x.s)) return 1;
+  // two 256-byte alignments
+  if (x.used + bytes + tiles * sizeof(unsigned) + 512 > XTC_HIP_NOALLOC_SCRATCH_BYTES) return 1;
+  if (x.fixed) return split_k;
+  if (capturing(x.s)) return 1;
   if (workspace(bytes, x.s) && split_counters(tiles, x.s)) return split_k;
   (void)hipGetLastError();  // of the failed allocation
   return 1;
