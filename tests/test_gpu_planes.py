@@ -140,6 +140,22 @@ def test_operands_near_the_ends_of_the_range(scale_a, scale_b):
     check(run_matmul(a, b, tile=TILES[2], split_k=1), a, b)
 
 
+@pytest.mark.parametrize("exp", [-126, -120, -117])
+@pytest.mark.parametrize("tile", [TILES[0], (64, 64, 32, 2, 2)])
+def test_small_normal_operands_that_cancel(tile, exp):
+    # normal operands below 2^-110 lose the bits below 2^-133: x and 2^exp
+    # have the same planes, so that every sum of the planes is exactly zero,
+    # where the product with 2^100 is not
+    M, N, K = (8, 8, 96) if tile[0] == 256 else (1500, 1500, 256)
+    a, b = np.zeros((M, K), np.float32), np.full((K, N), 2.0**100, np.float32)
+    x = np.ldexp(1 + 2.0 ** -np.arange(exp + 135, 24), exp).astype(np.float32)
+    for i in range(M):
+        k = (7 * i) % (K - 1)
+        a[i, k], a[i, k + 1] = x[i % len(x)], -np.float32(2.0**exp)
+    b[:, 1::2] = 2.0**-3
+    check(run_matmul(a, b, tile=tile, split_k=1), a, b)
+
+
 def test_infinities_and_nan():
     rng = np.random.default_rng(9)
     a = rng.integers(1, 5, (256, 160)).astype(np.float32)

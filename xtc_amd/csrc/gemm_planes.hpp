@@ -15,14 +15,18 @@
 // fp32 MFMA rounds at every product.
 //
 // What the split cannot hold is computed on fp32 MFMAs instead.  A lane keeps
-// the largest |operand| it staged and whether one was denormal; after the K
-// walk a wave looks at its sums.  An infinity or NaN among the operands (or an
-// operand above the bf16 range) leaves a non-finite sum; operands below 2^-110
-// lose bits of their m and l parts (bf16 ends at 2^-133), an error of at most
-// K 2^-126 max|operand|, which matters only to sums below 2^-90 max|operand|,
-// and to zeros only where denormals took part.  A wave that finds such a sum
-// repeats its tile with v_mfma_f32_16x16x4_f32 straight from global memory
-// (slow, and exact in the same cases as the fp32 MFMA).
+// the largest and the smallest nonzero |operand| it staged; after the K walk a
+// wave looks at its sums.  An infinity or NaN among the operands (or an
+// operand above the bf16 range) leaves a non-finite sum; operands below 2^-110,
+// denormal or not, lose bits of their m and l parts (bf16 ends at 2^-133), an
+// error of at most K 2^-126 max|operand|, which matters only to sums below
+// 2^-90 max|operand|, and to zeros only where such operands took part.  A wave
+// that finds such a sum repeats its tile with v_mfma_f32_16x16x4_f32 straight
+// from global memory (exact in the same cases as the fp32 MFMA).  A zero row
+// alone costs nothing; with one operand of 2^-112 in it a workgroup whose
+// waves hold zero sums repeats them: 2048x4096x1024 98 us, 286 with one such
+// row tile in the matrix, 388 with one in every wave; 4096^3 668, 1789, 2699;
+// 1024x1024x256 18, 58, 75.
 //
 // Structure (per workgroup = one BM x BN output tile, one split of K):
 //   * WGM x WGN waves of (BM/WGM) x (BN/WGN), K in slabs of BK through two
@@ -170,13 +174,15 @@ __device__ __forceinline__ void lds_write16(unsigned char* dst, u32x4 v) {
   *reinterpret_cast<lds_u32x4*>((lds_byte*)dst) = v;
 }
 
+// twice the bits of |x|, less one: orders nonzero magnitudes, zeros above all
+__device__ __forceinline__ unsigned nonzero_key(float x) { return (__float_as_uint(x) << 1) - 1u; }
+
 // dword e of the three planes of a unit: elements 2 e and 2 e + 1 split;
-// top: largest magnitude seen, denormal: whether any was one
-__device__ __forceinline__ void split2(const Unit<float>& u, int e, u32x4 (&w)[3], float& top, bool& denormal) {
+// top: largest magnitude seen, low: key of the smallest nonzero one
+__device__ __forceinline__ void split2(const Unit<float>& u, int e, u32x4 (&w)[3], float& top, unsigned& low) {
   f32x2 x = {u.v[2 * e], u.v[2 * e + 1]};
   top = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), top);
-  constexpr int kDenormal = 0x90;
-  denormal = denormal || __builtin_amdgcn_classf(x[0], kDenormal) || __builtin_amdgcn_classf(x[1], kDenormal);
+  low = min(min(nonzero_key(x[0]), nonzero_key(x[1])), low);
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
     const unsigned h = __builtin_bit_cast(unsigned, __builtin_convertvector(x, bf16x2));
@@ -289,7 +295,7 @@ gemm_planes(GemmArgs args) {
   Unit<T> areg[RING][X::A_PER], breg[RING][X::B_PER];
   unsigned a_in[RING][X::A_PER];  // conv: which vectors (or elements) of the unit lie inside the image
   float top = 0.f;                // fp32: largest |operand| staged by this lane
-  bool denormal = false;          // fp32: whether one of them was denormal
+  unsigned low = ~0u;             // fp32: key of the smallest nonzero one
 
   // Unit u of register set `slot` from a whole slab of VEC operands at k = kt.
   const bool inside = BT || n0 + BN <= args.N;
@@ -407,7 +413,7 @@ gemm_planes(GemmArgs args) {
                         : st + b_dst + (u - X::A_PER) * BR * (BT ? 2 * BK : 2 * BN);
   };
   auto split_pair = [&](int u, int slot, int e, u32x4 (&w)[3]) {
-    if constexpr (F32) split2(u < X::A_PER ? areg[slot][u] : breg[slot][u - X::A_PER], e, w, top, denormal);
+    if constexpr (F32) split2(u < X::A_PER ? areg[slot][u] : breg[slot][u - X::A_PER], e, w, top, low);
   };
   auto write_unit = [&](unsigned char* st, int u, const u32x4 (&w)[3]) {
     unsigned char* dst = unit_dst(st, u);
@@ -636,18 +642,18 @@ gemm_planes(GemmArgs args) {
 #pragma unroll
     for (int s = 1; s < 64; s *= 2) top = fmaxf(top, __shfl_xor(top, s));
     __shared__ float tops[WGM * WGN];
-    __shared__ unsigned denormals[WGM * WGN];
-    const bool any = __any(denormal);
+    __shared__ unsigned smalls[WGM * WGN];
+    const bool any = __any(low < nonzero_key(0x1p-110f));
     if (lane == 0) {
       tops[wave] = top;
-      denormals[wave] = any;
+      smalls[wave] = any;
     }
     __syncthreads();
-    unsigned seen = 0;
+    unsigned small = 0;
 #pragma unroll
     for (int w = 0; w < WGM * WGN; ++w) {
       top = fmaxf(top, tops[w]);
-      seen |= denormals[w];
+      small |= smalls[w];
     }
     const float floor = top * 0x1p-90f;
     bool bad = false;
@@ -658,7 +664,7 @@ gemm_planes(GemmArgs args) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float v = fabsf(acc[i][j][r]);
-          bad = bad || !(v < INFINITY) || (v == 0.f ? seen != 0 : v < floor);
+          bad = bad || !(v < INFINITY) || (v == 0.f ? small != 0 : v < floor);
         }
     if (__ballot(bad)) {
 #pragma unroll
