@@ -267,9 +267,21 @@ typedef struct {
 int xtc_hip_gemm_instance_count(void);
 int xtc_hip_gemm_instance_get(int index, xtc_hip_gemm_instance *out);
 
-/* Tile the library picks when a descriptor leaves `tile` zeroed. */
+/* Tile and split of a shape's class, from its sizes alone: where the library's
+ * choice for a descriptor that leaves `tile` zeroed starts
+ * (xtc_hip_matmul_default_tile, xtc_hip_conv2d_default_tile). */
 int xtc_hip_default_tile(int dtype, int conv, int M, int N, int K, xtc_hip_tile *out,
                          int *split_k);
+
+/* Tile and split a matmul descriptor gets when it leaves `tile` zeroed (a
+ * split_k that it names stays).  Unlike xtc_hip_default_tile(dtype, 0, ...) it
+ * sees the operands' layouts and strides: fp32 calls whose class is a 64x64x32
+ * or 128x128x32 tile of 2x2 waves move to an 8-wave tile of the bf16-plane
+ * kernel, with no more splits, where that is estimated to be faster, and bf16
+ * calls on 128-row tiles split K no more often than fills the CUs once.  A tile
+ * that a descriptor names runs as named, with the named split (but calls
+ * without whole 16-byte vectors, whose kernels have blocks of their own). */
+int xtc_hip_matmul_default_tile(const xtc_hip_matmul_desc *desc, xtc_hip_tile *out, int *split_k);
 
 /* Tile a conv2d descriptor gets when it leaves `tile` zeroed.  Unlike
  * xtc_hip_default_tile(dtype, 1, ...) it sees the window, strides and pads:

@@ -140,3 +140,75 @@ for fn in ("xtc_hip_matmul", "xtc_hip_matmul_noalloc"):
 """)
     kernel = "gemm_planes<float, 64, 64, 32, 2, 2, false, false, false, 1, 1>"
     assert grown[-1] == static[-1] == [kernel, splits, 256]
+
+
+@pytest.mark.parametrize("dtype,tile,split,shape,trans_b,kernel", [
+    ("float32", (64, 64, 32, 2, 2), 2, (2000, 2304, 2600), 0, "gemm_planes<float, 64, 64, 32, 2, 2, false, false, true, 1, 1>"),
+    ("float32", (64, 64, 32, 2, 2), 1, (2048, 2048, 1024), 1, "gemm_planes<float, 64, 64, 32, 2, 2, false, true, true, 1, 1>"),
+    ("float32", (64, 64, 32, 2, 2), 8, (1000, 1104, 1200), 0, "gemm_planes<float, 64, 64, 32, 2, 2, false, false, true, 1, 1>"),
+    ("float32", (64, 64, 32, 2, 2), 8, (768, 768, 4096), 0, "gemm_planes<float, 64, 64, 32, 2, 2, false, false, true, 1, 1>"),
+    ("float32", (128, 128, 32, 2, 2), 1, (3000, 3000, 3000), 0, "gemm_kernel<float, 128, 128, 32, 2, 2, false, 1>"),
+    ("float32", (128, 128, 32, 2, 2), 3, (256, 4608, 8192), 0, "gemm_kernel<float, 128, 128, 32, 2, 2, false, 1>"),
+    ("float32", (128, 256, 32, 2, 4), 2, (2048, 1024, 4096), 0, "gemm_planes<float, 128, 256, 32, 2, 4, false, false, true, 1, 1>"),
+    ("bfloat16", (128, 128, 64, 2, 2), 4, (256, 8192, 4608), 0, "gemm_planes<__bf16, 128, 128, 64, 2, 4, false, false, true, 2, 1>"),
+    ("bfloat16", (128, 128, 64, 2, 2), 2, (256, 8192, 4608), 0, "gemm_planes<__bf16, 128, 128, 64, 2, 4, false, false, true, 1, 2>"),
+    ("bfloat16", (128, 128, 64, 2, 2), 4, (256, 4608, 8192), 1, "gemm_planes<__bf16, 128, 128, 64, 2, 4, false, true, true, 1, 1>"),
+])
+def test_named_matmuls_run_their_tile_and_split(run, dtype, tile, split, shape, trans_b, kernel):
+    M, N, K = shape
+    (rows,) = run(f"out.append(matmul({dtype!r}, {M}, {N}, {K}, tile={tile}, split={split}, trans_b={trans_b}))")
+    assert [rows[-1][0], rows[-1][1]] == [kernel, split]
+
+
+@pytest.mark.parametrize("tile,split,shape", [((128, 64, 64, 2, 2), 4, (1, 34, 34, 256, 512, 3)),
+                                              ((128, 128, 64, 2, 2), 8, (1, 17, 17, 1024, 1024, 3))])
+def test_named_convs_run_their_split(run, tile, split, shape):
+    n, h, w, c, f, r = shape
+    (rows,) = run(f"out.append(conv('bfloat16', {n}, {h}, {w}, {c}, {f}, {r}, {r}, pad=1, tile={tile}, split={split}))")
+    assert rows[-1][0].startswith(f"gemm_planes<__bf16, {tile[0]}, {tile[1]}, 64,") and rows[-1][1] == split
+
+
+def test_default_queries_name_what_an_unnamed_call_runs(run):
+    # over shapes, layouts and strides: the tile and split that the query
+    # returns, named, launch what the zeroed tile does
+    pairs = run("""
+import random
+rng = random.Random(3)
+pick = lambda step: max(step, int(8 * 1024 ** rng.random()) // step * step)
+for i in range(400):
+    dtype, step = rng.choice(("float32", "bfloat16", "float64")), rng.choice((1, 8, 64, 128))
+    M, N, K = pick(rng.choice((1, 64))), pick(step), pick(step)
+    kw = dict(trans_b=rng.randint(0, 1), trans_a=int(rng.random() < 0.2), relu=rng.randint(0, 1))
+    if rng.random() < 0.2:
+        kw["ldb"] = (K if kw["trans_b"] else N) + rng.choice((1, 8, 64))
+    d = capi.MatmulDesc(dtype=capi.DTYPE_IDS[dtype], M=M, N=N, K=K, **kw)
+    tile, split = capi.matmul_default_tile(d)
+    out.append([repr((dtype, M, N, K, kw)), matmul(dtype, M, N, K, **kw),
+                matmul(dtype, M, N, K, tile=tile, split=split, **kw)])
+for i in range(200):
+    dtype, r = rng.choice(("float32", "bfloat16", "float64")), rng.choice((1, 3, 5))
+    h, c, f = rng.randint(7, 60), rng.choice((3, 16, 32, 64, 256)), rng.choice((7, 16, 64, 96, 512))
+    d = capi.Conv2dDesc(dtype=capi.DTYPE_IDS[dtype], N=1, H=h, W=h, C=c, F=f, R=r, S=r, stride_h=1, stride_w=1,
+                        pad_top=1, pad_bottom=1, pad_left=1, pad_right=1)
+    tile, split = capi.conv2d_default_tile(d)
+    out.append([repr((dtype, h, c, f, r)), conv(dtype, 1, h, h, c, f, r, r, pad=1),
+                conv(dtype, 1, h, h, c, f, r, r, pad=1, tile=tile, split=split)])
+""")
+    assert len(pairs) == 600
+    for what, unnamed, named in pairs:
+        assert isinstance(named, list), (what, named)
+        # but for counters cleared when they are first allocated
+        unnamed, named = ([r for r in rows if r[0] != "fill_zero_kernel"] for rows in (unnamed, named))
+        assert unnamed == named, what
+
+
+def test_default_configs_report_the_kernel_that_runs():
+    import xtc_amd.graphs.xtc.op as O
+    from xtc_amd.backends.hip import Backend
+
+    a, b = O.tensor((2048, 1024), "float32", name="A"), O.tensor((1024, 2048), "float32", name="B")
+    with O.graph(name="mm") as gb:
+        O.matmul(a, b, name="C")
+    backend = Backend(gb.graph)
+    cfg = backend.get_compiler().kernel_configs(backend.get_scheduler().schedule())["C"]
+    assert cfg.tile == (128, 128, 32, 2, 4) and cfg.split_k == 1 and cfg.source == "default"

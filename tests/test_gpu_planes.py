@@ -53,19 +53,27 @@ def test_edges(tile, M, N, K, split):
     check(run_matmul(a, b, tile=tile, split_k=split), a, b)
 
 
-# tiles of four waves whose product runs on an 8-wave tile instead: the generic
-# 128x128 one at its edges, the 64x64 one where the estimate says so (K split
-# less often than asked, cut by M and N); the bound covers every split count
-@pytest.mark.parametrize("tile,M,N,K,split", [((128, 128, 32, 2, 2), 1, 4, 4, 1), ((128, 128, 32, 2, 2), 129, 260, 100, 1),
-                                              ((128, 128, 32, 2, 2), 300, 132, 1156, 3),
-                                              ((64, 64, 32, 2, 2), 1000, 1104, 1200, 8),
-                                              ((64, 64, 32, 2, 2), 257, 2308, 2052, 8),
-                                              ((64, 64, 32, 2, 2), 1281, 3076, 516, 1)])
-def test_four_wave_tiles_on_eight_waves(tile, M, N, K, split):
-    print(f"[planes wide] {tile} {M}x{N}x{K} split {split}", flush=True)
+# default calls whose class is a 64x64 or 128x128 tile of four waves and which
+# run on an 8-wave one: cut by M, N and K, K split less often than the class says
+@pytest.mark.parametrize("trans_b,M,N,K,cls,tile,splits", [
+    (False, 1000, 1104, 1200, 64, (128, 128, 32, 2, 4), 3),
+    (True, 257, 2308, 2052, 64, (128, 128, 32, 2, 4), 4),
+    (True, 258, 4100, 4100, 64, (128, 256, 32, 2, 4), 4),
+    (False, 300, 2052, 8196, 64, (128, 128, 32, 2, 4), 5),
+    (True, 1284, 4612, 260, 64, (256, 128, 32, 4, 2), 1),
+    (False, 2049, 2052, 100, 128, (256, 128, 32, 4, 2), 1),
+    (True, 2050, 2308, 1156, 128, (256, 128, 32, 4, 2), 1),
+])
+def test_default_calls_on_eight_wave_tiles(trans_b, M, N, K, cls, tile, splits):
+    print(f"[planes wide] {M}x{N}x{K} trans_b {trans_b}", flush=True)
+    d = capi.MatmulDesc(dtype=capi.XTC_HIP_F32, M=M, N=N, K=K, trans_b=int(trans_b))
+    assert capi.default_tile("float32", False, M, N, K)[0][0] == cls
+    assert capi.matmul_default_tile(d) == (tile, splits)
     a, b = rng_uniform(M + K, (M, K)), rng_uniform(N + K, (K, N))
-    check(run_matmul(a, b, tile=tile, split_k=split), a, b)
-    check(run_matmul_layout(a, b, "float32", False, True, tile=tile, split_k=split), a, b)
+    out = run_matmul_layout(a, b, "float32", False, trans_b)
+    check(out, a, b)
+    # the tile and split by name: the same call
+    np.testing.assert_array_equal(run_matmul_layout(a, b, "float32", False, trans_b, tile=tile, split_k=splits), out)
 
 
 # no whole vectors anywhere: fp32 and bf16 rows at element alignment, units cut
@@ -110,11 +118,16 @@ def test_transposed_b(dtype, tile, M, N, K, split):
         np.testing.assert_array_equal(out, ai.astype(np.float64) @ bi)
 
 
-# bf16 workgroups of 4 or 8 waves (512 and 520 of them), and more splits asked
-# for than the 128-row tiles run (66 tiles, 18.1 and 4 slabs)
+# bf16 workgroups of 4 or 8 waves (512 and 520 of them); 128-row tiles whose
+# splits pass the 256 CUs (462 and 264 workgroups), fit them with fewer than 8
+# slabs, and fit them on two k-groups (198 workgroups of 12, 12 and 10 slabs, the
+# last one cut by K; 256 of 11 slabs, 6 and 5 a group)
 @pytest.mark.parametrize("tile,M,N,K,split", [((64, 64, 64, 2, 2), 1024, 2048, 136, 1), ((64, 64, 64, 2, 2), 505, 4136, 136, 1),
                                               ((64, 64, 64, 2, 2), 505, 2088, 264, 2), ((128, 128, 64, 2, 2), 129, 4104, 1160, 8),
-                                              ((128, 128, 64, 2, 2), 256, 4224, 256, 4)])
+                                              ((128, 128, 64, 2, 2), 256, 4224, 256, 4),
+                                              ((128, 128, 64, 2, 2), 256, 4224, 1160, 3),
+                                              ((128, 128, 64, 2, 2), 256, 4224, 2120, 3),
+                                              ((128, 128, 64, 2, 2), 250, 4088, 2816, 4)])
 def test_bf16_workgroups_and_splits(tile, M, N, K, split):
     print(f"[planes bf16] {tile} {M}x{N}x{K} split {split}", flush=True)
     ai, bi = ref.np_init((M, K), "float32"), ref.np_init((K, N), "float32")[::-1].copy()
@@ -176,7 +189,8 @@ def test_infinities_and_nan():
 
 
 def test_small_tile_edges():
-    # 64x64x32 runs here from 512 workgroups of 8 slabs unsplit
+    # 64x64x32 runs here from 512 workgroups of 8 slabs unsplit, and of 4 slabs
+    # from 1152 with K split
     for M, N, K in ((1400, 1540, 260), (2050, 1028, 1000)):
         a, b = rng_uniform(M, (M, K)), rng_uniform(N, (K, N))
         check(run_matmul(a, b, tile=(64, 64, 32, 2, 2), split_k=1), a, b)

@@ -157,20 +157,35 @@ def _default(dtype: str, conv: bool, M: int, N: int, K: int,
              attrs: dict[str, Any] | None = None) -> tuple[tuple[int, int, int, int, int], int]:
     from ...runtimes.hip import capi
 
-    if conv and attrs is not None:
-        return default_conv_tile(attrs)
+    if attrs is not None:
+        return default_conv_tile(attrs) if conv else default_matmul_tile(attrs)
     return capi.default_tile(dtype, conv, M, N, K)
+
+
+def default_matmul_tile(attrs: dict[str, Any]) -> tuple[tuple[int, int, int, int, int], int]:
+    """The library's default (tile, split_k) for a matmul launch: it sees the
+    operands' layouts and strides (xtc_hip_matmul_default_tile).  A piece of a
+    split matmul whose operands start off a 16-byte boundary keeps its class's."""
+    from ...runtimes.hip import capi
+
+    dtype, m, n, k, ta, tb = _attrs_key(attrs, False)
+    if not attrs.get("aligned", True):
+        return capi.default_tile(dtype, False, m, n, k)
+    return capi.matmul_default_tile(capi.MatmulDesc(dtype=capi.DTYPE_IDS[dtype], M=m, N=n, K=k, trans_a=int(ta),
+                                                    trans_b=int(tb), lda=attrs.get("lda", 0), ldb=attrs.get("ldb", 0),
+                                                    ldc=attrs.get("ldc", 0)))
 
 
 def default_conv_tile(attrs: dict[str, Any]) -> tuple[tuple[int, int, int, int, int], int]:
     """The library's default (tile, split_k) for a conv2d launch: it sees the
-    window and strides (xtc_hip_conv2d_default_tile)."""
+    window, strides and pads (xtc_hip_conv2d_default_tile)."""
     from ...runtimes.hip import capi
 
     _, nb, h, w, c, f, r, s, (sh, sw), (pt, pb, pl, pr) = _attrs_key(attrs, True)
     dt = capi.DTYPE_IDS[attrs["dtype"]]
+    pad = float(attrs.get("pad_value", 0.0))
     cd = capi.Conv2dDesc(dtype=dt, N=nb, H=h, W=w, C=c, F=f, R=r, S=s, stride_h=sh, stride_w=sw, pad_top=pt,
-                         pad_bottom=pb, pad_left=pl, pad_right=pr)
+                         pad_bottom=pb, pad_left=pl, pad_right=pr, pad_value=pad, pad_value_f64=pad)
     return capi.conv2d_default_tile(cd)
 
 
@@ -358,14 +373,21 @@ def map_node(
     segment (nested splits of a segment's own root included)."""
     if sched is None or not sched.segments:
         return map_gemm(launch_attrs, conv, sched, policy)
-    pieces = _split_pieces(launch_attrs, conv, sched, policy, 0, 0)
+    M, N, K = launch_attrs["M"], launch_attrs["N"], launch_attrs["K"]
+    ta, tb = launch_attrs.get("trans_a"), launch_attrs.get("trans_b")
+    whole = {**launch_attrs, "lda": M if ta else K, "ldb": K if tb else N, "ldc": N}
+    pieces = _split_pieces(whole, conv, sched, policy, 0, 0)
     return SplitConfig(tuple(pieces))
 
 
 def _split_pieces(attrs: dict[str, Any], conv: bool, sched: HipNodeSchedule, policy: str, m0: int,
                   n0: int) -> list[SplitPiece]:
     if not sched.segments:
-        return [SplitPiece(m0, attrs["M"], n0, attrs["N"], map_gemm(attrs, conv, sched, policy))]
+        vec = {"float32": 4, "float64": 2}.get(attrs["dtype"], 8)
+        a0 = m0 if attrs.get("trans_a") else m0 * attrs["lda"]
+        b0 = n0 * attrs["ldb"] if attrs.get("trans_b") else n0
+        piece = {**attrs, "aligned": a0 % vec == 0 and b0 % vec == 0}
+        return [SplitPiece(m0, attrs["M"], n0, attrs["N"], map_gemm(piece, conv, sched, policy))]
     where = f"{sched.node_name}: split()"
     if conv:
         raise ScheduleError(f"{where} has no HIP mapping for conv2d (one launch covers the whole tensor)")

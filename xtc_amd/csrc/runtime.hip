@@ -13,6 +13,7 @@
 #include <string.h>
 #include <time.h>
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <string>
@@ -1139,18 +1140,13 @@ const PlanesEntry* planes_entry(int dtype, int conv, int bt, int vec, const xtc_
   return nullptr;
 }
 
-// The instance that runs tile t over whole 16-byte vectors, and how many
-// splits of K it runs.  fp32 has one instance a tile.  bf16:
+// The instance that runs tile t, split `split_k` ways, over whole 16-byte
+// vectors.  fp32 has one instance a tile.  bf16:
 //  * 128-row tiles whose workgroups fit the 256 CUs once: two k-groups of 8
-//    waves each share a workgroup and walk half of its K.  A CU holds as many
-//    waves as from two workgroups, and half the splits leave as many partial
-//    chains with half the partial sums in memory; no chain is longer than
-//    asked for.  (us; two k-groups at half the splits, or as many as fit,
-//    against 8 waves at all of them) 256x8192x4608 split 4 39.9 -> 34.5,
-//    256x4608x8192 split 4 51.9 -> 38.2 on 3, 128x4096x8192 split 16 33.2 ->
-//    26.9, 1280x2048x4096 split 2 47.9 -> 43.5, 1280x2048x8192 unsplit 93.8 ->
-//    79.8.  Below 8 slabs a workgroup the second group's sums cost what it
-//    saves (1024x1024x1024 split 4: 14.9 against 14.7).
+//    waves each share a workgroup and walk half of its K, so that a CU holds as
+//    many waves as from two workgroups (1280x2048x8192 unsplit 93.8 -> 79.8 us).
+//    Below 8 slabs a workgroup the second group's sums cost what it saves
+//    (1024x1024x1024 split 4: 14.9 us against 14.7).
 //  * 128-row tiles otherwise: 8 waves.  Four of 64x64 each leave a CU's
 //    matrix cores idle behind their LDS reads (2000x2304x2600 54.8 -> 51.1,
 //    17x17x1024 1x1 over 28272 57.9 -> 46.4).
@@ -1162,20 +1158,28 @@ const PlanesEntry* planes_entry(int dtype, int conv, int bt, int vec, const xtc_
 //    over 256 (292) 16.6 -> 17.0, 8x56x56x64 over 64 (392) 10.7 -> 10.9,
 //    17x17x512 over 1024 split 8 (640) 16.5 -> 16.8, 128x4096x8192 split 8
 //    (1024) 27.2 -> 28.3.
-struct PlanesPick {
-  const PlanesEntry* e;
-  int split_k;
-};
-PlanesPick planes_pick(int dtype, int conv, int bt, const xtc_hip_tile& t, int M, int N, int K, int split_k) {
-  if (dtype == XTC_HIP_F32) return {planes_entry(dtype, conv, bt, 1, t), split_k};
+bool planes_two_groups(const xtc_hip_tile& t, int64_t groups, int K, int split_k) {
+  return t.bm == 128 && groups <= 256 && split_depth(K, split_k, t.bk) / t.bk >= 8;
+}
+const PlanesEntry* planes_pick(int dtype, int conv, int bt, const xtc_hip_tile& t, int M, int N, int K, int split_k) {
+  if (dtype == XTC_HIP_F32) return planes_entry(dtype, conv, bt, 1, t);
+  const int64_t groups = launch_groups(M, N, K, split_k, t);
+  if (t.bm == 128) return planes_entry(dtype, conv, bt, 1, t, 8, planes_two_groups(t, groups, K, split_k) ? 2 : 1);
+  return planes_entry(dtype, conv, bt, 1, t, groups <= (conv ? 256 : 512) ? 8 : 4, 1);
+}
+
+// Splits of K that bf16 tile t runs by default where the shape class says
+// `split_k`: on 128-row tiles as many as fit the 256 CUs once, if those are at
+// least half and run on two k-groups.  They leave as many partial chains with
+// half the partial sums in memory; no chain is longer (us; two k-groups at half
+// the splits, or as many as fit, against 8 waves at all of them) 256x8192x4608
+// split 4 39.9 -> 34.5, 256x4608x8192 split 4 51.9 -> 38.2 on 3, 128x4096x8192
+// split 16 33.2 -> 26.9, 1280x2048x4096 split 2 47.9 -> 43.5.
+int planes_default_split(const xtc_hip_tile& t, int M, int N, int K, int split_k) {
   const int splits = effective_splits(K, split_k, t.bk);
   const int64_t tiles = launch_groups(M, N, K, 1, t);
-  if (t.bm == 128) {
-    const int fit = (int)std::min<int64_t>(splits, 256 / tiles);
-    const bool two = fit > 0 && 2 * fit >= splits && split_depth(K, fit, t.bk) / t.bk >= 8;
-    return {planes_entry(dtype, conv, bt, 1, t, 8, two ? 2 : 1), two ? fit : split_k};
-  }
-  return {planes_entry(dtype, conv, bt, 1, t, tiles * splits <= (conv ? 256 : 512) ? 8 : 4, 1), split_k};
+  const int fit = (int)std::min<int64_t>(splits, 256 / tiles);
+  return fit > 0 && 2 * fit >= splits && planes_two_groups(t, tiles * fit, K, fit) ? fit : split_k;
 }
 
 bool generic_only() {
@@ -1234,11 +1238,11 @@ bool planes_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, in
 //    for matmuls: 272x272x32 over 64 44.0 -> 35.6, 34x34x256 over 512 split 4
 //    55.7 -> 41.3; but 14x14x256 over 256 split 16 15.9 -> 16.6, 4x56x56x64
 //    over 256 1x1 (2 slabs) 12.8 -> 13.9.
-PlanesPick planes_conv_pick(const xtc_hip_conv2d_desc& d, const xtc_hip_tile& t, int split_k, int M, int K) {
+const PlanesEntry* planes_conv_pick(const xtc_hip_conv2d_desc& d, const xtc_hip_tile& t, int split_k, int M, int K) {
   const bool applies = d.dtype == XTC_HIP_BF16
                            ? t.bk == 64
                            : launch_groups(M, d.F, K, split_k, t) >= 512 && split_depth(K, split_k, t.bk) >= 256;
-  if (!applies || generic_only() || !planes_offsets_fit(4, 1, d.F) || !planes_entry(d.dtype, 1, 0, 1, t)) return {nullptr, split_k};
+  if (!applies || generic_only() || !planes_offsets_fit(4, 1, d.F) || !planes_entry(d.dtype, 1, 0, 1, t)) return nullptr;
   return planes_pick(d.dtype, 1, 0, t, M, d.F, K, split_k);
 }
 
@@ -1253,9 +1257,9 @@ xtc_hip_tile planes_conv_any_tile(int dtype, int M, int N, int splits) {
   return {64, 64, 32, 2, 2};
 }
 
-// The gemm_planes tile and split that run an fp32 matmul of whole vectors named
-// with the 64x64x32 or 128x128x32 tile of 2x2 waves at the default depth, when
-// one of the 8-wave tiles is estimated to take less time (us; a workgroup of
+// The 8-wave gemm_planes tile and split that an fp32 matmul of whole vectors
+// gets by default where its shape class says the 64x64x32 or 128x128x32 tile of
+// 2x2 waves, if one of them is estimated to take less time (us; a workgroup of
 // those has a CU to itself):
 //   8 waves  rounds of 256 workgroups * (9 + slabs * 1.4 (128x128) or 2.3
 //            (256 wide), a third more with column tiles cut by N)
@@ -1263,27 +1267,24 @@ xtc_hip_tile planes_conv_any_tile(int dtype, int M, int N, int splits) {
 //   64x64    rounds of 256 * slabs * 0.55 (0.85 on the generic template) + 6
 //            (16 where gemm_planes splits K)
 // which follow the measured times of 20 shapes x 40 launches to 15 %.  The
-// generic 128x128 tile is never better.  K is split at most as often as asked
-// for, so the scratch holds the partials (us, before -> now): 3000^3 727 ->
+// generic 128x128 tile is never better.  K is split at most as often as the
+// class says, or as the descriptor does (us, before -> now): 3000^3 727 ->
 // 446, 2048x2048x1024 89.7 -> 54.2, 256x4608x8192 153 -> 117, 768x768x4096
 // 58.4 -> 44.8, 1280x4096x2048 159 -> 145, 1000x1104x1200 44.3 -> 34.5,
 // 2000x2304x2600 187 -> 182.
-struct WidePick {
-  const PlanesEntry* e;
-  int split_k;
-};
-WidePick planes_wide_pick(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_k, int lda, int ldb, bool bt,
-                          bool on_planes) {
-  const bool small = t.bm == 64 && t.bn == 64;
-  if (generic_only() || d.dtype != XTC_HIP_F32 || d.stages != 0 || t.bk != 32 || t.wgm != 2 || t.wgn != 2 ||
-      !(small || (t.bm == 128 && t.bn == 128)) || !planes_offsets_fit(4, lda, ldb))
-    return {nullptr, split_k};
-  const int asked = effective_splits(d.K, split_k, t.bk);
-  WidePick best{nullptr, split_k};
+bool planes_wide_tile(const xtc_hip_matmul_desc& d, int lda, int ldb, bool bt, bool on_planes, xtc_hip_tile* t,
+                      int* split_k) {
+  const bool small = t->bm == 64 && t->bn == 64;
+  if (generic_only() || d.dtype != XTC_HIP_F32 || t->bk != 32 || t->wgm != 2 || t->wgn != 2 ||
+      !(small || (t->bm == 128 && t->bn == 128)) || !planes_offsets_fit(4, lda, ldb))
+    return false;
+  const int asked = effective_splits(d.K, *split_k, t->bk);
+  xtc_hip_tile best{0, 0, 0, 0, 0};
+  int best_split = asked;
   double least = 1e30;
   if (small) {
-    const int64_t rounds = (launch_groups(d.M, d.N, d.K, split_k, t) + 255) / 256;
-    const int slabs = split_depth(d.K, split_k, 32) / 32;
+    const int64_t rounds = (launch_groups(d.M, d.N, d.K, *split_k, *t) + 255) / 256;
+    const int slabs = split_depth(d.K, *split_k, 32) / 32;
     // 12 % off: near ties stay (3072x1408x2432 166 -> 179, 1449x3416x140 24.2
     // -> 25.1 at 8 %)
     least = 0.88 * (rounds * slabs * (on_planes ? 0.55 : 0.85) + (on_planes && asked > 1 ? 16 : 6));
@@ -1291,18 +1292,22 @@ WidePick planes_wide_pick(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, i
   const xtc_hip_tile wide[] = {{256, 128, 32, 4, 2}, {128, 256, 32, 2, 4}, {128, 128, 32, 2, 4}};
   for (const xtc_hip_tile& w : wide) {
     const double slab = (w.bm == w.bn ? 1.4 : 2.3) * (d.N % w.bn && !bt ? 1.3 : 1.0);
-    for (int want = 1; want <= std::min(asked, 16); ++want) {
+    for (int want = d.split_k > 0 ? asked : 1; want <= std::min(asked, 16); ++want) {
       const int s = effective_splits(d.K, want, 32), slabs = split_depth(d.K, want, 32) / 32;
       if (s != want || (s > 1 && slabs < 4)) continue;
       const int64_t rounds = (launch_groups(d.M, d.N, d.K, s, w) + 255) / 256;
       const double us = rounds * (9 + slabs * slab) + (s > 1 ? 0.93 * s * (w.bm * w.bn / 16384) : 0.0);
       if (us < least) {
         least = us;
-        best = {planes_entry(d.dtype, 0, bt, 1, w), s};
+        best = w;
+        best_split = s;
       }
     }
   }
-  return best;
+  if (!best.bm) return false;
+  *t = best;
+  *split_k = best_split;
+  return true;
 }
 
 bool splitwave_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_k, int lda, const void* A);
@@ -1579,8 +1584,8 @@ int launch_direct_conv(const xtc_hip_conv2d_desc& d, const xtc_hip_tile& t, int 
   return 0;
 }
 
-// The tile a conv2d descriptor gets when it leaves `tile` zeroed: the shape
-// class default of default_tile, upgraded from the 8x8 direct conv block to
+// The tile of a conv2d of whole vectors: the shape class default of
+// default_tile, upgraded from the 8x8 direct conv block to
 // a 1x4-wave one when the direct kernel takes the shape with it, the window
 // is wider than 1x1 (the wider block shares more of the input halo) and its
 // blocks fit in one wave over the chip's 256 CUs: 7x14 (6.125 tiles of MFMA
@@ -1590,7 +1595,7 @@ int launch_direct_conv(const xtc_hip_conv2d_desc& d, const xtc_hip_tile& t, int 
 // (68x68, 3x3, 180 blocks) 47.6 -> 41.3 us from 8x8 to 8x14; but
 // Yolo9000_04 (340 blocks) 39.8 -> 41.4 us, and the 1x1 convs lose
 // (Yolo9000_09 10.6 -> 15.6 us, ResNet18_03 5.0 -> 6.8).
-void default_conv_tile(const xtc_hip_conv2d_desc& d, int OH, int OW, xtc_hip_tile* t, int* split_k) {
+void conv_class_tile(const xtc_hip_conv2d_desc& d, int OH, int OW, xtc_hip_tile* t, int* split_k) {
   default_tile(d.dtype, 1, d.N * OH * OW, d.F, d.R * d.S * d.C, t, split_k);
   if (d.R * d.S == 1 || !same_tile(*t, xtc_hip_tile{64, 64, 16, 2, 2})) return;
   const void* p = (const void*)(uintptr_t)256;
@@ -1604,6 +1609,52 @@ void default_conv_tile(const xtc_hip_conv2d_desc& d, int OH, int OW, xtc_hip_til
       return;
     }
   }
+}
+
+int conv_vec(const xtc_hip_conv2d_desc& d) { return d.dtype == XTC_HIP_F32 ? 4 : d.dtype == XTC_HIP_F64 ? 2 : 8; }
+
+// Whether d's operands can be copied to whole vectors of channels: a zero
+// channel times a finite pad value adds exact zeros.
+bool conv_can_stage(const xtc_hip_conv2d_desc& d) {
+  const bool padded = d.pad_top || d.pad_bottom || d.pad_left || d.pad_right;
+  return d.F % conv_vec(d) == 0 &&
+         (!padded || isfinite(d.dtype == XTC_HIP_F64 ? d.pad_value_f64 : (double)d.pad_value));
+}
+
+// Whether gemm_planes gathers the windows of d, whose channels or filters are
+// not whole 16-byte vectors or whose operands are not 16-byte aligned, element
+// by element, and in how many splits of K (those of the copied conv).  fp32
+// always; bf16, whose products are cheaper beside the gather, below 16 channels
+// (56x56x50 3x3 over 64: 20.3 us gathered, 18.9 copied to whole vectors first)
+// and where the copy cannot be made.
+bool conv_gathers(const xtc_hip_conv2d_desc& d, int OH, int OW, int* split_k) {
+  if (d.dtype == XTC_HIP_F64 || generic_only() || !planes_offsets_fit(4, 1, d.F)) return false;
+  const bool can_stage = conv_can_stage(d);
+  xtc_hip_conv2d_desc dc = d;  // the tile, split and refusals of the copied conv
+  if (can_stage) dc.C = (d.C + conv_vec(d) - 1) / conv_vec(d) * conv_vec(d);
+  xtc_hip_tile t = d.tile;
+  *split_k = d.split_k;
+  if (t.bm == 0) {
+    int sk = 1;
+    conv_class_tile(dc, OH, OW, &t, &sk);
+    if (*split_k <= 0) *split_k = sk;
+  }
+  if (!can_stage) return !short_sums(d.dtype, (int64_t)d.N * OH * OW, d.F, d.R * d.S * d.C);
+  const GemmEntry* e = find_entry(d.dtype, 1, t);
+  const void* p = (const void*)(uintptr_t)256;
+  return e && e->launch && (d.dtype == XTC_HIP_F32 || d.C < 16) && !direct_conv_applies(dc, t, *split_k, OH, OW, p, p, p, nullptr);
+}
+
+// The tile and split of a conv2d descriptor that leaves `tile` zeroed: those
+// of its class, with the split fitted to the chip in bf16.
+void default_conv_tile(const xtc_hip_conv2d_desc& d, int OH, int OW, xtc_hip_tile* t, int* split_k) {
+  conv_class_tile(d, OH, OW, t, split_k);
+  int gathered;
+  if (d.dtype != XTC_HIP_BF16 || ((d.C % 8 || d.F % 8) && conv_gathers(d, OH, OW, &gathered))) return;
+  // channels as they are staged
+  const int M = d.N * OH * OW, K = d.R * d.S * ((d.C + 7) / 8 * 8);
+  if (d.F % 8 == 0 && planes_conv_pick(d, *t, *split_k, M, K))
+    *split_k = planes_default_split(*t, M, d.F, K, *split_k);
 }
 
 int launch_lds_dma_gemm(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_k, int stages, int lda,
@@ -1893,14 +1944,19 @@ int path_depths(MatmulPath p, const xtc_hip_tile& t, int ring, int* out, int max
   return n;
 }
 
+bool has_depth(MatmulPath p, const xtc_hip_tile& t, int ring, int stages) {
+  int depths[16];
+  const int n = path_depths(p, t, ring, depths, 16);
+  return std::find(depths, depths + n, stages) != depths + n;
+}
+
 // 0 if `stages` (0 = default) is a depth of path p for tile t, else fails.
 int check_depth(MatmulPath p, const xtc_hip_tile& t, int ring, int stages) {
-  if (stages == 0) return 0;
+  if (stages == 0 || has_depth(p, t, ring, stages)) return 0;
   int depths[16];
   const int n = path_depths(p, t, ring, depths, 16);
   char list[96] = "";
   for (int i = 0; i < n; ++i) {
-    if (depths[i] == stages) return 0;
     const size_t used = strlen(list);
     snprintf(list + used, sizeof(list) - used, i ? ", %d" : "%d", depths[i]);
   }
@@ -1908,9 +1964,68 @@ int check_depth(MatmulPath p, const xtc_hip_tile& t, int ring, int stages) {
               t.bn, t.bk, t.wgm, t.wgn, list, stages);
 }
 
+int natural_path(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_k, int lda, int ldb, int ldc,
+                 const void* A, const void* B, const void* C, const void* bias, MatmulPath* path);
+
+// The path of a matmul on the operands as they are stored, and whether
+// gemm_planes reads B^T in place: a transposed operand that no kernel reads in
+// place becomes a dense, aligned copy first.
+int stored_path(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int split_k, int lda, int ldb, int ldc,
+                const void* A, const void* B, const void* C, const void* bias, MatmulPath* path, bool* bt) {
+  const void* const copy = (const void*)(uintptr_t)256;
+  *bt = false;
+  if (d.trans_b && !d.trans_a) {
+    if (lds_dma_gemm_applies(d, t, split_k, lda, ldb, ldc, A, B, (const float*)C, (const float*)bias, true)) {
+      *path = MatmulPath::LdsDmaBt;
+      return 0;
+    }
+    if (planes_bt_applies(d, t, split_k, lda, ldb, A, B)) {
+      *bt = true;
+      *path = MatmulPath::Planes;
+      return 0;
+    }
+  }
+  if (d.trans_a) {
+    lda = d.K;
+    A = copy;
+  }
+  if (d.trans_b) {
+    ldb = d.N;
+    B = copy;
+  }
+  return natural_path(d, t, split_k, lda, ldb, ldc, A, B, C, bias, path);
+}
+
+// The tile and split of a descriptor that leaves the tile zeroed: the shape
+// class default of default_tile, with its split fitted to the chip in bf16 and
+// upgraded in fp32 to an 8-wave tile where gemm_planes runs the call.  A named
+// depth stays one that the tile has.
+int default_matmul_tile(const xtc_hip_matmul_desc& d, int lda, int ldb, int ldc, const void* A, const void* B,
+                        const void* C, const void* bias, xtc_hip_tile* t, int* split_k) {
+  int sk = 1;
+  default_tile(d.dtype, 0, d.M, d.N, d.K, t, &sk);
+  *split_k = d.split_k > 0 ? d.split_k : sk;
+  MatmulPath path;
+  bool bt;
+  if (stored_path(d, *t, *split_k, lda, ldb, ldc, A, B, C, bias, &path, &bt)) return 1;
+  if (path != MatmulPath::Planes && path != MatmulPath::Generic) return 0;
+  if (path == MatmulPath::Planes && d.dtype == XTC_HIP_BF16 && d.split_k <= 0)
+    *split_k = planes_default_split(*t, d.M, d.N, d.K, *split_k);
+  xtc_hip_tile wide = *t;
+  int wide_split = *split_k;
+  if (!planes_wide_tile(d, d.trans_a ? d.K : lda, d.trans_b && !bt ? d.N : ldb, bt, path == MatmulPath::Planes, &wide,
+                        &wide_split) ||
+      (d.stages && !has_depth(MatmulPath::Planes, wide, 0, d.stages)))
+    return 0;
+  *t = wide;
+  *split_k = wide_split;
+  return 0;
+}
+
 // Strides, tile and split of descriptor d after defaults.  Returns 0, or
 // fails.
-int resolve_matmul(const xtc_hip_matmul_desc& d, int* lda, int* ldb, int* ldc, xtc_hip_tile* t, int* split_k) {
+int resolve_matmul(const xtc_hip_matmul_desc& d, const void* A, const void* B, const void* C, const void* bias, int* lda,
+                   int* ldb, int* ldc, xtc_hip_tile* t, int* split_k) {
   if (d.dtype != XTC_HIP_F32 && d.dtype != XTC_HIP_BF16 && d.dtype != XTC_HIP_F64) return fail("bad dtype %d", d.dtype);
   if (d.M <= 0 || d.N <= 0 || d.K <= 0) return fail("bad shape %dx%dx%d", d.M, d.N, d.K);
   if (d.stages < 0) return fail("bad pipeline depth %d", d.stages);
@@ -1922,12 +2037,7 @@ int resolve_matmul(const xtc_hip_matmul_desc& d, int* lda, int* ldb, int* ldc, x
     return fail("leading dimension smaller than shape");
   *t = d.tile;
   *split_k = d.split_k;
-  if (t->bm == 0) {
-    int sk = 1;
-    default_tile(d.dtype, 0, d.M, d.N, d.K, t, &sk);
-    if (*split_k <= 0) *split_k = sk;
-  }
-  return 0;
+  return t->bm == 0 ? default_matmul_tile(d, *lda, *ldb, *ldc, A, B, C, bias, t, split_k) : 0;
 }
 
 // The path of a matmul whose operands, after any transposed copy, are A/B
@@ -2033,7 +2143,7 @@ int matmul_impl(const xtc_hip_matmul_desc& d, const void* A, const void* B, void
   if (!A || !B || !C) return fail("null operand");
   int lda, ldb, ldc, split_k;
   xtc_hip_tile t;
-  if (resolve_matmul(d, &lda, &ldb, &ldc, &t, &split_k)) return 1;
+  if (resolve_matmul(d, A, B, C, biasv, &lda, &ldb, &ldc, &t, &split_k)) return 1;
   const bool ta = d.trans_a != 0, tb = d.trans_b != 0;
   const hipStream_t s = x.s;
   // B stored transposed feeds the LDS-DMA kernel and gemm_planes directly
@@ -2093,26 +2203,15 @@ int matmul_impl(const xtc_hip_matmul_desc& d, const void* A, const void* B, void
     split_k = splits_with_room(split_k, d.M, d.N, d.K, u, x);
   } else if (path == MatmulPath::F32Lds || path == MatmulPath::Planes) {
     // same tiles, split-K set-up and grid as the generic instance; only the
-    // kernel and, in bf16, the number of splits differ
+    // kernel differs
     own = *e;
     if (path == MatmulPath::F32Lds) {
       own.launch = f32_lds_variant(t, d.stages)->launch;
     } else {
-      const PlanesPick p = planes_pick(d.dtype, 0, bt, t, d.M, d.N, d.K, split_k);
-      own.launch = p.e->launch;
-      split_k = p.split_k;
+      own.launch = planes_pick(d.dtype, 0, bt, t, d.M, d.N, d.K, split_k)->launch;
     }
     own.launch_ring = nullptr;
     e = &own;
-  }
-  bool planes = path == MatmulPath::Planes || path == MatmulPath::PlanesAny;
-  if (path == MatmulPath::Planes || path == MatmulPath::Generic) {
-    if (const WidePick w = planes_wide_pick(d, t, split_k, lda, ldb, bt, planes); w.e) {
-      own = GemmEntry{d.dtype, 0, w.e->bm, w.e->bn, 32, w.e->wgm, w.e->wgn, 0, 0, w.e->launch, nullptr};
-      e = &own;
-      split_k = w.split_k;
-      planes = true;
-    }
   }
   GemmArgs a;
   memset(&a, 0, sizeof(a));
@@ -2128,7 +2227,7 @@ int matmul_impl(const xtc_hip_matmul_desc& d, const void* A, const void* B, void
   a.ldc = ldc;
   a.relu = d.relu;
   a.relu_threshold = d.relu_threshold;
-  if (planes) a.ldp = planes_ldp(d.N);
+  if (path == MatmulPath::Planes || path == MatmulPath::PlanesAny) a.ldp = planes_ldp(d.N);
   return launch_gemm_common(a, e, split_k, path == MatmulPath::Generic ? d.stages : 0, d.group_m, d.xcd_remap, x);
 }
 
@@ -2422,6 +2521,15 @@ int xtc_hip_default_tile(int dtype, int conv, int M, int N, int K, xtc_hip_tile*
   return 0;
 }
 
+int xtc_hip_matmul_default_tile(const xtc_hip_matmul_desc* desc, xtc_hip_tile* out, int* split_k) {
+  if (!desc || !out || !split_k) return fail("null argument");
+  xtc_hip_matmul_desc d = *desc;
+  d.tile = xtc_hip_tile{0, 0, 0, 0, 0};
+  const void* p = (const void*)(uintptr_t)256;
+  int lda, ldb, ldc;
+  return resolve_matmul(d, p, p, p, nullptr, &lda, &ldb, &ldc, out, split_k);
+}
+
 int xtc_hip_conv2d_default_tile(const xtc_hip_conv2d_desc* desc, xtc_hip_tile* out, int* split_k) {
   if (!desc || !out || !split_k) return fail("null argument");
   const xtc_hip_conv2d_desc& d = *desc;
@@ -2438,19 +2546,12 @@ int xtc_hip_matmul_pipeline_depths(const xtc_hip_matmul_desc* desc, int* depths,
   const xtc_hip_matmul_desc& d = *desc;
   int lda, ldb, ldc, split_k;
   xtc_hip_tile t;
-  if (resolve_matmul(d, &lda, &ldb, &ldc, &t, &split_k)) return -1;
   // operands as the allocators hand them out: 256-byte aligned
   const void* p = (const void*)(uintptr_t)256;
+  if (resolve_matmul(d, p, p, p, nullptr, &lda, &ldb, &ldc, &t, &split_k)) return -1;
   MatmulPath path;
-  if (d.trans_b && !d.trans_a && lds_dma_gemm_applies(d, t, split_k, lda, ldb, ldc, p, p, p, nullptr, true)) {
-    path = MatmulPath::LdsDmaBt;
-  } else if (d.trans_b && !d.trans_a && planes_bt_applies(d, t, split_k, lda, ldb, p, p)) {
-    path = MatmulPath::Planes;
-  } else {
-    if (d.trans_a) lda = d.K;
-    if (d.trans_b) ldb = d.N;
-    if (natural_path(d, t, split_k, lda, ldb, ldc, p, p, p, nullptr, &path)) return -1;
-  }
+  bool bt;
+  if (stored_path(d, t, split_k, lda, ldb, ldc, p, p, p, nullptr, &path, &bt)) return -1;
   const int ring = path == MatmulPath::Generic || path == MatmulPath::Planes
                        ? generic_ring(find_entry(d.dtype, 0, t), effective_splits(d.K, split_k, t.bk))
                        : 0;
@@ -2465,10 +2566,8 @@ int xtc_hip_conv2d_pipeline_depths(const xtc_hip_conv2d_desc* desc, int* depths,
   if (d.stride_h <= 0 || d.stride_w <= 0 || HP < d.R || WP < d.S) return -fail("bad conv2d descriptor");
   const int OH = (HP - d.R) / d.stride_h + 1;
   const int OW = (WP - d.S) / d.stride_w + 1;
-  const int vec = d.dtype == XTC_HIP_F32 ? 4 : d.dtype == XTC_HIP_F64 ? 2 : 8;
-  const bool padded = d.pad_top || d.pad_bottom || d.pad_left || d.pad_right;
-  const double pad_value = d.dtype == XTC_HIP_F64 ? d.pad_value_f64 : (double)d.pad_value;
-  if (d.C % vec && d.F % vec == 0 && (!padded || isfinite(pad_value))) {
+  const int vec = conv_vec(d);
+  if (d.C % vec && conv_can_stage(d)) {
     // xtc_hip_conv2d stages such a conv with zero channels up to the next
     // whole vector and runs the MFMA conv on the copies: describe that kernel
     d.C = (d.C + vec - 1) / vec * vec;
@@ -2548,44 +2647,22 @@ int xtc_hip_conv2d(const xtc_hip_conv2d_desc* desc, const void* input, const voi
   const int OH = (HP - d.R) / d.stride_h + 1;
   const int OW = (WP - d.S) / d.stride_w + 1;
   hipStream_t s = pick_stream(d.stream);
-  const int vec = d.dtype == XTC_HIP_F32 ? 4 : f64 ? 2 : 8;
+  const int vec = conv_vec(d);
   const int M = d.N * OH * OW;
   const int K = d.R * d.S * d.C;
   const bool vec_ok = d.C % vec == 0 && d.F % vec == 0 && aligned16(input) && aligned16(weight);
-  const bool padded = d.pad_top || d.pad_bottom || d.pad_left || d.pad_right;
-  const bool can_stage = d.F % vec == 0 && (!padded || isfinite(f64 ? d.pad_value_f64 : (double)d.pad_value));
-  if (!vec_ok && !f64 && !generic_only() && planes_offsets_fit(4, 1, d.F)) {
-    // Channels or filters that are not whole 16-byte vectors, or operands not
-    // 16-byte aligned: gemm_planes gathers the window element by element.
-    // fp32 always; bf16, whose products are cheaper beside the gather, below
-    // 16 channels (56x56x50 3x3 over 64: 20.3 us gathered, 18.9 copied to
-    // whole vectors first) and where the copy cannot be made.
-    xtc_hip_conv2d_desc dc = d;  // the tile, split and refusals of the copied conv
-    if (can_stage) dc.C = (d.C + vec - 1) / vec * vec;
-    xtc_hip_tile t = d.tile;
-    int split_k = d.split_k;
-    if (t.bm == 0) {
-      int sk = 1;
-      default_conv_tile(dc, OH, OW, &t, &sk);
-      if (split_k <= 0) split_k = sk;
-    }
-    const GemmEntry* e = can_stage ? find_entry(d.dtype, 1, t) : nullptr;
-    const void* p = (const void*)(uintptr_t)256;
-    const bool gather = (!can_stage && !short_sums(d.dtype, M, d.F, K)) || (e && e->launch && (d.dtype == XTC_HIP_F32 || d.C < 16) &&
-                                       !direct_conv_applies(dc, t, split_k, OH, OW, p, p, p, nullptr));
-    if (gather) {
-      Scratch x{s};
-      xtc_hip_tile u = planes_conv_any_tile(d.dtype, M, d.F, 1);
-      split_k = splits_with_room(split_k < 1 ? 1 : split_k, M, d.F, K, u, x);
-      u = planes_conv_any_tile(d.dtype, M, d.F, effective_splits(K, split_k, u.bk));
-      const GemmEntry own{d.dtype, 1, u.bm, u.bn, u.bk, u.wgm, u.wgn, 0, 0, planes_entry(d.dtype, 1, 0, 0, u)->launch,
-                          nullptr};
-      GemmArgs a = conv_args(d, OH, OW, input, weight, out, bias);
-      a.ldp = planes_ldp(d.F);
-      return launch_gemm_common(a, &own, split_k, 0, d.group_m, d.xcd_remap, x);
-    }
+  if (int split_k; !vec_ok && conv_gathers(d, OH, OW, &split_k)) {
+    Scratch x{s};
+    xtc_hip_tile u = planes_conv_any_tile(d.dtype, M, d.F, 1);
+    split_k = splits_with_room(split_k < 1 ? 1 : split_k, M, d.F, K, u, x);
+    u = planes_conv_any_tile(d.dtype, M, d.F, effective_splits(K, split_k, u.bk));
+    const GemmEntry own{d.dtype, 1, u.bm, u.bn, u.bk, u.wgm, u.wgn, 0, 0, planes_entry(d.dtype, 1, 0, 0, u)->launch,
+                        nullptr};
+    GemmArgs a = conv_args(d, OH, OW, input, weight, out, bias);
+    a.ldp = planes_ldp(d.F);
+    return launch_gemm_common(a, &own, split_k, 0, d.group_m, d.xcd_remap, x);
   }
-  if (!vec_ok && can_stage) {
+  if (!vec_ok && conv_can_stage(d)) {
     // Channels that are not whole 16-byte vectors (C = 3 image inputs): the
     // input and the weights are copied with zero channels up to Cp, a
     // multiple of the vector, and the MFMA conv runs on the copies.  A zero
@@ -2691,11 +2768,10 @@ int xtc_hip_conv2d(const xtc_hip_conv2d_desc* desc, const void* input, const voi
   GemmArgs a = conv_args(d, OH, OW, input, weight, out, bias);
   Scratch x{s};
   GemmEntry own;
-  if (const PlanesPick p = planes_conv_pick(d, t, split_k, M, K); p.e) {
+  if (const PlanesEntry* p = planes_conv_pick(d, t, split_k, M, K)) {
     own = *e;
-    own.launch = p.e->launch;
+    own.launch = p->launch;
     own.launch_ring = nullptr;
-    split_k = p.split_k;
     a.ldp = planes_ldp(d.F);
     e = &own;
   }

@@ -198,6 +198,7 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
         _i,
         [_i, _i, _i, _i, _i, ctypes.POINTER(Tile), ctypes.POINTER(_i)],
     ),
+    "xtc_hip_matmul_default_tile": (_i, [ctypes.POINTER(MatmulDesc), ctypes.POINTER(Tile), ctypes.POINTER(_i)]),
     "xtc_hip_conv2d_default_tile": (_i, [ctypes.POINTER(Conv2dDesc), ctypes.POINTER(Tile), ctypes.POINTER(_i)]),
     "xtc_hip_matmul_pipeline_depths": (_i, [ctypes.POINTER(MatmulDesc), ctypes.POINTER(_i), _i]),
     "xtc_hip_conv2d_pipeline_depths": (_i, [ctypes.POINTER(Conv2dDesc), ctypes.POINTER(_i), _i]),
@@ -296,7 +297,7 @@ DTYPE_NAMES = {v: k for k, v in _DTYPE_IDS.items()}
 
 
 def default_tile(dtype: str, conv: bool, M: int, N: int, K: int) -> tuple[tuple[int, int, int, int, int], int]:
-    """(tile, split_k) the library picks for a shape when none is given."""
+    """(tile, split_k) of a shape's class (xtc_hip_default_tile)."""
     t = Tile()
     sk = ctypes.c_int(1)
     check(lib().xtc_hip_default_tile(_DTYPE_IDS[dtype], int(conv), M, N, K, ctypes.byref(t), ctypes.byref(sk)), "default_tile")
@@ -319,6 +320,14 @@ def conv2d_pipeline_depths(desc: Conv2dDesc) -> list[int]:
     if n < 0:
         raise HipError(f"conv2d_pipeline_depths: {last_error()}")
     return list(out[: min(n, 16)])
+
+
+def matmul_default_tile(desc: MatmulDesc) -> tuple[tuple[int, int, int, int, int], int]:
+    """(tile, split_k) a matmul descriptor gets when it leaves the tile zeroed."""
+    t = Tile()
+    sk = ctypes.c_int(1)
+    check(lib().xtc_hip_matmul_default_tile(ctypes.byref(desc), ctypes.byref(t), ctypes.byref(sk)), "matmul_default_tile")
+    return t.as_tuple(), int(sk.value)
 
 
 def conv2d_default_tile(desc: Conv2dDesc) -> tuple[tuple[int, int, int, int, int], int]:

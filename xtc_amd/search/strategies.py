@@ -613,7 +613,6 @@ class Strategy_HIP(BaseStrategy):
                             if s == 1 or (self._K % s == 0 and 64 <= self._K // s <= self._C)]
         else:
             self._splits = [s for s in splits if s == 1 or (self._K % s == 0 and self._K // s >= 64)]
-        self._dtype = dtype
 
     @staticmethod
     def _launch_attrs(graph: Any, node: str) -> dict[str, Any]:
@@ -698,14 +697,9 @@ class Strategy_HIP(BaseStrategy):
             sch.unroll({slab_loop: depth})  # `depth` slabs in flight through LDS
 
     def _default_schedule(self, opt_level: int) -> list[int]:
-        from ..runtimes.hip import capi
+        from ..backends.hip.mapping import default_conv_tile, default_matmul_tile
 
-        if self._conv:
-            from ..backends.hip.mapping import default_conv_tile
-
-            tile, split = default_conv_tile(self._attrs)
-        else:
-            tile, split = capi.default_tile(self._dtype, self._conv, self._M, self._N, self._K)
+        tile, split = default_conv_tile(self._attrs) if self._conv else default_matmul_tile(self._attrs)
         bm, bn, bk, wgm, wgn = tile
         split = max(1, split)
         if split not in self._splits:
