@@ -51,9 +51,9 @@ def matmul(dtype, M, N, K, tile=None, split=0, fn="xtc_hip_matmul", a=256, b=256
     rc = getattr(L, fn)(ctypes.byref(d), p(a), p(b), p(256), None)
     return capi.last_error() if rc else launched()
 
-def conv(dtype, n, h, w, c, f, r, s, stride=1, pad=0, tile=None, split=0):
+def conv(dtype, n, h, w, c, f, r, s, stride=1, pad=0, tile=None, split=0, pad_value=0.0):
     d = capi.Conv2dDesc(dtype=capi.DTYPE_IDS[dtype], N=n, H=h, W=w, C=c, F=f, R=r, S=s, stride_h=stride,
-                        stride_w=stride, pad_top=pad, pad_bottom=pad, pad_left=pad, pad_right=pad, split_k=split)
+                        stride_w=stride, pad_top=pad, pad_bottom=pad, pad_left=pad, pad_right=pad, split_k=split, pad_value=pad_value)
     if tile:
         d.tile = capi.Tile(*tile)
     p = ctypes.c_void_p
@@ -166,6 +166,41 @@ def test_named_convs_run_their_split(run, tile, split, shape):
     n, h, w, c, f, r = shape
     (rows,) = run(f"out.append(conv('bfloat16', {n}, {h}, {w}, {c}, {f}, {r}, {r}, pad=1, tile={tile}, split={split}))")
     assert rows[-1][0].startswith(f"gemm_planes<__bf16, {tile[0]}, {tile[1]}, 64,") and rows[-1][1] == split
+
+
+@pytest.mark.parametrize("dtype,tile,pad_value,launches", [
+    # by default and on the gather's own tiles in place, else on whole-vector copies
+    ("float32", None, 0.0, ["gemm_planes<float, 128, 64, 32, 4, 2, true, false, false, 1, 1>"]),
+    ("float32", (128, 64, 32, 4, 2), 0.0, ["gemm_planes<float, 128, 64, 32, 4, 2, true, false, false, 1, 1>"]),
+    ("float32", (64, 64, 32, 2, 2), 0.0, ["gemm_planes<float, 64, 64, 32, 2, 2, true, false, false, 1, 1>"]),
+    ("float32", (64, 64, 16, 2, 2), 0.0, ["pad_channels_kernel<float>"] * 2 + ["gemm_kernel<float, 64, 64, 16, 2, 2, true, 1>"]),
+    ("float32", (128, 64, 32, 2, 2), 0.0, ["pad_channels_kernel<float>"] * 2 + ["gemm_kernel<float, 128, 64, 32, 2, 2, true, 1>"]),
+    ("bfloat16", None, 0.0, ["gemm_planes<__bf16, 64, 64, 64, 2, 2, true, false, false, 1, 1>"]),
+    ("bfloat16", (32, 64, 32, 1, 2), 0.0, ["pad_channels_kernel<unsigned short>"] * 2 + ["gemm_kernel<__bf16, 32, 64, 32, 1, 2, true, 1>"]),
+    # an infinite pad value cannot be copied beside zero channels: any tile is gathered
+    ("float32", (32, 32, 16, 1, 1), float("inf"), ["gemm_planes<float, 128, 64, 32, 4, 2, true, false, false, 1, 1>"]),
+])
+def test_named_convs_without_whole_vectors_run_their_tile(run, dtype, tile, pad_value, launches):
+    pad_value = f"float('{pad_value}')"
+    (rows,) = run(f"out.append(conv({dtype!r}, 4, 224, 224, 3, 64, 7, 7, stride=2, pad=3, tile={tile}, split=1, "
+                  f"pad_value={pad_value}))")
+    assert [r[0] for r in rows] == launches
+
+
+def test_default_conv_sample_of_the_explorer_maps_on_the_gather():
+    import xtc_amd.graphs.xtc.op as O
+    from xtc_amd.backends.hip import Backend
+    from xtc_amd.search.strategies import Strategies
+
+    x, w = O.tensor((4, 224, 224, 3), "float32", name="I"), O.tensor((7, 7, 3, 64), "float32", name="W")
+    with O.graph(name="stem") as gb:
+        O.conv2d(x, w, stride=(2, 2), name="C")
+    backend, strategy = Backend(gb.graph), Strategies.create("tile_hip", gb.graph)
+    sch = backend.get_scheduler()
+    strategy.generate(sch, strategy.default_schedule())
+    compiler = backend.get_compiler(schedule_policy="strict")
+    tiles = [compiler.kernel_configs(s.schedule())["C"].tile for s in (sch, backend.get_scheduler())]
+    assert tiles == [(128, 64, 32, 4, 2)] * 2
 
 
 def test_default_queries_name_what_an_unnamed_call_runs(run):

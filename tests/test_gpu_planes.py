@@ -222,6 +222,8 @@ def check_conv(dtype, n, h, w, c, f, r, s, stride, pads, pad_value, tile, split)
 ])
 def test_conv_any_alignment(dtype, n, h, w, c, f, r, s, stride, pads, pad_value, split):
     check_conv(dtype, n, h, w, c, f, r, s, stride, pads, pad_value, None, split)
+    for tile in ((64, 64, 32, 2, 2), (128, 64, 32, 4, 2)) if dtype == "float32" else ((64, 64, 64, 2, 2),):
+        check_conv(dtype, n, h, w, c, f, r, s, stride, pads, pad_value, tile, split)
 
 
 @pytest.mark.parametrize("dtype,tile", [("bfloat16", (64, 64, 64, 2, 2)), ("bfloat16", (128, 64, 64, 2, 2)),

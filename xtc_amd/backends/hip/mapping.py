@@ -311,7 +311,7 @@ def map_gemm(
     req_bk = bk or dflt_tile[2]
     matches = [
         t
-        for t in cands
+        for t in dict.fromkeys([*cands, dflt_tile])  # the default may be a tile of this shape's kernel only
         if t[0] == req_bm
         and t[1] == req_bn
         and t[2] == req_bk

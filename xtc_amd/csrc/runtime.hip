@@ -1246,11 +1246,13 @@ const PlanesEntry* planes_conv_pick(const xtc_hip_conv2d_desc& d, const xtc_hip_
   return planes_pick(d.dtype, 1, 0, t, M, d.F, K, split_k);
 }
 
-// Block of a conv2d whose channels or filters are not whole vectors on
+// Default block of a conv2d whose channels or filters are not whole vectors on
 // gemm_planes: 64x64, or in fp32 128x64 over 8 waves from 192 workgroups of
-// it.  4x224x224x3, 7x7 stride 2 over 64 filters: 27.5 us on 64x64, 22.4 on
-// 128x64 (35.5 with the channels copied to whole vectors first); 56x56x10 3x3
-// over 64 (25 blocks): 9.6 and 10.5 us (13.8).
+// it (us, 64x64 and 128x64, by workgroups of 128x64; 3 channels unless noted):
+// 25 (56x56x10 3x3) 9.5 10.5; 64 6.4 7.0; 98 6.6 7.2; 128 6.8 7.3; 162 7.6 7.5;
+// 196 (2x224x224 7x7 stride 2) 16.1 15.0, (112x112x10 5x5) 21.9 20.3; 200
+// (80x80x35) 25.6 23.8; 208 (40x40x50 split 4) 16.7 17.2; 256 8.2 8.0; 294
+// (3x224x224 7x7 stride 2) 20.2 21.9; 392 (4x224x224) 26.5 22.4; 784 40.3 39.5.
 xtc_hip_tile planes_conv_any_tile(int dtype, int M, int N, int splits) {
   if (dtype == XTC_HIP_BF16) return {64, 64, 64, 2, 2};
   if ((int64_t)((M + 127) / 128) * ((N + 63) / 64) * splits >= 192) return {128, 64, 32, 4, 2};
@@ -1623,34 +1625,40 @@ bool conv_can_stage(const xtc_hip_conv2d_desc& d) {
 
 // Whether gemm_planes gathers the windows of d, whose channels or filters are
 // not whole 16-byte vectors or whose operands are not 16-byte aligned, element
-// by element, and in how many splits of K (those of the copied conv).  fp32
-// always; bf16, whose products are cheaper beside the gather, below 16 channels
-// (56x56x50 3x3 over 64: 20.3 us gathered, 18.9 copied to whole vectors first)
-// and where the copy cannot be made.
-bool conv_gathers(const xtc_hip_conv2d_desc& d, int OH, int OW, int* split_k) {
+// by element, on which tile and in how many splits of K (those of its class, in
+// a query, or of the copied conv's).  By default fp32 always; bf16, whose
+// products are cheaper beside the gather, below 16 channels (56x56x50 3x3 over
+// 64: 20.3 us gathered, 18.9 copied to whole vectors first).  A named tile has to
+// be one of the gather's, or the copied conv runs it; where no copy can be made
+// it is gathered on the default's.
+bool conv_gathers(const xtc_hip_conv2d_desc& d, int OH, int OW, bool query, xtc_hip_tile* tile, int* split_k) {
   if (d.dtype == XTC_HIP_F64 || generic_only() || !planes_offsets_fit(4, 1, d.F)) return false;
-  const bool can_stage = conv_can_stage(d);
-  xtc_hip_conv2d_desc dc = d;  // the tile, split and refusals of the copied conv
-  if (can_stage) dc.C = (d.C + conv_vec(d) - 1) / conv_vec(d) * conv_vec(d);
-  xtc_hip_tile t = d.tile;
-  *split_k = d.split_k;
-  if (t.bm == 0) {
+  const int M = d.N * OH * OW, K = d.R * d.S * d.C;
+  const bool can_stage = conv_can_stage(d), named = d.tile.bm != 0;
+  const int bk = d.dtype == XTC_HIP_F32 ? 32 : 64;
+  const bool own = named && d.tile.bk == bk && planes_entry(d.dtype, 1, 0, 0, d.tile);
+  *split_k = d.split_k < 1 ? 1 : d.split_k;
+  bool gather = can_stage ? (d.dtype == XTC_HIP_F32 || d.C < 16) && (own || !named) : !short_sums(d.dtype, M, d.F, K);
+  if (gather && !named) {
+    xtc_hip_conv2d_desc dc = d;
+    if (can_stage) dc.C = (d.C + conv_vec(d) - 1) / conv_vec(d) * conv_vec(d);
     int sk = 1;
-    conv_class_tile(dc, OH, OW, &t, &sk);
-    if (*split_k <= 0) *split_k = sk;
+    conv_class_tile(query ? d : dc, OH, OW, tile, &sk);
+    if (d.split_k <= 0) *split_k = sk;
+    const GemmEntry* e = find_entry(d.dtype, 1, *tile);
+    const void* p = (const void*)(uintptr_t)256;
+    if (can_stage) gather = e && e->launch && !direct_conv_applies(dc, *tile, *split_k, OH, OW, p, p, p, nullptr);
   }
-  if (!can_stage) return !short_sums(d.dtype, (int64_t)d.N * OH * OW, d.F, d.R * d.S * d.C);
-  const GemmEntry* e = find_entry(d.dtype, 1, t);
-  const void* p = (const void*)(uintptr_t)256;
-  return e && e->launch && (d.dtype == XTC_HIP_F32 || d.C < 16) && !direct_conv_applies(dc, t, *split_k, OH, OW, p, p, p, nullptr);
+  *tile = own ? d.tile : planes_conv_any_tile(d.dtype, M, d.F, effective_splits(K, *split_k, bk));
+  return gather;
 }
 
-// The tile and split of a conv2d descriptor that leaves `tile` zeroed: those
-// of its class, with the split fitted to the chip in bf16.
+// The tile and split of a conv2d descriptor that leaves `tile` zeroed: the
+// gather's, or those of its class with the split fitted to the chip in bf16.
 void default_conv_tile(const xtc_hip_conv2d_desc& d, int OH, int OW, xtc_hip_tile* t, int* split_k) {
+  if ((d.C % conv_vec(d) || d.F % conv_vec(d)) && conv_gathers(d, OH, OW, true, t, split_k)) return;
   conv_class_tile(d, OH, OW, t, split_k);
-  int gathered;
-  if (d.dtype != XTC_HIP_BF16 || ((d.C % 8 || d.F % 8) && conv_gathers(d, OH, OW, &gathered))) return;
+  if (d.dtype != XTC_HIP_BF16) return;
   // channels as they are staged
   const int M = d.N * OH * OW, K = d.R * d.S * ((d.C + 7) / 8 * 8);
   if (d.F % 8 == 0 && planes_conv_pick(d, *t, *split_k, M, K))
@@ -2567,6 +2575,12 @@ int xtc_hip_conv2d_pipeline_depths(const xtc_hip_conv2d_desc* desc, int* depths,
   const int OH = (HP - d.R) / d.stride_h + 1;
   const int OW = (WP - d.S) / d.stride_w + 1;
   const int vec = conv_vec(d);
+  xtc_hip_tile u;
+  if (int sk; d.tile.bm && !find_entry(d.dtype, 1, d.tile) && (d.C % vec || d.F % vec) && conv_gathers(d, OH, OW, true, &u, &sk) &&
+              same_tile(u, d.tile)) {
+    depths[0] = 2;  // the gather's own tile: two LDS buffers
+    return 1;
+  }
   if (d.C % vec && conv_can_stage(d)) {
     // xtc_hip_conv2d stages such a conv with zero channels up to the next
     // whole vector and runs the MFMA conv on the copies: describe that kernel
@@ -2651,11 +2665,10 @@ int xtc_hip_conv2d(const xtc_hip_conv2d_desc* desc, const void* input, const voi
   const int M = d.N * OH * OW;
   const int K = d.R * d.S * d.C;
   const bool vec_ok = d.C % vec == 0 && d.F % vec == 0 && aligned16(input) && aligned16(weight);
-  if (int split_k; !vec_ok && conv_gathers(d, OH, OW, &split_k)) {
+  xtc_hip_tile u;
+  if (int split_k; !vec_ok && conv_gathers(d, OH, OW, false, &u, &split_k)) {
     Scratch x{s};
-    xtc_hip_tile u = planes_conv_any_tile(d.dtype, M, d.F, 1);
-    split_k = splits_with_room(split_k < 1 ? 1 : split_k, M, d.F, K, u, x);
-    u = planes_conv_any_tile(d.dtype, M, d.F, effective_splits(K, split_k, u.bk));
+    split_k = splits_with_room(split_k, M, d.F, K, u, x);
     const GemmEntry own{d.dtype, 1, u.bm, u.bn, u.bk, u.wgm, u.wgn, 0, 0, planes_entry(d.dtype, 1, 0, 0, u)->launch,
                         nullptr};
     GemmArgs a = conv_args(d, OH, OW, input, weight, out, bias);
