@@ -152,7 +152,7 @@ typedef struct {
  * buffers of the stream that grow on demand; a call fails with a message when
  * one cannot be allocated.  fp32 and bf16 calls without whole 16-byte vectors
  * (strides, K, N or operand addresses), which no scratch may stop, run unsplit
- * instead: where their scratch would not fit in
+ * instead: where their partial sums would not fit in
  * XTC_HIP_NOALLOC_SCRATCH_BYTES or cannot be allocated, and on a stream that is
  * being captured, so that the graph keeps no address of a buffer that a later
  * call replaces (the sums are then in another order). */
@@ -174,7 +174,10 @@ int xtc_hip_matmul(const xtc_hip_matmul_desc *desc, const void *A, const void *B
  * static array per device of XTC_HIP_NOALLOC_SCRATCH_BYTES, set up by
  * xtc_hip_init.  A call that needs more fails with a message instead of
  * launching its GEMM; an fp32 or bf16 call without whole 16-byte vectors runs
- * unsplit instead, here and in xtc_hip_matmul.  The counters are cleared by a kernel on the call's stream before the GEMM.
+ * unsplit instead, here and in xtc_hip_matmul, and here alone (its sums in
+ * another order) where copies of transposed operands leave its partial sums no
+ * room.  The counters are cleared by a kernel on the call's stream before the
+ * GEMM.
  * Every call on a device shares that device's array, whatever its stream:
  * calls that overlap on one device race, so callers order them (one stream,
  * or a wait between streams). */

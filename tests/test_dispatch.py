@@ -127,7 +127,6 @@ out.append(L.xtc_hip_last_error().decode())
 @pytest.mark.parametrize("shape,split,trans_a,splits", [
     ((509, 1021, 777), 4, 0, 4),
     ((4097, 4097, 300), 2, 0, 1),  # 134 MB of partial sums
-    ((2500, 1001, 4001), 3, 1, 1),  # 30 MB of them behind a 40 MB copy of A
     ((2500, 1001, 2001), 3, 1, 3),
 ])
 def test_both_entry_points_split_ragged_calls_alike(run, shape, split, trans_a, splits):
@@ -140,6 +139,21 @@ for fn in ("xtc_hip_matmul", "xtc_hip_matmul_noalloc"):
 """)
     kernel = "gemm_planes<float, 64, 64, 32, 2, 2, false, false, false, 1, 1>"
     assert grown[-1] == static[-1] == [kernel, splits, 256]
+
+
+@pytest.mark.parametrize("shape,splits,static_splits", [
+    ((2500, 1001, 4001), 3, 1),  # 30 MB of partial sums beside a 40 MB copy of A
+    ((2900, 429, 7572), 4, None),  # an 88 MB copy, which the static scratch refuses
+])
+def test_copies_of_transposed_operands_cost_growing_calls_no_split(run, shape, splits, static_splits):
+    M, N, K = shape
+    grown, static = run(f"""
+for fn in ("xtc_hip_matmul", "xtc_hip_matmul_noalloc"):
+    out.append(matmul("float32", {M}, {N}, {K}, split={splits}, trans_a=1, tile=(64, 64, 32, 2, 2), fn=fn))
+""")
+    kernel = "gemm_planes<float, 64, 64, 32, 2, 2, false, false, false, 1, 1>"
+    assert grown[-1] == [kernel, splits, 256]
+    assert static[-1] == [kernel, static_splits, 256] if static_splits else "scratch" in static
 
 
 @pytest.mark.parametrize("dtype,tile,split,shape,trans_b,kernel", [

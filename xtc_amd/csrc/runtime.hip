@@ -197,7 +197,7 @@ struct Scratch {
   hipStream_t s;
   char* fixed = nullptr;
   size_t cap = 0;
-  size_t used = 0;  // in growing mode: by staged copies
+  size_t used = 0;
 
   void* take(size_t bytes, const char* what) {
     const size_t off = (used + 255) & ~(size_t)255;
@@ -230,7 +230,6 @@ struct Scratch {
   }
   void* stage(int slot, size_t bytes) {
     if (fixed) return take(bytes, "transposed operand copies");
-    used = ((used + 255) & ~(size_t)255) + bytes;  // as take() counts (splits_with_room)
     void* p = staging(slot, bytes, s);
     if (!p) fail("cannot allocate %zu bytes of transpose staging", bytes);
     return p;
@@ -2126,7 +2125,8 @@ bool capturing(hipStream_t s) {
 // calls took none before they ran on gemm_planes): `split_k`, or 1 where the
 // split-K scratch would not fit in the no-allocation entry point's, whichever
 // entry point is called, so that both take their sums in the same order (the
-// library's own splits need 38 MB at most).  In growing mode also 1 where it
+// library's own splits need 38 MB at most), but where copies of transposed
+// operands fill the fixed scratch.  In growing mode also 1 where it
 // cannot be allocated, and on a stream that is being captured: the graph would
 // keep the address of a growable buffer, which a later call frees to enlarge it
 // and a replay on another stream shares with the launches of this one.
@@ -2135,7 +2135,7 @@ int splits_with_room(int split_k, int M, int N, int K, const xtc_hip_tile& t, co
   if (splits == 1) return 1;
   const size_t tiles = (size_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
   const size_t bytes = (size_t)splits * M * planes_ldp(N) * sizeof(float);
-  // two 256-byte alignments
+  // two 256-byte alignments; `used`: copies of transposed operands in the fixed scratch
   if (x.used + bytes + tiles * sizeof(unsigned) + 512 > XTC_HIP_NOALLOC_SCRATCH_BYTES) return 1;
   if (x.fixed) return split_k;
   if (capturing(x.s)) return 1;
