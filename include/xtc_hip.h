@@ -294,17 +294,21 @@ int xtc_hip_matmul_default_tile(const xtc_hip_matmul_desc *desc, xtc_hip_tile *o
  * 112x64x16). */
 int xtc_hip_conv2d_default_tile(const xtc_hip_conv2d_desc *desc, xtc_hip_tile *out, int *split_k);
 
-/* Pipeline depths the kernel that runs `desc` (with 256-byte aligned
- * operands) is compiled for: the LDS stages of the LDS-DMA kernels, 2 for
- * the register-staged generic template (and 4 for its 64x64 tiles, with
- * three register sets of loads in flight: the default when K is split), 1
- * for the scalar kernel.  Writes up
+/* Pipeline depths that `desc` (with 256-byte aligned operands) may name: the
+ * LDS stages of the LDS-DMA kernels, the register ring of the split-wave
+ * kernel, 2 for the register-staged generic template (and 4 for its 64x64
+ * tiles, with three register sets of loads in flight: the default when K is
+ * split), 1 for the scalar kernel and for calls without whole 16-byte vectors.
+ * The bf16-plane kernel has one pipeline and takes every depth that its tiles
+ * had before it; xtc_hip_matmul_pipelines says how many of the listed depths,
+ * from the first, are pipelines of their own.  Writes up
  * to max_depths of them, the default first, and returns their count (-1 on
  * error).  A schedule's unroll of the K-slab loop selects one
  * (MlirCompilerPasses.py:579-596 unrolls loops by the scheduled factor; here
  * the factor of the loop that walks the LDS slabs is how many slabs are in
  * flight).  The conv2d kernels are compiled for one depth each. */
 int xtc_hip_matmul_pipeline_depths(const xtc_hip_matmul_desc *desc, int *depths, int max_depths);
+int xtc_hip_matmul_pipelines(const xtc_hip_matmul_desc *desc);
 int xtc_hip_conv2d_pipeline_depths(const xtc_hip_conv2d_desc *desc, int *depths, int max_depths);
 
 /* ---------------------------------------------------------- timing harness */

@@ -182,6 +182,35 @@ def test_named_convs_run_their_split(run, tile, split, shape):
     assert rows[-1][0].startswith(f"gemm_planes<__bf16, {tile[0]}, {tile[1]}, 64,") and rows[-1][1] == split
 
 
+def test_split_wave_depths_behind_the_64x64_tile(run):
+    # 512^3 at split 4: the tile's depths 4 (the default) and 2 are the split-wave kernel's ring
+    rows = run("""
+for stages in (0, 4, 2):
+    out.append(matmul("float32", 512, 512, 512, tile=(64, 64, 32, 2, 2), split=4, stages=stages))
+""")
+    assert [r[-1][0] for r in rows] == [f"gemm_f32_splitwave<4, {depth}>" for depth in (4, 4, 2)]
+
+
+def test_explorer_points_are_kernels_of_their_own(run):
+    # every sample of the explorer's space launches something else: a depth that
+    # only renames the one pipeline of gemm_planes is no point
+    points, launches = run("""
+import xtc_amd.graphs.xtc.op as O
+from xtc_amd.search.strategies import Strategies
+a, b = O.tensor((1024, 1024), "float32", name="A"), O.tensor((1024, 1024), "float32", name="B")
+with O.graph(name="mm") as gb:
+    O.matmul(a, b, name="C")
+wide = [x for x in Strategies.create("tile_hip", gb.graph)._points()
+        if (x[0], x[2], x[4]) in ((256, 128, 32), (128, 256, 32), (128, 128, 32), (64, 64, 32))]
+out.append([tuple(x) for x in wide])
+out.append([matmul("float32", 1024, 1024, 1024, tile=(x[0], x[2], x[4], x[0] // x[1], x[2] // x[3]), split=x[5],
+                   stages=x[6])[-1] for x in wide])
+""")
+    assert len(points) > 20
+    kernels = [tuple(x) + tuple(p[:6]) for p, x in zip(points, launches)]
+    assert len(set(kernels)) == len(kernels)
+
+
 @pytest.mark.parametrize("dtype,tile,pad_value,launches", [
     # by default and on the gather's own tiles in place, else on whole-vector copies
     ("float32", None, 0.0, ["gemm_planes<float, 128, 64, 32, 4, 2, true, false, false, 1, 1>"]),

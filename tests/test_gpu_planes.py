@@ -97,12 +97,13 @@ def test_any_alignment(dtype, M, N, K, split):
     np.testing.assert_array_equal(run_matmul(ai, bi, dtype, split_k=split), ai.astype(np.float64) @ bi)
 
 
-def test_splitwave_behind_the_default_depth_of_64x64x32():
-    # the same splits in the same order: bit-identical to the template
+def test_splitwave_behind_64x64x32():
+    # the same splits in the same order as the template, which runs 80 rows (no
+    # whole 32-row blocks): its rows bit for bit, at both depths
     a, b = rng_uniform(3, (96, 512)), rng_uniform(4, (512, 160))
-    runs = [_run_depth(a, b, "float32", (64, 64, 32, 2, 2), 4, depth, False) for depth in (0, 2, 4)]
-    np.testing.assert_array_equal(runs[0], runs[1])
-    np.testing.assert_array_equal(runs[0], runs[2])
+    template = _run_depth(a[:80].copy(), b, "float32", (64, 64, 32, 2, 2), 4, 0, False)
+    for depth in (0, 2, 4):
+        np.testing.assert_array_equal(_run_depth(a, b, "float32", (64, 64, 32, 2, 2), 4, depth, False)[:80], template)
 
 
 # B stored transposed, read in place: rows of B^T cut by N, slabs cut by K
@@ -116,6 +117,18 @@ def test_transposed_b(dtype, tile, M, N, K, split):
     for bt in (True, False):
         out = run_matmul_layout(ai, bi, dtype, False, bt, tile=tile, split_k=split, pad_a=8, pad_b=16)
         np.testing.assert_array_equal(out, ai.astype(np.float64) @ bi)
+
+
+# B^T in place with bias and relu in the epilogue and in the finishing workgroup
+@pytest.mark.parametrize("dtype,tile", [("float32", TILES[2]), ("float32", (64, 64, 32, 2, 2)),
+                                        ("bfloat16", (64, 64, 64, 2, 2)), ("bfloat16", (128, 128, 64, 2, 2))])
+@pytest.mark.parametrize("split", [1, 2])
+def test_transposed_b_bias_relu(dtype, tile, split):
+    M, N, K = 130, 264, 1048
+    ai, bi = ref.np_init((M, K), "float32"), ref.np_init((K, N), "float32")[::-1].copy() - 4
+    bias = (np.arange(N) % 9 - 4).astype(np.float32)
+    out = run_matmul_layout(ai, bi, dtype, False, True, tile=tile, split_k=split, relu=True, bias=bias)
+    np.testing.assert_array_equal(out, np.maximum(ai.astype(np.float64) @ bi + bias, 0))
 
 
 # bf16 workgroups of 4 or 8 waves (512 and 520 of them); 128-row tiles whose

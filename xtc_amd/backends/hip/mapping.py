@@ -19,12 +19,13 @@ where (b,h,w) form GEMM-M, f GEMM-N and (r,s,c) GEMM-K):
     otherwise tiles are rastered in groups of 8 tile-rows (L2 reuse)
   * unroll of the loop that walks the K slabs (k without split-K, k1 with
     it; c for conv) by S -> pipeline depth S: S slabs in flight through S
-    LDS stages.  It must be a depth the kernel is compiled for
+    LDS stages.  It must be a depth that the kernel takes
     (xtc_hip_matmul_pipeline_depths: 3-6 for the fp32 LDS-DMA BK-16 tiles,
-    2-3 for its BK-32 256-wide tiles, 2-4 for 128x128, 3-5 for the bf16
-    ping-pong kernel, 2-4 for the skinny bf16 kernel, 2 for the generic
-    template and 4 on its 64x64 tiles, which keep three slabs of loads in
-    flight in registers); absent, the kernel's default.  Unroll factors of
+    3-5 for the bf16 ping-pong kernel, 2-4 for the skinny bf16 kernel, 2 for
+    the generic template and 4 on its 64x64 tiles, which keep three slabs of
+    loads in flight in registers; the bf16-plane kernel runs its one pipeline
+    behind 2-3 on the fp32 256-wide tiles, 2-4 on 128x128 of eight waves and
+    the template's depths elsewhere); absent, the kernel's default.  Unroll factors of
     the other loops are recorded: the MFMA loop over a slab and the wave's
     sub-tiles are always fully unrolled, and the block and wave tiles are
     spread over waves and lanes
@@ -198,7 +199,9 @@ def _attrs_key(attrs: dict[str, Any], conv: bool) -> tuple[Any, ...]:
 
 
 @lru_cache(maxsize=4096)
-def _depths(key: tuple[Any, ...], conv: bool, tile: tuple[int, int, int, int, int], split_k: int) -> tuple[int, ...]:
+def _depths(key: tuple[Any, ...], conv: bool, tile: tuple[int, int, int, int, int],
+            split_k: int) -> tuple[tuple[int, ...], int]:
+    """The depths that a launch may name, and how many of them differ."""
     from ...runtimes.hip import capi
 
     dt = capi.DTYPE_IDS[key[0]]
@@ -206,17 +209,24 @@ def _depths(key: tuple[Any, ...], conv: bool, tile: tuple[int, int, int, int, in
         _, nb, h, w, c, f, r, s, (sh, sw), (pt, pb, pl, pr) = key
         cd = capi.Conv2dDesc(dtype=dt, N=nb, H=h, W=w, C=c, F=f, R=r, S=s, stride_h=sh, stride_w=sw, pad_top=pt,
                              pad_bottom=pb, pad_left=pl, pad_right=pr, tile=capi.Tile(*tile), split_k=split_k)
-        return tuple(capi.conv2d_pipeline_depths(cd))
+        return tuple(capi.conv2d_pipeline_depths(cd)), 1
     _, m, n, k, ta, tb = key
     md = capi.MatmulDesc(dtype=dt, M=m, N=n, K=k, tile=capi.Tile(*tile), split_k=split_k, trans_a=int(ta),
                          trans_b=int(tb))
-    return tuple(capi.matmul_pipeline_depths(md))
+    return tuple(capi.matmul_pipeline_depths(md)), capi.matmul_pipelines(md)
 
 
 def pipeline_depths(attrs: dict[str, Any], conv: bool, tile: tuple[int, int, int, int, int], split_k: int) -> list[int]:
-    """Pipeline depths of the kernel that runs this launch with `tile` and
-    `split_k`, its default first (xtc_hip_*_pipeline_depths)."""
-    return list(_depths(_attrs_key(attrs, conv), conv, tuple(tile), int(split_k)))
+    """Pipeline depths that this launch may name with `tile` and `split_k`,
+    its default first (xtc_hip_*_pipeline_depths)."""
+    return list(_depths(_attrs_key(attrs, conv), conv, tuple(tile), int(split_k))[0])
+
+
+def distinct_depths(attrs: dict[str, Any], conv: bool, tile: tuple[int, int, int, int, int], split_k: int) -> list[int]:
+    """Those of pipeline_depths that are pipelines of their own, the default
+    first (xtc_hip_matmul_pipelines)."""
+    depths, pipelines = _depths(_attrs_key(attrs, conv), conv, tuple(tile), int(split_k))
+    return list(depths[:pipelines])
 
 
 def _slab_loop(sched: HipNodeSchedule, k_dims: list[str], split: bool) -> str:

@@ -1411,8 +1411,7 @@ bool splitwave_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t,
   if (d.M % 32 || d.N % 32 || d.K % (16 * split_k)) return false;
   if (lda % 4 || !aligned16(A)) return false;
   if (t.bm == 32 && t.bn == 32 && t.bk == 16 && t.wgm == 1 && t.wgn == 1) return true;
-  // The default depth of the 64x64x32 tile (2x2 waves of 32x32), when its
-  // 32x32 blocks fit in one wave of 256 CUs: the wave blocks become workgroups
+  // The 64x64x32 tile (2x2 waves of 32x32), when its 32x32 blocks fit in one wave of 256 CUs: the wave blocks become workgroups
   // whose waves are the splits, which meet in LDS instead of memory, in the
   // same order (the results are bit-identical when a split is whole slabs).
   // 512^3 at split 4 11.0 -> 5.5 us, 256^3 at split 2 9.5 -> 4.9, 32x4096x1024
@@ -1423,7 +1422,7 @@ bool splitwave_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t,
   // 32x2048x1280 11.5 -> 12.2, 32x4096x4864 33.2 -> 39.3; but 32x4096x2048
   // 19.9 -> 18.2, 32x8192x1536 23.0 -> 15.2).
   const int64_t blocks = (int64_t)(d.M / 32) * (d.N / 32);
-  return t.bm == 64 && t.bn == 64 && t.bk == 32 && t.wgm == 2 && t.wgn == 2 && d.stages == 0 &&
+  return t.bm == 64 && t.bn == 64 && t.bk == 32 && t.wgm == 2 && t.wgn == 2 &&
          d.K % (32 * split_k) == 0 && blocks <= 256 &&
          (split_k <= 4 || (blocks >= 128 && d.K <= 256 * split_k));
 }
@@ -1881,7 +1880,7 @@ const char* path_name(MatmulPath p) {
   }
 }
 
-// Pipeline depths the kernel of path p compiles for tile t: LDS stages of
+// Pipeline depths that the kernel of path p takes for tile t: LDS stages of
 // the LDS-DMA kernels, the generic template's register-staged double buffer
 // (2) and, for the tiles with a ring instance (`ring`, generic_ring), its
 // three register sets (4), the split-wave kernel's ring of register chunks,
@@ -1906,7 +1905,7 @@ int path_depths(MatmulPath p, const xtc_hip_tile& t, int ring, int* out, int max
       tmp[n++] = 2;
       break;
     case MatmulPath::SplitWave:
-      if (t.bm == 64) {  // the 64x64x32 tile's own depths: its default runs here, a named one on the template
+      if (t.bm == 64) {  // as the template's of that tile
         tmp[n++] = 4;
         tmp[n++] = 2;
         break;
@@ -1914,8 +1913,9 @@ int path_depths(MatmulPath p, const xtc_hip_tile& t, int ring, int* out, int max
       for (int v : kSplitWaveDepths) tmp[n++] = v;
       break;
     case MatmulPath::Planes:
-      // one pipeline behind every depth a schedule may name: two LDS buffers
-      // and the next slab in registers
+      // one pipeline (two LDS buffers and the next slab or two in registers)
+      // behind every depth that the tile's kernels before this one had
+      // (path_pipelines)
       if (t.bk == 64 && t.bm == 128) {
         tmp[n++] = 2;
         break;
@@ -1950,6 +1950,10 @@ int path_depths(MatmulPath p, const xtc_hip_tile& t, int ring, int* out, int max
   for (int i = 0; i < n && i < max; ++i) out[i] = tmp[i];
   return n;
 }
+
+// How many of path_depths' depths are pipelines of their own, from the first;
+// the rest run the default's.
+int path_pipelines(MatmulPath p, int depths) { return p == MatmulPath::Planes ? 1 : depths; }
 
 bool has_depth(MatmulPath p, const xtc_hip_tile& t, int ring, int stages) {
   int depths[16];
@@ -2549,9 +2553,8 @@ int xtc_hip_conv2d_default_tile(const xtc_hip_conv2d_desc* desc, xtc_hip_tile* o
   return 0;
 }
 
-int xtc_hip_matmul_pipeline_depths(const xtc_hip_matmul_desc* desc, int* depths, int max_depths) {
-  if (!desc || !depths || max_depths < 1) return -fail("null argument");
-  const xtc_hip_matmul_desc& d = *desc;
+// The depths that desc may name and, in *pipelines, how many of them differ.
+static int matmul_depths(const xtc_hip_matmul_desc& d, int* depths, int max_depths, int* pipelines) {
   int lda, ldb, ldc, split_k;
   xtc_hip_tile t;
   // operands as the allocators hand them out: 256-byte aligned
@@ -2563,7 +2566,21 @@ int xtc_hip_matmul_pipeline_depths(const xtc_hip_matmul_desc* desc, int* depths,
   const int ring = path == MatmulPath::Generic || path == MatmulPath::Planes
                        ? generic_ring(find_entry(d.dtype, 0, t), effective_splits(d.K, split_k, t.bk))
                        : 0;
-  return path_depths(path, t, ring, depths, max_depths);
+  const int n = path_depths(path, t, ring, depths, max_depths);
+  *pipelines = path_pipelines(path, n);
+  return n;
+}
+
+int xtc_hip_matmul_pipeline_depths(const xtc_hip_matmul_desc* desc, int* depths, int max_depths) {
+  if (!desc || !depths || max_depths < 1) return -fail("null argument");
+  int pipelines;
+  return matmul_depths(*desc, depths, max_depths, &pipelines);
+}
+
+int xtc_hip_matmul_pipelines(const xtc_hip_matmul_desc* desc) {
+  if (!desc) return -fail("null argument");
+  int depths[16], pipelines;
+  return matmul_depths(*desc, depths, 16, &pipelines) < 0 ? -1 : pipelines;
 }
 
 int xtc_hip_conv2d_pipeline_depths(const xtc_hip_conv2d_desc* desc, int* depths, int max_depths) {

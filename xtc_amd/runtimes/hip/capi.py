@@ -201,6 +201,7 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     "xtc_hip_matmul_default_tile": (_i, [ctypes.POINTER(MatmulDesc), ctypes.POINTER(Tile), ctypes.POINTER(_i)]),
     "xtc_hip_conv2d_default_tile": (_i, [ctypes.POINTER(Conv2dDesc), ctypes.POINTER(Tile), ctypes.POINTER(_i)]),
     "xtc_hip_matmul_pipeline_depths": (_i, [ctypes.POINTER(MatmulDesc), ctypes.POINTER(_i), _i]),
+    "xtc_hip_matmul_pipelines": (_i, [ctypes.POINTER(MatmulDesc)]),
     "xtc_hip_conv2d_pipeline_depths": (_i, [ctypes.POINTER(Conv2dDesc), ctypes.POINTER(_i), _i]),
     "xtc_hip_evaluate_perf": (
         None,
@@ -305,12 +306,21 @@ def default_tile(dtype: str, conv: bool, M: int, N: int, K: int) -> tuple[tuple[
 
 
 def matmul_pipeline_depths(desc: MatmulDesc) -> list[int]:
-    """Pipeline depths of the kernel that runs `desc`, the default first."""
+    """Pipeline depths that `desc` may name, the default first."""
     out = (ctypes.c_int * 16)()
     n = lib().xtc_hip_matmul_pipeline_depths(ctypes.byref(desc), out, 16)
     if n < 0:
         raise HipError(f"matmul_pipeline_depths: {last_error()}")
     return list(out[: min(n, 16)])
+
+
+def matmul_pipelines(desc: MatmulDesc) -> int:
+    """How many of matmul_pipeline_depths' depths, from the first, are pipelines
+    of their own; the others run the default's."""
+    n = lib().xtc_hip_matmul_pipelines(ctypes.byref(desc))
+    if n < 0:
+        raise HipError(f"matmul_pipelines: {last_error()}")
+    return n
 
 
 def conv2d_pipeline_depths(desc: Conv2dDesc) -> list[int]:

@@ -572,7 +572,7 @@ class Strategy_HIP(BaseStrategy):
         with split_k > 1, {c1: K/split_k, c2: bk} plus parallelize(c), for
         the splits whose slice K/split_k is at most C;
       * stages: unroll of the slab loop (k, or k1 under split-K; c or c1 for conv)
-        by the pipeline depth, one of the depths the tile's kernel is
+        by the pipeline depth, one of the pipelines the tile's kernel is
         compiled for on this shape (the default first).
 
     Its default sample is the library's own choice for the shape, and the
@@ -625,9 +625,9 @@ class Strategy_HIP(BaseStrategy):
         raise ValueError(f"tile_hip: node {node} has no matmul/conv2d kernel launch")
 
     def _depths(self, tile: tuple[int, int, int, int, int], split: int) -> list[int]:
-        from ..backends.hip.mapping import pipeline_depths
+        from ..backends.hip.mapping import distinct_depths
 
-        return pipeline_depths(self._attrs, self._conv, tile, split)
+        return distinct_depths(self._attrs, self._conv, tile, split)
 
     def _points(self) -> list[list[int]]:
         from ..runtimes.hip import capi
