@@ -546,7 +546,7 @@ def test_mapping_unroll_of_the_slab_loop_selects_the_pipeline_depth():
         (ln,) = [l for l in b.plan.launches if l.kind == "matmul"]
         return map_gemm(ln.attrs, False, sch.schedule().node(ln.node), "strict"), ln.attrs
 
-    # LDS-DMA fp32 256x128x32: 3 stages (default) or 2
+    # bf16-plane kernel behind 256x128x32: its one pipeline is named 3 (default) or 2
     c, attrs = cfg(tiles, {"k": 2})
     assert c.tile == (256, 128, 32, 4, 2) and c.stages == 2
     assert pipeline_depths(attrs, False, c.tile, 1) == [3, 2]
@@ -751,7 +751,7 @@ def test_instances_and_default_tile():
     assert ("bfloat16", False, (256, 256, 64, 2, 4)) in tiles
     assert ("bfloat16", False, (256, 256, 32, 2, 4)) in tiles
     assert any(d == "float32" and c for d, c, _ in tiles)
-    # large aligned fp32: the LDS-DMA fp32 kernel's tile when it fills the chip
+    # large aligned fp32: the 8-wave tile when it fills the chip
     assert tuple(capi.default_tile("float32", False, 4096, 4096, 4096)[0]) == (256, 128, 32, 4, 2)
     assert tuple(capi.default_tile("float32", False, 2048, 2048, 2048)[0]) == (128, 128, 32, 2, 2)
     tile, split = capi.default_tile("bfloat16", False, 8192, 8192, 8192)

@@ -695,7 +695,7 @@ def test_pingpong_bf16_split_k_bias_relu_strided():
     np.testing.assert_array_equal(out, again)
 
 
-# ------------- LDS-DMA fp32 kernel (BK 32: 128x256, 256x128, 128x128; BK 16: 128x256, 256x128)
+# ------------- 8-wave fp32 tiles: bf16-plane kernel (BK 32), LDS-DMA fp32 kernel (BK 16)
 
 F32_LDS = [(128, 256, 32, 2, 4), (256, 128, 32, 4, 2), (128, 128, 32, 2, 4), (128, 256, 16, 2, 4), (256, 128, 16, 4, 2)]
 
@@ -704,9 +704,10 @@ F32_LDS = [(128, 256, 32, 2, 4), (256, 128, 32, 4, 2), (128, 128, 32, 2, 4), (12
 @pytest.mark.parametrize("K,split", [(16, 1), (32, 1), (64, 1), (80, 1), (96, 1), (1024, 1), (1056, 1), (512, 2),
                                      (1024, 4), (2048, 8)])
 def test_f32_lds_integer_exact_every_pipeline_depth(tile, K, split):
-    # K / BK / split slabs below, at and above the DMA lead (2 for BK 32, 3
-    # or 4 for BK 16; K = 16 and 80 take the generic kernel at BK 32);
-    # split-K finished in the kernel
+    # K / BK / split slabs below, at and above the loads' lead (2 slabs for BK
+    # 32, whose last one K cuts at K = 16 and 80; 3 or 4 for BK 16, which takes
+    # the generic kernel where K is no whole slabs a split); split-K finished in
+    # the kernel
     M, N = 512, 512
     a, b = _int_operands(M, N, K, 7)
     out = run_matmul(a, b, "float32", tile=tile, split_k=split)
@@ -974,7 +975,9 @@ def test_every_pipeline_depth(case):
 
 # the generic template's ring instances (64x64 tiles): three register sets
 # of loads in flight; one and two slabs, slab counts that are not multiples
-# of 3, ragged M, N, K, one split and several
+# of 3, ragged M, N, K, one split and several.  512^3 (split-wave kernel) and
+# bf16 64x64x64 (bf16-plane kernel) reach the template with
+# XTC_HIP_GENERIC_GEMM=1 only
 RING_CASES = [
     ("float32", (64, 64, 32, 2, 2), 4, (512, 512, 512)),
     ("float32", (64, 64, 32, 2, 2), 1, (200, 224, 240)),

@@ -83,16 +83,23 @@ def _both(dtype, M, N, K, tile, split_k, seed, trans_a=False, trans_b=False, rel
 # (dtype, tile, split_k, first (M, N, K), second (M, N, K), options): every
 # kernel family that takes scratch, plus one that takes none.
 CASES = [
-    # generic template, grid split-K: partials [4][M][N] and per-tile counters
+    # split-wave kernel behind 64x64x32: scratch-free
     ("float32", (64, 64, 32, 2, 2), 4, (384, 320, 2048), (128, 192, 1024), {}),
-    # LDS-DMA fp32 kernel with split-K 2, relu and bias in the finishing workgroup
+    # generic template, grid split-K: partials [4][M][N] and per-tile counters
+    ("float32", (64, 64, 16, 2, 2), 4, (384, 320, 2048), (128, 192, 1024), {}),
+    ("bfloat16", (64, 64, 32, 2, 2), 3, (256, 256, 1600), (64, 128, 704), {}),
+    # bf16-plane kernel with split-K 2, relu and bias in the finishing workgroup
     ("float32", (128, 128, 32, 2, 4), 2, (1024, 512, 2048), (512, 256, 512), {"relu": True, "bias": True}),
     # skinny bf16 kernel: split-K 8 over 1024-deep, then 512-deep chunks
     ("bfloat16", (16, 128, 64, 1, 4), 8, (16, 8192, 8192), (8, 4096, 4096), {}),
-    # generic bf16 template with split-K 3 (ragged K per split)
+    # bf16-plane kernel on bf16 operands, split-K 3 (ragged K per split); on two
+    # k-groups; B^T in place
     ("bfloat16", (64, 64, 64, 2, 2), 3, (256, 256, 1600), (64, 128, 704), {}),
-    # transposed A and B: both staged in the scratch, then split-K 2
+    ("bfloat16", (128, 128, 64, 2, 2), 3, (256, 512, 2120), (128, 128, 1600), {"relu": True, "bias": True}),
+    ("bfloat16", (128, 128, 64, 2, 2), 4, (130, 264, 2312), (128, 128, 512), {"trans_b": True}),
+    # transposed A and B: both staged in the scratch, then split-wave, then split-K 2
     ("float32", (64, 64, 32, 2, 2), 2, (512, 256, 384), (96, 160, 256), {"trans_a": True, "trans_b": True}),
+    ("float32", (64, 64, 16, 2, 2), 2, (500, 260, 388), (96, 160, 256), {"trans_a": True, "trans_b": True}),
     # split-wave kernel: scratch-free (partials meet in LDS)
     ("float32", (32, 32, 16, 1, 1), 4, (512, 512, 512), (256, 128, 256), {}),
     # ping-pong bf16 kernel, no split: scratch-free
@@ -109,7 +116,7 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("case", CASES, ids=[f"{c[0]}-{c[1]}-sk{c[2]}" for c in CASES])
+@pytest.mark.parametrize("case", CASES, ids=[f"{c[0]}-{c[1]}-sk{c[2]}{'-ta' if 'trans_a' in c[5] else ''}" for c in CASES])
 def test_noalloc_matches_matmul_on_two_calls(case):
     dtype, tile, split_k, first, second, opts = case
     for seed, (M, N, K) in enumerate((first, second)):
