@@ -115,8 +115,8 @@ def instances() -> list[tuple[int, int, int, int, int, int, int]]:
                             continue
                         if tile_legal(dtype, 0, bm, bn, bk, wgm, wgn):
                             out.append((dtype, 0, bm, bn, bk, wgm, wgn))
-    # fp32 128x128x32 with 8 waves (2x4 of 64x32): the LDS-DMA fp32 kernel's
-    # tile for N-narrow GEMMs (runtime.hip routes aligned shapes to it)
+    # fp32 128x128x32 with 8 waves (2x4 of 64x32): gemm_planes' tile for
+    # N-narrow GEMMs; this instance backs operand strides past 32-bit offsets
     if tile_legal(F32, 0, 128, 128, 32, 2, 4) and (F32, 0, 128, 128, 32, 2, 4) not in out:
         out.append((F32, 0, 128, 128, 32, 2, 4))
     # implicit-GEMM conv loaders: the conv shapes have small N (= F channels)

@@ -2,8 +2,9 @@
 // fp32 GEMM on fp32 MFMAs for aligned shapes on gfx950, LDS-DMA pipeline, one workgroup
 // of 8 waves per CU:
 //   C[M,N] = epilogue( A[M,K] @ B[K,N] ), fp32 row-major, optional split-K
-// with M % BM == 0, N % BN == 0, each split's K range a multiple of BK (16 or 32),
-// lda and ldb multiples of 4 and 16-byte aligned operands.
+// with M % BM == 0, N % BN == 0, each split's K range a multiple of BK = 16,
+// lda and ldb multiples of 4 and 16-byte aligned operands.  (The same blocks
+// over slabs of 32 run on bf16 MFMAs, gemm_planes.hpp.)
 //
 // v_mfma_f32_16x16x4_f32 issues at full rate with one or two waves per SIMD
 // from one workgroup, and drops to about 65 % with four (measured on MI355X
@@ -13,8 +14,8 @@
 //   * 8 waves (WGM x WGN), one workgroup per CU (the stages fill the LDS):
 //     two waves per SIMD;
 //   * global -> LDS by LDS DMA (global_load_lds_dwordx4, issued from asm),
-//     STAGES stages of one BK-deep slab, D = STAGES - 1 slabs ahead of the
-//     MFMAs;
+//     STAGES (3 to 6) stages of one slab of 24 KB, D = STAGES - 1 slabs ahead
+//     of the MFMAs;
 //   * per slab, each wave issues the DMA of slab t+D, reads its fragments of
 //     slab t (ds_read_b128 for A, ds_read_b32 for B), issues its MFMAs,
 //     waits for its own DMA of slab t+1 (s_waitcnt vmcnt) and meets the other
@@ -23,13 +24,13 @@
 // LDS layouts (16-byte chunks, XOR-swizzled so that a wave's fragment reads
 // hit distinct banks):
 //   * A: BM rows of BK floats; chunk c of row r holds global chunk
-//     c ^ swz_a(r).  Lane (l16, g) reads A[r][16 kc + 4 g .. +3] with one
+//     c ^ swz_a(r).  Lane (l16, g) reads A[r][4 g .. +3] with one
 //     ds_read_b128: the A values of 4 MFMAs (s = 0..3).
 //   * B: BK rows of BN floats; chunk c of row k holds global chunk
-//     c ^ (4 ((k >> 2) & 3)).  Lane (l16, g) reads B[16 kc + 4 g + s][n] with
+//     c ^ (4 ((k >> 2) & 3)).  Lane (l16, g) reads B[4 g + s][n] with
 //     ds_read_b32: the four lane groups read rows 4 apart, which the swizzle
 //     moves 16 floats (16 banks) apart.
-// The MFMA k index of lane group g at step s is physical k = 16 kc + 4 g + s
+// The MFMA k index of lane group g at step s is physical k = 4 g + s
 // for both operands, as in gemm.hpp, and the per-accumulator MFMA sequence
 // is the generic kernel's; B is the first operand, so a lane ends up holding
 // C[m][n .. n+3] and stores float4s.  Split-K uses the protocol of
@@ -53,11 +54,8 @@ typedef __attribute__((address_space(3))) float lds_f32;
 
 constexpr int waitcnt_vm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | (((n >> 4) & 3) << 14); }
 
-// 16-byte chunk swizzle of an A row of BK floats
-template <int BK>
-__device__ __forceinline__ int swz_a(int r) {
-  return BK == 16 ? ((r >> 2) & 3) : ((r >> 1) & 7);
-}
+// 16-byte chunk swizzle of an A row
+__device__ __forceinline__ int swz_a(int r) { return (r >> 2) & 3; }
 // 16-byte chunk swizzle of B row k
 __device__ __forceinline__ int swz_b(int k) { return ((k >> 2) & 3) << 2; }
 
@@ -74,11 +72,11 @@ __device__ __forceinline__ void slab_barrier() {
 
 }  // namespace f32lds
 
-template <int BM, int BN, int BK, int WGM, int WGN, int STAGES>
+template <int BM, int BN, int WGM, int WGN, int STAGES>
 __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512))) gemm_f32_lds(GemmArgs args) {
   using namespace f32lds;
   constexpr int TM = BM / WGM / 16, TN = BN / WGN / 16;  // 16x16 tiles per wave
-  constexpr int KC = BK / 16;                            // 16-deep k chunks per slab
+  constexpr int BK = 16;
   constexpr int A_STAGE = BM * BK * 4;
   constexpr int B_STAGE = BK * BN * 4;
   constexpr int STAGE = A_STAGE + B_STAGE;
@@ -91,15 +89,14 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512))) gemm_f32_
   constexpr int B_CHUNKS = BN / 4;
   constexpr int D = STAGES - 1;
   static_assert(WGM * WGN == 8 && TM >= 1 && TN >= 1 && TM * 16 * WGM == BM && TN * 16 * WGN == BN, "8 waves");
-  static_assert(BK == 16 || BK == 32, "BK");
   static_assert(BN * 4 <= 1024 && 1024 % (BN * 4) == 0, "a DMA kilobyte holds whole B rows");
   static_assert(A_KB * 8 * 1024 == A_STAGE && B_KB * 8 * 1024 == B_STAGE, "stage must split over 8 waves");
-  static_assert(STAGES >= 2 && STAGES <= 6 && STAGES * STAGE <= 160 * 1024, "LDS");
+  static_assert(STAGES >= 3 && STAGES <= 6 && STAGES * STAGE <= 160 * 1024, "LDS");
   static_assert(D * DMA_PER_SLAB < 64, "vmcnt range");
 
   __shared__ __attribute__((aligned(1024))) unsigned char st0[STAGE];
   __shared__ __attribute__((aligned(1024))) unsigned char st1[STAGE];
-  __shared__ __attribute__((aligned(1024))) unsigned char st2[STAGES > 2 ? STAGE : 16];
+  __shared__ __attribute__((aligned(1024))) unsigned char st2[STAGE];
   __shared__ __attribute__((aligned(1024))) unsigned char st3[STAGES > 3 ? STAGE : 16];
   __shared__ __attribute__((aligned(1024))) unsigned char st4[STAGES > 4 ? STAGE : 16];
   __shared__ __attribute__((aligned(1024))) unsigned char st5[STAGES > 5 ? STAGE : 16];
@@ -128,7 +125,7 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512))) gemm_f32_
   for (int i = 0; i < A_KB; ++i) {
     const int kb = wave * A_KB + i;
     const int r = kb * A_ROWS_PER_KB + lane / A_CHUNKS;
-    a_off[i] = r * args.lda + ((lane % A_CHUNKS) ^ swz_a<BK>(r)) * 4;
+    a_off[i] = r * args.lda + ((lane % A_CHUNKS) ^ swz_a(r)) * 4;
   }
 #pragma unroll
   for (int i = 0; i < B_KB; ++i) {
@@ -153,7 +150,7 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512))) gemm_f32_
   const int l16 = lane & 15;
   const int g = lane >> 4;
   const int a_row0 = wm * (16 * TM) + l16;  // + 16 i
-  const int a_sw = swz_a<BK>(a_row0);  // unchanged by + 16 i
+  const int a_sw = swz_a(a_row0);  // unchanged by + 16 i
   const int b_col0 = wn * (16 * TN) + l16;  // + 16 j
 
   f32x4 acc[TM][TN];
@@ -177,33 +174,27 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512))) gemm_f32_
     const unsigned char* sa = stage(s);
     const unsigned char* sb = sa + A_STAGE;
     // the slab's fragments, then its MFMAs
-    f32x4 af[KC][TM];
-    float bf[KC][4][TN];
+    f32x4 af[TM];
+    float bf[4][TN];
 #pragma unroll
-    for (int kc = 0; kc < KC; ++kc) {
+    for (int i = 0; i < TM; ++i) af[i] = *(const lds_f32x4*)(sa + (a_row0 + 16 * i) * (BK * 4) + 16 * (g ^ a_sw));
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
-        af[kc][i] = *(const lds_f32x4*)(sa + (a_row0 + 16 * i) * (BK * 4) + 16 * ((kc * 4 + g) ^ a_sw));
+    for (int q = 0; q < 4; ++q) {
+      const int k = 4 * g + q;
+      const int sw = swz_b(k);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int k = kc * 16 + 4 * g + q;
-        const int sw = swz_b(k);
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const int col = b_col0 + 16 * j;
-          bf[kc][q][j] = *(const lds_f32*)(sb + k * (BN * 4) + 16 * ((col >> 2) ^ sw) + 4 * (col & 3));
-        }
+      for (int j = 0; j < TN; ++j) {
+        const int col = b_col0 + 16 * j;
+        bf[q][j] = *(const lds_f32*)(sb + k * (BN * 4) + 16 * ((col >> 2) ^ sw) + 4 * (col & 3));
       }
     }
 #pragma unroll
-    for (int kc = 0; kc < KC; ++kc)
+    for (int q = 0; q < 4; ++q)
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
+      for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[kc][q][j], af[kc][i][q], acc[i][j], 0, 0, 0);
+        for (int j = 0; j < TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[q][j], af[i][q], acc[i][j], 0, 0, 0);
     // this wave's DMA of slab t+1 has landed (slabs through min(t+D, nk-1) issued)
     if (t + D < nk)
       __builtin_amdgcn_s_waitcnt(waitcnt_vm((D - 1) * DMA_PER_SLAB));

@@ -929,9 +929,10 @@ void default_tile(int dtype, int conv, int M, int N, int K, xtc_hip_tile* t, int
     }
   }
   // aligned fp32 shapes with fewer than 256 128x128 tiles (the M = 128-256
-  // projections): the LDS-DMA fp32 kernel behind 128x128x32, 2x4 waves,
-  // split K by powers of two, at least 1024 deep each, to between 224 and
-  // 256 workgroups, one wave over the chip (Gemma27B_QKV 256x8192x4608, 128 tiles: 201 -> 154 us at
+  // projections): 128x128x32 of 2x4 waves, split K by powers of two, at least
+  // 1024 deep each, to between 224 and 256 workgroups, one wave over the chip
+  // (times of the fp32-MFMA kernel that ran this tile when the line was drawn;
+  // now gemm_planes.hpp: Gemma27B_QKV 256x8192x4608, 128 tiles: 201 -> 154 us at
   // split 2; Gemma9B_QK 256x3584x8192, 56 tiles: 162 -> 138 us at split 4;
   // Llama3_QKV 86 -> 76 us).  Past 256 workgroups the second wave costs more
   // than the split gains (Gemma27B_QK, 72 tiles: 261 us at split 2, 264 us
@@ -948,8 +949,8 @@ void default_tile(int dtype, int conv, int M, int N, int K, xtc_hip_tile* t, int
       return;
     }
   }
-  // large aligned fp32 shapes with at least one 256x128 tile per CU: the
-  // LDS-DMA fp32 kernel behind this tile
+  // large aligned fp32 shapes with at least one 256x128 tile per CU: this
+  // 8-wave tile (gemm_planes.hpp)
   if (f32 && !conv && M % 256 == 0 && N % 128 == 0 && K % 32 == 0 && (int64_t)(M / 256) * (N / 128) >= 256 &&
       pick(256, 128, 32, 4, 2))
     return;
@@ -1365,9 +1366,9 @@ bool f32_lds_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, i
   return true;
 }
 
-template <int BM, int BN, int BK, int WGM, int WGN, int STAGES>
+template <int BM, int BN, int WGM, int WGN, int STAGES>
 void launch_f32_lds(const GemmArgs& a, dim3 grid, hipStream_t s) {
-  hipLaunchKernelGGL((gemm_f32_lds<BM, BN, BK, WGM, WGN, STAGES>), grid, dim3(512), 0, s, a);
+  hipLaunchKernelGGL((gemm_f32_lds<BM, BN, WGM, WGN, STAGES>), grid, dim3(512), 0, s, a);
 }
 
 // Compiled pipeline depths (LDS stages) of the LDS-DMA fp32 kernel, per tile;
@@ -1377,14 +1378,14 @@ struct F32LdsVariant {
   GemmLaunch launch;
 };
 const F32LdsVariant kF32Lds[] = {
-    {256, 128, 16, 4, 2, 4, &launch_f32_lds<256, 128, 16, 4, 2, 4>},
-    {256, 128, 16, 4, 2, 3, &launch_f32_lds<256, 128, 16, 4, 2, 3>},
-    {256, 128, 16, 4, 2, 5, &launch_f32_lds<256, 128, 16, 4, 2, 5>},
-    {256, 128, 16, 4, 2, 6, &launch_f32_lds<256, 128, 16, 4, 2, 6>},
-    {128, 256, 16, 2, 4, 5, &launch_f32_lds<128, 256, 16, 2, 4, 5>},
-    {128, 256, 16, 2, 4, 3, &launch_f32_lds<128, 256, 16, 2, 4, 3>},
-    {128, 256, 16, 2, 4, 4, &launch_f32_lds<128, 256, 16, 2, 4, 4>},
-    {128, 256, 16, 2, 4, 6, &launch_f32_lds<128, 256, 16, 2, 4, 6>},
+    {256, 128, 16, 4, 2, 4, &launch_f32_lds<256, 128, 4, 2, 4>},
+    {256, 128, 16, 4, 2, 3, &launch_f32_lds<256, 128, 4, 2, 3>},
+    {256, 128, 16, 4, 2, 5, &launch_f32_lds<256, 128, 4, 2, 5>},
+    {256, 128, 16, 4, 2, 6, &launch_f32_lds<256, 128, 4, 2, 6>},
+    {128, 256, 16, 2, 4, 5, &launch_f32_lds<128, 256, 2, 4, 5>},
+    {128, 256, 16, 2, 4, 3, &launch_f32_lds<128, 256, 2, 4, 3>},
+    {128, 256, 16, 2, 4, 4, &launch_f32_lds<128, 256, 2, 4, 4>},
+    {128, 256, 16, 2, 4, 6, &launch_f32_lds<128, 256, 2, 4, 6>},
 };
 
 // The variant of tile t with `stages` (0: the tile's default), or null.
