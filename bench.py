@@ -40,9 +40,23 @@ sys.path.insert(0, str(ROOT))
 
 PEAK_TFLOPS = {"bfloat16": 2516.6, "float32": 157.3}  # dense MFMA, MI355X datasheet
 PEAK_HBM_GBS = 8000.0
+# fp32 matmul tiles whose products run as six bf16 MFMAs each (gemm_planes.hpp)
+PLANE_TILES = {(256, 128, 32, 4, 2), (128, 256, 32, 2, 4), (128, 128, 32, 2, 4)}
 
 
 from xtc_amd import configs as workloads  # noqa: E402  (graphs, seeded inputs, tuned schedules)
+
+
+def _on_planes(module) -> bool:  # type: ignore[no-untyped-def]
+    """Whether every matmul of the module is an fp32 one on bf16 MFMAs."""
+    configs = list(module.configs.values())
+    return (os.environ.get("XTC_HIP_GENERIC_GEMM") != "1" and bool(configs)
+            and all(getattr(c, "dtype", "") == "float32" and not c.conv and c.tile in PLANE_TILES for c in configs))
+
+
+def _peak_tflops(dtype: str, module) -> float:  # type: ignore[no-untyped-def]
+    """Peak of the MFMAs that the module's kernels issue, in TFLOP/s of `dtype`."""
+    return round(PEAK_TFLOPS["bfloat16"] / 6, 1) if _on_planes(module) else PEAK_TFLOPS[dtype]
 
 
 def _traffic(cfg: str) -> float | None:
@@ -223,7 +237,7 @@ def _xtc_protocol(cfg: str, backend, sch, dev, cargs, flops: int, dtype: str) ->
     if status():
         raise SystemExit("payload reported an error under the evaluate_perf protocol")
     rate = (workloads.alg_bytes(cfg) / (proto["device_min_ms"] * 1e-3) / 1e9 / PEAK_HBM_GBS if cfg == "C3b"
-            else flops / (proto["device_min_ms"] * 1e-3) / 1e12 / PEAK_TFLOPS[dtype])
+            else flops / (proto["device_min_ms"] * 1e-3) / 1e12 / _peak_tflops(dtype, module))
     proto["device_min_pct_of_peak"] = round(100 * rate, 2)
     return proto
 
@@ -315,8 +329,8 @@ def _named_ops(steps: int, warmup_ms: float, dtype: str = "float32") -> int:
     layer registry, src/xtc/artifacts) with the backend's default schedule,
     one JSON line each: kernel time per payload call over `steps`
     back-to-back calls at steady clocks (HIP events, seeded uniform inputs),
-    TFLOP/s, and the fraction of the op's roofline max(FLOP / MFMA peak of
-    `dtype`, algorithmic bytes / 8 TB/s), algorithmic bytes being every
+    TFLOP/s, and the fraction of the op's roofline max(FLOP / peak of the MFMAs
+    that its kernels issue, algorithmic bytes / 8 TB/s), algorithmic bytes being every
     input read once and the output written once (bf16 inputs, fp32
     output).  A last line summarises."""
     import numpy as np
@@ -362,7 +376,7 @@ def _named_ops(steps: int, warmup_ms: float, dtype: str = "float32") -> int:
         us = ms.value * 1e3 / steps
         flops = 2 * int(np.prod(dims[:7] if op == "conv2d" else dims))
         nbytes = sum(d.nbytes for d in (*d_in, *d_out))
-        t_mfma, t_hbm = flops / (PEAK_TFLOPS[dtype] * 1e12), nbytes / (PEAK_HBM_GBS * 1e9)
+        t_mfma, t_hbm = flops / (_peak_tflops(dtype, module) * 1e12), nbytes / (PEAK_HBM_GBS * 1e9)
         roof_us = max(t_mfma, t_hbm) * 1e6
         fracs.append(roof_us / us)
         print(json.dumps({"named_op": name, "operator": op, "dtype": dtype, "dims": dims, "us": round(us, 2),
@@ -545,7 +559,9 @@ def main(argv: list[str] | None = None) -> int:
         roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s"}
     else:
         achieved = flops / kernel_s / 1e12
-        roof = {"bound": "mfma", "achieved": round(achieved, 1), "peak": PEAK_TFLOPS[dtype], "unit": "TFLOP/s"}
+        roof = {"bound": "mfma", "achieved": round(achieved, 1), "peak": _peak_tflops(dtype, module), "unit": "TFLOP/s"}
+        if _on_planes(module):
+            roof["instructions"] = "six bf16 MFMAs per fp32 product: a sixth of the bf16 peak"
     roof["frac"] = round(roof["achieved"] / roof["peak"], 4)
     roof["traffic"] = _traffic(cfg)
     line = {
@@ -585,7 +601,8 @@ def main(argv: list[str] | None = None) -> int:
         # the measured MFMA ceiling (register-only MFMA loop, xtc_hip_evaluate_flops):
         # on random operands the board's power limit holds it below the datasheet
         print(f"[bench] {cfg}: measured MFMA ceiling", file=sys.stderr, flush=True)
-        ceil = {op: 2 * dev.evaluate_flops(dtype, op) / 1e12 for op in ("zero", "random")}
+        per, issued = (6, "bfloat16") if _on_planes(module) else (1, dtype)
+        ceil = {op: 2 * dev.evaluate_flops(issued, op) / 1e12 / per for op in ("zero", "random")}
         line["config"]["mfma_ceiling"] = {
             "probe": "register-only MFMA loop, xtc_hip_evaluate_flops_operands",
             "zero_tflops": round(ceil["zero"], 1),
