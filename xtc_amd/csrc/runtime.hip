@@ -1269,11 +1269,15 @@ xtc_hip_tile planes_conv_any_tile(int dtype, int M, int N, int splits) {
 //   64x64    rounds of 256 * slabs * 0.55 (0.85 on the generic template) + 6
 //            (16 where gemm_planes splits K)
 // which follow the measured times of 20 shapes x 40 launches to 15 %.  The
-// generic 128x128 tile is never better.  K is split at most as often as the
-// class says, or as the descriptor does (us, before -> now): 3000^3 727 ->
-// 446, 2048x2048x1024 89.7 -> 54.2, 256x4608x8192 153 -> 117, 768x768x4096
-// 58.4 -> 44.8, 1280x4096x2048 159 -> 145, 1000x1104x1200 44.3 -> 34.5,
-// 2000x2304x2600 187 -> 182.
+// generic 128x128 tile is never chosen: its fp32 MFMAs round at every product,
+// and it is only faster over a slab or two (2318x3344x48: 27.2 us against 31.5).
+// K is split at most as often as the class says, or as the descriptor does (us,
+// before -> now): 3000^3 727 -> 446, 2048x2048x1024 89.7 -> 54.2, 256x4608x8192
+// 153 -> 117, 768x768x4096 58.4 -> 44.8, 1280x4096x2048 159 -> 145,
+// 1000x1104x1200 44.3 -> 34.5.  Over 110 random shapes that it moves (or splits
+// less in bf16) it is 1.19 times as fast in the mean; ten lose over 3 %, the worst
+// 98x5128x808 B^T 18.6 -> 22.4, 1615x440x568 B^T 17.5 -> 20.7, 2386x192x3904
+// 46.4 -> 52.4, 695x576x2368 30.1 -> 33.5.
 bool planes_wide_tile(const xtc_hip_matmul_desc& d, int lda, int ldb, bool bt, bool on_planes, xtc_hip_tile* t,
                       int* split_k) {
   const bool small = t->bm == 64 && t->bn == 64;
@@ -1331,7 +1335,8 @@ bool planes_bt_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t, int 
 // of gemm_planes, whose pipeline takes 4 to 6 us to fill: fp32 205x329 at K 17
 // 3.7 against 6.1 us, at K 33 5.5 against 7.0, at K 49 7.5 against 7.0; bf16 at
 // K 17 3.7 against 4.6, at K 25 4.6 each; fp32 1501x1499 at K 9 10.7 against
-// 10.9 us.
+// 10.9 us.  From K 33 on fp32 stays with gemm_planes, which rounds once per 32
+// products where the thread rounds at each (30x1674x37: 6.6 us against 6.0).
 bool short_sums(int dtype, int64_t M, int64_t N, int K) {
   return K <= (dtype == XTC_HIP_F32 ? 32 : 16) && M * N * K <= (16 << 20);
 }
