@@ -290,3 +290,20 @@ def test_default_configs_report_the_kernel_that_runs():
     backend = Backend(gb.graph)
     cfg = backend.get_compiler().kernel_configs(backend.get_scheduler().schedule())["C"]
     assert cfg.tile == (128, 128, 32, 2, 4) and cfg.split_k == 1 and cfg.source == "default"
+
+
+@pytest.mark.parametrize("cut,tile", [(2048, (256, 128, 32, 4, 2)), (2, (128, 128, 32, 2, 2))])
+def test_default_pieces_of_a_split_see_their_alignment(cut, tile):
+    # 2048 columns from `cut` on: whole vectors, or B rows that start 8 bytes past one
+    import xtc_amd.graphs.xtc.op as O
+    from xtc_amd.backends.hip import Backend
+
+    a, b = O.tensor((3000, 1024), "float32", name="A"), O.tensor((1024, 4104), "float32", name="B")
+    with O.graph(name="mm") as gb:
+        O.matmul(a, b, name="C")
+    backend = Backend(gb.graph)
+    sch = backend.get_scheduler()
+    sch.split("j", {"l": 0, "m": cut, "r": cut + 2048})
+    pieces = backend.get_compiler().kernel_configs(sch.schedule())["C"].pieces
+    assert (pieces[1].n0, pieces[1].N) == (cut, 2048)
+    assert pieces[1].config.tile == tile and pieces[1].config.source == "default"
