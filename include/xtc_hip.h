@@ -191,8 +191,12 @@ int xtc_hip_matmul_noalloc(const xtc_hip_matmul_desc *desc, const void *A,
  * producer (operators.py:350-591, MlirOps.py:719-735) fused into the loader.
  * Output and bias are fp32 for fp32 / bf16 operands and fp64 for fp64 ones.
  * Channels or filters that are not whole 16-byte vectors: fp32, and bf16 below
- * 16 channels or with such filters, gather the window in place; other bf16 and
- * fp64 calls stage zero channels; short sums run a scalar kernel. */
+ * 16 channels, gather the window in place by default and on the gather's own
+ * tiles by name (fp32 64x64x32 of 2x2 waves and 128x64x32 of 4x2, bf16 64x64x64
+ * of 2x2); on any other tile, and for other bf16 and fp64 calls, zero channels
+ * are staged.  Where they cannot be (such filters, a pad value that is not
+ * finite) fp32 and bf16 gather on any tile; short sums and fp64 then run a
+ * scalar kernel. */
 typedef struct {
   int dtype;
   int N, H, W, C;        /* unpadded input */
@@ -282,8 +286,10 @@ int xtc_hip_default_tile(int dtype, int conv, int M, int N, int K, xtc_hip_tile 
  * or 128x128x32 tile of 2x2 waves move to an 8-wave tile of the bf16-plane
  * kernel, with no more splits, where that is estimated to be faster, and bf16
  * calls on 128-row tiles split K no more often than fills the CUs once.  A tile
- * that a descriptor names runs as named, with the named split (but calls
- * without whole 16-byte vectors, whose kernels have blocks of their own). */
+ * that a descriptor names runs as named, with the named split (small 64x64x32
+ * grids split 2 to 8 ways as 32x32 workgroups of the split-wave kernel, the same
+ * sums in the same order; calls without whole 16-byte vectors on blocks of
+ * their kernels' own). */
 int xtc_hip_matmul_default_tile(const xtc_hip_matmul_desc *desc, xtc_hip_tile *out, int *split_k);
 
 /* Tile a conv2d descriptor gets when it leaves `tile` zeroed.  Unlike
@@ -291,7 +297,9 @@ int xtc_hip_matmul_default_tile(const xtc_hip_matmul_desc *desc, xtc_hip_tile *o
  * for a window wider than 1x1 the direct conv kernel's wider 1x4-wave block
  * replaces the 8x8 one when its input halo fits and its blocks fit in one
  * wave of 256 CUs, 7x14 pixels (tile 98x64x16) first, else 8x14 (tile
- * 112x64x16). */
+ * 112x64x16); a conv without whole 16-byte vectors gets the tile that its
+ * windows are gathered on; a bf16 conv on a 128-row tile splits K no more often
+ * than fills the CUs once. */
 int xtc_hip_conv2d_default_tile(const xtc_hip_conv2d_desc *desc, xtc_hip_tile *out, int *split_k);
 
 /* Pipeline depths that `desc` (with 256-byte aligned operands) may name: the

@@ -1417,9 +1417,10 @@ bool splitwave_gemm_applies(const xtc_hip_matmul_desc& d, const xtc_hip_tile& t,
   if (d.M % 32 || d.N % 32 || d.K % (16 * split_k)) return false;
   if (lda % 4 || !aligned16(A)) return false;
   if (t.bm == 32 && t.bn == 32 && t.bk == 16 && t.wgm == 1 && t.wgn == 1) return true;
-  // The 64x64x32 tile (2x2 waves of 32x32), when its 32x32 blocks fit in one wave of 256 CUs: the wave blocks become workgroups
-  // whose waves are the splits, which meet in LDS instead of memory, in the
-  // same order (the results are bit-identical when a split is whole slabs).
+  // The 64x64x32 tile (2x2 waves of 32x32), when its 32x32 blocks fit in one
+  // wave of 256 CUs: the wave blocks become workgroups whose waves are the
+  // splits, which meet in LDS instead of memory, in the same order (the results
+  // are bit-identical when a split is whole slabs).
   // 512^3 at split 4 11.0 -> 5.5 us, 256^3 at split 2 9.5 -> 4.9, 32x4096x1024
   // at split 8 13.2 -> 10.7; with 512 blocks it loses (512x1024x1024 at split 8
   // 18.9 -> 20.7 us).  Up to 4 splits it wins at every depth (512x512x2048 at 4
@@ -2599,8 +2600,8 @@ int xtc_hip_conv2d_pipeline_depths(const xtc_hip_conv2d_desc* desc, int* depths,
   const int OW = (WP - d.S) / d.stride_w + 1;
   const int vec = conv_vec(d);
   xtc_hip_tile u;
-  if (int sk; d.tile.bm && !find_entry(d.dtype, 1, d.tile) && (d.C % vec || d.F % vec) && conv_gathers(d, OH, OW, true, &u, &sk) &&
-              same_tile(u, d.tile)) {
+  if (int sk; d.tile.bm && !find_entry(d.dtype, 1, d.tile) && (d.C % vec || d.F % vec) &&
+              conv_gathers(d, OH, OW, true, &u, &sk) && same_tile(u, d.tile)) {
     depths[0] = 2;  // the gather's own tile: two LDS buffers
     return 1;
   }
